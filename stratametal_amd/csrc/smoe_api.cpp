@@ -619,19 +619,43 @@ smoe_status smoe_forward(const smoe_geom* g, const smoe_weights* w, const float*
 
 // ------------------------------------------------------------------------------------------------ layer ends
 namespace {
-// gr_read's scratch: proj [T][hc_lr] and rs [T][hc]
+// gr_read's scratch: proj [T][hc_lr] and rs [T][hc]; for a batch that runs on the matrix cores, also the bf16
+// activations, the projection's K-slice sums and lq
 struct HcLayout {
-    size_t proj, rs, total;
+    size_t proj, rs, act, part, lq, total;
 };
-HcLayout hc_layout(const smoe_hc& h, int64_t T) {
+HcLayout hc_layout(const smoe_hc& h, int n_embd, int64_t T) {
     HcLayout L{};
     size_t o = 0;
     L.proj = o;
     o = up(o + (size_t)T * h.hc_lr * 4);
     L.rs = o;
     o = up(o + (size_t)T * h.hc * 4);
+    if (smoe::hc_mm_shape(T, n_embd, h.hc, h.hc_lr)) {
+        size_t act, part, lq;
+        smoe::hc_mm_bytes(T, n_embd, h.hc, h.hc_lr, &act, &part, &lq);
+        L.act = o;
+        o = up(o + act);
+        L.part = o;
+        o = up(o + part);
+        L.lq = o;
+        o = up(o + lq);
+    }
     L.total = o;
     return L;
+}
+
+// The read's launches: the matrix cores for a batch (its kernels take R, norm and mixed as 16-byte vectors), else the
+// row-per-wave kernels.
+hipError_t hc_read(const smoe_hc& h, int n_embd, const float* R, int T, float* mixed, float* inject, uint8_t* ws,
+                   const HcLayout& L, hipStream_t st) {
+    float* rs = reinterpret_cast<float*>(ws + L.rs);
+    if (smoe::hc_mm_shape(T, n_embd, h.hc, h.hc_lr) && aligned(R, 16) && aligned(h.norm, 16) && aligned(mixed, 16))
+        return smoe::launch_hc_read_mm(R, h.norm, h.down, h.up, h.inject, T, n_embd, h.hc, h.hc_lr, h.eps, rs,
+                                       reinterpret_cast<uint16_t*>(ws + L.act), reinterpret_cast<float*>(ws + L.part),
+                                       reinterpret_cast<uint16_t*>(ws + L.lq), mixed, inject, st);
+    return smoe::launch_hc_read(const_cast<float*>(R), h.norm, h.down, h.up, h.inject, T, n_embd, h.hc, h.hc_lr, h.eps,
+                                reinterpret_cast<float*>(ws + L.proj), rs, mixed, inject, nullptr, nullptr, nullptr, st);
 }
 
 smoe_status check_hc(const smoe_hc* h, int32_t n_embd) {
@@ -651,7 +675,7 @@ extern "C" {
 
 size_t smoe_hc_read_workspace_bytes(const smoe_hc* hc, int32_t n_embd, int32_t max_tokens) {
     if (check_hc(hc, n_embd) != SMOE_OK || max_tokens < 0) return 0;
-    return hc_layout(*hc, max_tokens).total;
+    return hc_layout(*hc, n_embd, max_tokens).total;
 }
 
 smoe_status smoe_hc_read(const smoe_hc* hc, int32_t n_embd, const float* R, int32_t n_tokens, float* mixed,
@@ -663,16 +687,12 @@ smoe_status smoe_hc_read(const smoe_hc* hc, int32_t n_embd, const float* R, int3
     if (!R || !mixed || !workspace) return fail(SMOE_ENULL, "hc_read: NULL buffer");
     if (!aligned(R, 4) || !aligned(mixed, 4) || (inject && !aligned(inject, 4)) || !aligned(workspace, kAlign))
         return fail(SMOE_EALIGN, "hc_read: R, mixed, inject 4-byte, workspace 256-byte aligned");
-    const HcLayout L = hc_layout(*hc, n_tokens);
+    const HcLayout L = hc_layout(*hc, n_embd, n_tokens);
     if (workspace_bytes < L.total)
         return fail(SMOE_ESIZE, "hc_read workspace is " + std::to_string(workspace_bytes) + " bytes, needs " +
                                     std::to_string(L.total));
     uint8_t* ws = static_cast<uint8_t*>(workspace);
-    SMOE_TRY(smoe::launch_hc_read(const_cast<float*>(R), hc->norm, hc->down, hc->up, hc->inject, n_tokens, n_embd,
-                                  hc->hc, hc->hc_lr, hc->eps, reinterpret_cast<float*>(ws + L.proj),
-                                  reinterpret_cast<float*>(ws + L.rs), mixed, inject, nullptr, nullptr, nullptr,
-                                  stream_of(hip_stream)),
-             "hc_read");
+    SMOE_TRY(hc_read(*hc, n_embd, R, n_tokens, mixed, inject, ws, L, stream_of(hip_stream)), "hc_read");
     return ok();
 }
 
@@ -708,7 +728,7 @@ FfnLayout ffn_layout(const smoe_geom& g, const smoe_hc& h, int64_t T) {
     L.y = o;
     o = up(o + (size_t)T * g.n_embd * 4);
     L.hc = o;
-    o = up(o + hc_layout(h, T).total);
+    o = up(o + hc_layout(h, g.n_embd, T).total);
     L.total = o;
     return L;
 }
@@ -746,12 +766,8 @@ smoe_status smoe_ffn_run(const smoe_geom* g, const smoe_weights* w, const smoe_h
     const size_t moe_bytes = layout(*g, n_tokens).total;
     s = check_forward(g, w, mixed, n_tokens, yb, ws + L.moe, moe_bytes, SMOE_PATH_AUTO, nullptr, nullptr);
     if (s != SMOE_OK) return s;
-    const HcLayout H = hc_layout(*hc, n_tokens);
-    SMOE_TRY(smoe::launch_hc_read(const_cast<float*>(residual), hc->norm, hc->down, hc->up, hc->inject, n_tokens,
-                                  g->n_embd, hc->hc, hc->hc_lr, hc->eps,
-                                  reinterpret_cast<float*>(ws + L.hc + H.proj), reinterpret_cast<float*>(ws + L.hc + H.rs),
-                                  mixed, inj, nullptr, nullptr, nullptr, stream_of(hip_stream)),
-             "hc_read");
+    const HcLayout H = hc_layout(*hc, g->n_embd, n_tokens);
+    SMOE_TRY(hc_read(*hc, g->n_embd, residual, n_tokens, mixed, inj, ws + L.hc, H, stream_of(hip_stream)), "hc_read");
     s = forward_impl(g, w, mixed, n_tokens, yb, add_shared, ws + L.moe, moe_bytes, trace, SMOE_PATH_AUTO, hip_stream,
                      nullptr, nullptr, 0.0f);
     if (s != SMOE_OK) return s;

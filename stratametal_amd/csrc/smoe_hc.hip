@@ -7,14 +7,16 @@
 //          proj_r = act . down_r (r < hc_lr), lq = bf16(silu(proj_r / hc)); gate_i = lq . up_i (i < hc * n);
 //          mixed_d = (sum_c xn_cd * sigmoid(gate_cd)) / hc;  inject_c = act . inj_c;
 //   write: out_cd = R_cd + y_d * 2 sigmoid(inject_c / hc).
-// The read is two bandwidth-bound bf16 GEMVs in a chain (about 10.5 MB of weights per token at n 2048, hc 4, hc_lr 320,
-// as much as the MoE block itself), so it is two launches: k_hc_proj (the norm, the activations staged in LDS, the
-// down and inject rows) and k_hc_mix (lq, the up rows, the gated mean).  The write is a third; the stacked call forms
-// it inside the next layer's k_hc_proj.  Reduction orders are fixed and restated by the test oracle
-// (or_hc_read_dev, or_hc_write_dev).
+// For few tokens the read is two bandwidth-bound bf16 GEMVs in a chain (about 10.5 MB of weights per call at n 2048,
+// hc 4, hc_lr 320, as much as the MoE block itself), so it is two launches: k_hc_proj (the norm, the activations staged
+// in LDS, the down and inject rows) and k_hc_mix (lq, the up rows, the gated mean).  Their reduction orders are fixed
+// and restated by the test oracle (or_hc_read_dev, or_hc_write_dev).  For a batch of tokens (kHcMmTokens) both products
+// run on the matrix cores: k_hc_act, k_hc_proj_mm, k_hc_lq, k_hc_mix_mm.
 #include "smoe_device.hpp"
 #include "smoe_gemv.hpp"
 #include "smoe_launch.hpp"
+
+#include <type_traits>
 
 namespace smoe {
 
@@ -225,6 +227,335 @@ __global__ __launch_bounds__(256) void k_hc_write(const float* R, const float* _
     const int64_t t = row / hc;
     const float s = sigmoid(inject[row] / (float)hc);
     out[i] = R[i] + y[t * n + d] * (2.0f * s);
+}
+
+// ------------------------------------------------------------------------------------------------ many tokens
+// The read as two bf16 matrix products: every bf16 product is exact in f32 and the sums are the matrix core's f32
+// accumulation, in the hardware's order and over the K slices below, so proj, inject and the gates are the exact dots
+// to f32 sums' accuracy, not bit for bit the row-per-wave kernels' (each GEMV launch reads all the weights once per
+// token from the caches: 1591 + 393 us at 1000 tokens of n 2048, hc 4, hc_lr 320).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// k_hc_act: one work-group per token: the stream scales (as k_hc_proj forms them) into rs, and act = bf16((R * rs) *
+// w_norm) through LDS to memory as 16-byte pieces.  Bound by reading R once.
+template <int HC, int NM>
+__global__ __launch_bounds__(256) void k_hc_act(const float* __restrict__ R, const float* __restrict__ norm, int n,
+                                                 int hc, float eps, uint16_t* __restrict__ act,
+                                                 float* __restrict__ rs_out) {
+    extern __shared__ __align__(16) uint16_t act_s[];  // hc * n bf16
+    __shared__ float wsum[HC][4];
+    __shared__ float rs_s[HC];
+    const int t = blockIdx.x, tid = threadIdx.x;
+    const int hd = hc * n;
+    const float* Rt = R + (size_t)t * hd;
+    float v[HC][NM];
+#pragma unroll
+    for (int c = 0; c < HC; ++c)
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const int d = tid + 256 * m;
+            v[c][m] = (c < hc && d < n) ? Rt[(size_t)c * n + d] : 0.0f;
+        }
+    stream_scales<HC, NM>(v, hc, n, eps, wsum, rs_s);
+    if (tid < hc) rs_out[(size_t)t * hc + tid] = rs_s[tid];
+#pragma unroll
+    for (int c = 0; c < HC; ++c)
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const int d = tid + 256 * m;
+            if (c < hc && d < n) {
+                const size_t i = (size_t)c * n + d;
+                act_s[i] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * norm[i]);
+            }
+        }
+    __syncthreads();
+    u32x4* dst = reinterpret_cast<u32x4*>(act + (size_t)t * hd);
+    for (int p = tid; p < hd / 8; p += 256) dst[p] = reinterpret_cast<const u32x4*>(act_s)[p];
+}
+
+// k_hc_proj_mm: part[s][t][r] = act[t] . [down; inj][r] over K slice s.  Work-group tile 64 tokens x 128 rows (wave w:
+// rows 32 w .. + 31, two row tiles by four token tiles), K in chunks of 64 through two LDS buffers (rows at a 144-byte
+// pitch: a 16-row fragment read covers the 64 banks once), the next two chunks' loads in flight in registers, one
+// barrier per chunk.  The product has few output tiles (48 at 1000 tokens of 324 rows) and a deep K (8192), so K is split
+// over `splits` work-groups (hc_splits), whose partial sums k_hc_lq adds in slice order.  Slices are the fastest index
+// and a power of two: the work-groups of an XCD share their K slices of the weights and activations, which its L2 holds.
+constexpr int kHpTok = 64, kHpRows = 128, kHpK = 64, kHpPitch = kHpK * 2 + 16;
+constexpr int kHpLa = kHpTok * 8 / 256, kHpLb = kHpRows * 8 / 256;  // 16-byte pieces of a chunk per thread
+
+__global__ __launch_bounds__(256) void k_hc_proj_mm(const uint16_t* __restrict__ act, const uint16_t* __restrict__ down,
+                                                     const uint16_t* __restrict__ inj, int hd, int hc_lr, int rows,
+                                                     int ld, int T, int splits, int per, int n_rb,
+                                                     float* __restrict__ part) {
+    __shared__ __align__(16) uint8_t sa[2][kHpTok * kHpPitch];
+    __shared__ __align__(16) uint8_t sb[2][kHpRows * kHpPitch];
+    const int s = blockIdx.x % splits, tile = blockIdx.x / splits;
+    const int t0 = (tile / n_rb) * kHpTok, r0 = (tile % n_rb) * kHpRows;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, i = lane & 15;
+    const int nk = min(per, hd / kHpK - s * per);  // this slice's chunks, at least one
+    // a thread's pieces of a chunk: piece tid % 8 of rows tid / 8 + 32 j (rows clamped: the tails' loads stay in bounds,
+    // their results are not stored)
+    const int pc = tid & 7, pr = tid >> 3;
+    const uint16_t* asrc[kHpLa];
+    const uint16_t* bsrc[kHpLb];
+#pragma unroll
+    for (int j = 0; j < kHpLa; ++j)
+        asrc[j] = act + (size_t)min(t0 + pr + 32 * j, T - 1) * hd + (size_t)s * per * kHpK + 8 * pc;
+#pragma unroll
+    for (int j = 0; j < kHpLb; ++j) {
+        const int r = min(r0 + pr + 32 * j, rows - 1);
+        bsrc[j] = (r < hc_lr ? down + (size_t)r * hd : inj + (size_t)(r - hc_lr) * hd) + (size_t)s * per * kHpK + 8 * pc;
+    }
+    u32x4 ra[2][kHpLa], rw[2][kHpLb];
+    auto load = [&](auto slot, int k0) {
+        constexpr int P = decltype(slot)::value;
+#pragma unroll
+        for (int j = 0; j < kHpLa; ++j) ra[P][j] = *reinterpret_cast<const u32x4*>(asrc[j] + k0);
+#pragma unroll
+        for (int j = 0; j < kHpLb; ++j) rw[P][j] = *reinterpret_cast<const u32x4*>(bsrc[j] + k0);
+    };
+    auto stash = [&](auto slot) {
+        constexpr int P = decltype(slot)::value;
+#pragma unroll
+        for (int j = 0; j < kHpLa; ++j) *reinterpret_cast<u32x4*>(&sa[P][(pr + 32 * j) * kHpPitch + 16 * pc]) = ra[P][j];
+#pragma unroll
+        for (int j = 0; j < kHpLb; ++j) *reinterpret_cast<u32x4*>(&sb[P][(pr + 32 * j) * kHpPitch + 16 * pc]) = rw[P][j];
+    };
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    load(Zero{}, 0);
+    load(One{}, min(1, nk - 1) * kHpK);
+    stash(Zero{});
+    __syncthreads();
+    f32x4 acc[2][4];
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[m][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto chunk = [&](int kc, auto parity) {
+        constexpr int P = decltype(parity)::value;
+        using Q = std::integral_constant<int, 1 - P>;
+        load(parity, min(kc + 2, nk - 1) * kHpK);  // (past the end: the last chunk again, which nobody reads)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int st = 0; st < kHpK / 32; ++st) {
+            bf16x8 w[2], a[4];
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+                w[m] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+                                                      &sb[P][(32 * wave + 16 * m + i) * kHpPitch + 64 * st + 16 * q]));
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+                a[b] = __builtin_bit_cast(bf16x8,
+                                          *reinterpret_cast<const u32x4*>(&sa[P][(16 * b + i) * kHpPitch + 64 * st + 16 * q]));
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[m], a[b], acc[m][b], 0, 0, 0);
+        }
+        stash(Q{});
+        __syncthreads();
+    };
+    int kc = 0;
+    for (; kc + 1 < nk; kc += 2) {
+        chunk(kc, Zero{});
+        chunk(kc + 1, One{});
+    }
+    if (kc < nk) chunk(kc, Zero{});
+    // lane (q, i) holds rows 4 q .. + 3 of token i of each tile: one 16-byte store (ld % 4 == 0)
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const int t = t0 + 16 * b + i, r = r0 + 32 * wave + 16 * m + 4 * q;
+            if (t < T && r < ld) *reinterpret_cast<f32x4*>(part + ((size_t)s * T + t) * ld + r) = acc[m][b];
+        }
+}
+
+// k_hc_lq: one work-group per token: the K slices' sums in slice order, lq = bf16(silu(proj / hc)) (zero from hc_lr to
+// kp, the mix kernel's whole chunks) and inject.
+__global__ __launch_bounds__(256) void k_hc_lq(const float* __restrict__ part, int T, int splits, int ld, int hc,
+                                                int hc_lr, int kp, uint16_t* __restrict__ lq, float* __restrict__ inject) {
+    const int t = blockIdx.x, n = max(kp, hc_lr + hc);
+    for (int r = threadIdx.x; r < n; r += 256) {
+        float v = 0.0f;
+        if (r < hc_lr + hc) {
+            const float* p = part + (size_t)t * ld + r;
+            v = p[0];
+#pragma unroll 8
+            for (int s = 1; s < splits; ++s) v = v + p[(size_t)s * T * ld];
+        }
+        if (r < kp) {
+            const float z = v / (float)hc;
+            lq[(size_t)t * kp + r] = r < hc_lr ? (uint16_t)f32_to_bf16(z / (1.0f + expf_smoe(-z))) : (uint16_t)0;
+        }
+        if (inject && r >= hc_lr && r < hc_lr + hc) inject[(size_t)t * hc + r - hc_lr] = v;
+    }
+}
+
+// k_hc_mix_mm: mixed[t][d] for 16 NT tokens x 64 values of d per work-group; wave w owns 16 values of d in every
+// stream, so that a lane ends with the gates of all streams of its (token, d) and forms the gated mean in registers.
+// lq of the tokens in LDS (pitch kp * 2 + 16 bytes); the wave's `up` rows stream from memory in chunks of 64 of K, the
+// next chunk's loads in flight.  The d ranges are the fastest index, so that where n / 64 is a multiple of 8 the token
+// blocks of a d range share an XCD, whose L2 serves the rows each of them reads again.  Bound by reading R and writing
+// mixed once the rows are in the caches.
+template <int HC, int NT>
+__global__ __launch_bounds__(256) void k_hc_mix_mm(const float* __restrict__ R, const float* __restrict__ norm,
+                                                    const uint16_t* __restrict__ up, const uint16_t* __restrict__ lq,
+                                                    const float* __restrict__ rs, int n, int hc, int hc_lr, int kp,
+                                                    int T, float* __restrict__ mixed) {
+    extern __shared__ __align__(16) uint8_t lq_s[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = lane >> 4, i = lane & 15;
+    const int nd = n >> 6;
+    const int t0 = (blockIdx.x / nd) * 16 * NT, d0 = (blockIdx.x % nd) * 64 + 16 * wave;
+    const int hd = hc * n, pitch = kp * 2 + 16, pieces = kp >> 3;
+    const uint16_t* wrow[HC];
+#pragma unroll
+    for (int c = 0; c < HC; ++c) wrow[c] = up + ((size_t)min(c, hc - 1) * n + d0 + i) * hc_lr;
+    u32x4 w[2][HC][2];
+    auto load = [&](auto slot, int k0) {
+        constexpr int P = decltype(slot)::value;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            const int k = k0 + 32 * st + 8 * q;  // (the tail past hc_lr: zeros, not the next row's values)
+#pragma unroll
+            for (int c = 0; c < HC; ++c)
+                w[P][c][st] = k < hc_lr ? *reinterpret_cast<const u32x4*>(wrow[c] + k) : u32x4{0, 0, 0, 0};
+        }
+    };
+    using Zero = std::integral_constant<int, 0>;
+    using One = std::integral_constant<int, 1>;
+    load(Zero{}, 0);
+    for (int p = tid; p < 16 * NT * pieces; p += 256) {
+        const int r = p / pieces, o = p - r * pieces;
+        *reinterpret_cast<u32x4*>(lq_s + (size_t)r * pitch + 16 * o) =
+            *reinterpret_cast<const u32x4*>(lq + (size_t)min(t0 + r, T - 1) * kp + 8 * o);
+    }
+    __syncthreads();
+    f32x4 acc[HC][NT];
+#pragma unroll
+    for (int c = 0; c < HC; ++c)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) acc[c][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto chunk = [&](int k0, auto parity) {
+        constexpr int P = decltype(parity)::value;
+        load(std::integral_constant<int, 1 - P>{}, k0 + 64);  // (past the end: zeros)
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            bf16x8 a[NT];
+#pragma unroll
+            for (int b = 0; b < NT; ++b)
+                a[b] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(lq_s + (size_t)(16 * b + i) * pitch +
+                                                                                  2 * (k0 + 32 * st + 8 * q)));
+#pragma unroll
+            for (int c = 0; c < HC; ++c) {
+                const bf16x8 wv = __builtin_bit_cast(bf16x8, w[P][c][st]);
+#pragma unroll
+                for (int b = 0; b < NT; ++b) acc[c][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, a[b], acc[c][b], 0, 0, 0);
+            }
+        }
+    };
+    int k0 = 0;
+    for (; k0 + 64 < kp; k0 += 128) {
+        chunk(k0, Zero{});
+        chunk(k0 + 64, One{});
+    }
+    if (k0 < kp) chunk(k0, Zero{});
+    const int d = d0 + 4 * q;  // lane (q, i): the gates of d .. d + 3 of token i of each tile
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+        const int t = t0 + 16 * b + i;
+        if (t >= T) continue;
+        f32x4 m = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < HC; ++c) {
+            if (c >= hc) break;
+            const f32x4 x = *reinterpret_cast<const f32x4*>(R + (size_t)t * hd + (size_t)c * n + d);
+            const f32x4 nv = *reinterpret_cast<const f32x4*>(norm + (size_t)c * n + d);
+            const float sc = rs[(size_t)t * hc + c];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) m[r] = m[r] + ((x[r] * sc) * nv[r]) * sigmoid(acc[c][b][r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m[r] = m[r] / (float)hc;
+        *reinterpret_cast<f32x4*>(mixed + (size_t)t * n + d) = m;
+    }
+}
+
+// From how many tokens the read runs on the matrix cores: from 17 tokens (a second 16-token tile) and 2^23 products of
+// the projection, where its four launches cost what the two of the row-per-wave kernels do (hc 2, hc_lr 64, n 2048: 16.3
+// us row-per-wave and 17.3 on the matrix cores at 32 tokens, 23.1 and 20.1 at 64; hc 4, hc_lr 320: 44.6 and 32.7 at 17
+// tokens, 140 and 37 at 64, 1965 and 66 at 1000).  The shapes that do: whole 64-value chunks of a stream and an lq tile
+// within 64 KiB of LDS; others keep the row-per-wave kernels.
+constexpr int kHcMmTokens = 17;
+constexpr int64_t kHcMmProducts = (int64_t)1 << 23;
+constexpr int kHcMmMaxLr = 960;
+static int hc_kp(int hc_lr) { return (hc_lr + 63) / 64 * 64; }
+static int hc_ld(int hc_lr, int hc) { return (hc_lr + hc + 3) / 4 * 4; }
+// K slices: a power of two up to 32 that fills the chip about once with two work-groups per CU.
+constexpr int kHpGroups = 512;
+static int hc_splits(int tiles, int chunks) {
+    int s = 1;
+    while (s < 32 && 2 * s <= chunks && 2 * s * tiles <= kHpGroups) s *= 2;
+    return s;
+}
+
+bool hc_mm_shape(int64_t T, int n, int hc, int hc_lr) {
+    return T >= kHcMmTokens && hc_shape_ok(n, hc, hc_lr) && T * hc * n * hc_lr >= kHcMmProducts && n % 64 == 0 &&
+           hc_lr <= kHcMmMaxLr;
+}
+// The scratch of the matrix-core read (act, the K slices' sums, lq), growing with T: part is bounded by the slices'
+// largest count for few tokens, by the launch's work-groups' tiles, or by one slice.
+void hc_mm_bytes(int64_t T, int n, int hc, int hc_lr, size_t* act, size_t* part, size_t* lq) {
+    const size_t rows = (size_t)T * hc_ld(hc_lr, hc) * 4, tiles = (size_t)kHpGroups * kHpTok * kHpRows * 4;
+    *act = (size_t)T * hc * n * 2;
+    *part = rows > tiles ? rows : (32 * rows < tiles ? 32 * rows : tiles);
+    *lq = (size_t)T * hc_kp(hc_lr) * 2;
+}
+
+hipError_t launch_hc_read_mm(const float* R, const float* norm, const uint16_t* down, const uint16_t* up,
+                             const uint16_t* inj, int T, int n, int hc, int hc_lr, float eps, float* rs, uint16_t* act,
+                             float* part, uint16_t* lq, float* mixed, float* inject, hipStream_t s) {
+    if (!hc_mm_shape(T, n, hc, hc_lr)) return hipErrorInvalidValue;
+    const int hd = hc * n, nm = (n + 255) / 256, rows = hc_lr + hc, ld = hc_ld(hc_lr, hc), kp = hc_kp(hc_lr);
+    const size_t lds = (size_t)hd * 2;
+#define SMOE_HCA(HCv, NMv) \
+    hipLaunchKernelGGL((k_hc_act<HCv, NMv>), dim3((unsigned)T), dim3(256), lds, s, R, norm, n, hc, eps, act, rs)
+    if (hc <= 4) {
+        if (nm <= 2) SMOE_HCA(4, 2);
+        else if (nm <= 8) SMOE_HCA(4, 8);
+        else SMOE_HCA(4, 16);
+    } else {
+        if (nm <= 2) SMOE_HCA(8, 2);
+        else if (nm <= 8) SMOE_HCA(8, 8);
+        else SMOE_HCA(8, 16);
+    }
+#undef SMOE_HCA
+    const int n_tb = (T + kHpTok - 1) / kHpTok, n_rb = (rows + kHpRows - 1) / kHpRows, chunks = hd / kHpK;
+    int splits = hc_splits(n_tb * n_rb, chunks);
+    const int per = (chunks + splits - 1) / splits;
+    splits = (chunks + per - 1) / per;  // every slice holds a chunk
+    hipLaunchKernelGGL(k_hc_proj_mm, dim3((unsigned)(splits * n_tb * n_rb)), dim3(256), 0, s, act, down, inj, hd, hc_lr,
+                       rows, ld, T, splits, per, n_rb, part);
+    hipLaunchKernelGGL(k_hc_lq, dim3((unsigned)T), dim3(256), 0, s, part, T, splits, ld, hc, hc_lr, kp, lq, inject);
+    const int nt = T > 32 && hc <= 4 && kp <= 448 ? 4 : 2;
+    const unsigned grid = (unsigned)((T + 16 * nt - 1) / (16 * nt)) * (unsigned)(n / 64);
+    const size_t tile = (size_t)16 * nt * (kp * 2 + 16);
+#define SMOE_HCM(HCv, NTv)                                                                                         \
+    hipLaunchKernelGGL((k_hc_mix_mm<HCv, NTv>), dim3(grid), dim3(256), tile, s, R, norm, up, lq, rs, n, hc, hc_lr, kp, T, \
+                       mixed)
+    if (hc <= 2) {
+        if (nt == 4) SMOE_HCM(2, 4);
+        else SMOE_HCM(2, 2);
+    } else if (hc <= 4) {
+        if (nt == 4) SMOE_HCM(4, 4);
+        else SMOE_HCM(4, 2);
+    } else {
+        SMOE_HCM(8, 2);
+    }
+#undef SMOE_HCM
+    return hipGetLastError();
 }
 
 bool hc_shape_ok(int n, int hc, int hc_lr) {

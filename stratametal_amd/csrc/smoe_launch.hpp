@@ -148,6 +148,13 @@ bool hc_shape_ok(int n, int hc, int hc_lr);
 hipError_t launch_hc_read(float* R, const float* norm, const uint16_t* down, const uint16_t* up, const uint16_t* inj,
                           int n_tok, int n, int hc, int hc_lr, float eps, float* proj, float* rs, float* mixed,
                           float* inject, const float* rprev, const float* yprev, const float* injprev, hipStream_t s);
+// the read of a batch of tokens on the matrix cores, where hc_mm_shape says so: its scratch (hc_mm_bytes: act, the K
+// slices' sums, lq) and launches; R, norm and mixed 16-byte aligned
+bool hc_mm_shape(int64_t T, int n, int hc, int hc_lr);
+void hc_mm_bytes(int64_t T, int n, int hc, int hc_lr, size_t* act, size_t* part, size_t* lq);
+hipError_t launch_hc_read_mm(const float* R, const float* norm, const uint16_t* down, const uint16_t* up,
+                             const uint16_t* inj, int T, int n, int hc, int hc_lr, float eps, float* rs, uint16_t* act,
+                             float* part, uint16_t* lq, float* mixed, float* inject, hipStream_t s);
 hipError_t launch_hc_write(const float* R, const float* y, const float* inject, int n_tok, int n, int hc, float* out,
                            hipStream_t s);
 
