@@ -384,8 +384,14 @@ smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float
         if (e == hipSuccess && gate) e = smoe::launch_sigmoid_rows(y, T, n_out, gate, st);
         return e;
     };
-    SMOE_TRY(gemv(sh_gate_t(g), w->gate_sh, nxq, H, Fn, ngu, nullptr), "shared gate");
-    SMOE_TRY(gemv(sh_up_t(g), w->up_sh, nxq, H, Fn, ngu + (size_t)T * Fn, nullptr), "shared up");
+    if (smoe::native_type(sh_gate_t(g)) && sh_gate_t(g) == sh_up_t(g)) {  // gate and up in one launch
+        SMOE_TRY(smoe::launch_mmvq_native(sh_gate_t(g), static_cast<const uint8_t*>(w->gate_sh), nxq, H, Fn, T, ngu, Fn,
+                                          nullptr, st, static_cast<const uint8_t*>(w->up_sh), ngu + (size_t)T * Fn),
+                 "shared gate/up");
+    } else {
+        SMOE_TRY(gemv(sh_gate_t(g), w->gate_sh, nxq, H, Fn, ngu, nullptr), "shared gate");
+        SMOE_TRY(gemv(sh_up_t(g), w->up_sh, nxq, H, Fn, ngu + (size_t)T * Fn, nullptr), "shared up");
+    }
     SMOE_TRY(smoe::launch_swiglu_q8(ngu, ngu + (size_t)T * Fn, (int64_t)T * Fn, nhq, st), "shared swiglu");
     SMOE_TRY(gemv(sh_down_t(g), w->down_sh, nhq, Fn, H, out, sg), "shared down");
     return SMOE_OK;

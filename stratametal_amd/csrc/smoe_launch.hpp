@@ -102,8 +102,9 @@ hipError_t launch_swiglu_q8(const float* gate, const float* up, int64_t n, uint8
 bool native_type(int type);
 int native_block_values(int type);
 int64_t native_row_bytes(int type, int64_t n);  // -1: not native, or n not a whole number of blocks
+// (with w2, a second matrix of the same type and shape into y2 by the same launch)
 hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y,
-                              int ldy, const float* sg, hipStream_t s);
+                              int ldy, const float* sg, hipStream_t s, const uint8_t* w2 = nullptr, float* y2 = nullptr);
 hipError_t launch_sigmoid_rows(float* y, int T, int n, const float* sg, hipStream_t s);  // y[t][.] *= sigmoid(sg[t])
 hipError_t launch_add_rows(float* y, const float* r, int T, int n, hipStream_t s);       // y[t][.] += r[t][.]
 hipError_t launch_q2_mmvq(const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y, hipStream_t s);

@@ -6,8 +6,9 @@
 // activations (metal/shaders/iq.metal:224-442), taken by 32 lanes -- lane l adds partials l, l + 32, ... in order
 // from 0 -- then an xor butterfly 16, 8, 4, 2, 1 (iq_row / iq_mmvq_body, metal/shaders/iq.metal:458-513).  Here a
 // 32-lane half wave owns one row, so that order runs unchanged (oracle: or_native_gemv, which is also the
-// reference's own host order, metal/src/pack_parity.cpp:2785-3475).  Bandwidth is not the aim: these are the shared
-// expert's few rows per layer.
+// reference's own host order, metal/src/pack_parity.cpp:2785-3475).  One partial is decoded into registers once
+// (NativePart) and taken against every column of a tile: a few columns read x from memory (k_mmvq_native), more stage
+// it in LDS (k_mmvq_native_cols).
 #include "smoe_device.hpp"
 #include "smoe_gemv.hpp"
 #include "smoe_launch.hpp"
@@ -29,9 +30,13 @@ template <> struct NativeType<12> { static constexpr int qk = 256, bytes = 144, 
 template <> struct NativeType<13> { static constexpr int qk = 256, bytes = 176, ipb = 16, step = 2; };
 template <> struct NativeType<14> { static constexpr int qk = 256, bytes = 210, ipb = 32, step = 1; };
 
-// Block fields are 2-byte aligned (every block size is even); a 32-bit field is read as two halves.
+// Block fields are 2-byte aligned (every block size is even); a 32-bit field is one load at that alignment.
 __device__ __forceinline__ uint32_t rd16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
-__device__ __forceinline__ int32_t rd32(const uint8_t* p) { return (int32_t)(rd16(p) | (rd16(p + 2) << 16)); }
+__device__ __forceinline__ int32_t rd32(const uint8_t* p) {
+    int32_t v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 4);
+    return v;
+}
 __device__ __forceinline__ float rdh(const uint8_t* p) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)rd16(p));  // exact fp16 -> f32
 }
@@ -41,18 +46,14 @@ __device__ __forceinline__ int32_t qword(const uint8_t* b, int w) {
 }
 __device__ __forceinline__ int32_t dot4(int32_t a, int32_t b, int32_t c) { return __builtin_amdgcn_sdot4(a, b, c, false); }
 
-__constant__ int8_t kNl4[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
-// the codebook bytes of the low and high nibbles of four code bytes
-__device__ __forceinline__ void nl_bytes(int32_t codes, int32_t& lo, int32_t& hi) {
-    uint32_t a = 0, b = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t c = ((uint32_t)codes >> (8 * i)) & 0xFFu;
-        a |= (uint32_t)(uint8_t)kNl4[c & 15u] << (8 * i);
-        b |= (uint32_t)(uint8_t)kNl4[c >> 4] << (8 * i);
-    }
-    lo = (int32_t)a;
-    hi = (int32_t)b;
+// The IQ4 codebook as bytes: four signed values from four 4-bit indices (one per byte), two byte permutes of the
+// table's halves and a select by the indices' top bit.
+__device__ __forceinline__ int32_t nl4_bytes(uint32_t idx) {
+    const uint32_t sel = idx & 0x07070707u;
+    const uint32_t lo = __builtin_amdgcn_perm(0xF6EADDCFu, 0xBFAD9881u, sel);  // -49 -35 -22 -10, -127 -104 -83 -65
+    const uint32_t hi = __builtin_amdgcn_perm(0x71594535u, 0x26190D01u, sel);  // 53 69 89 113, 1 13 25 38
+    const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xFFu;
+    return (int32_t)((hi & m) | (lo & ~m));
 }
 
 // Q4_K / Q5_K: the 6-bit scale and min pair of two 32-value groups (iq_k_scale_min, metal/shaders/iq.metal:254-262)
@@ -67,61 +68,133 @@ __device__ __forceinline__ void k_scale_min(const uint8_t* s, int bq8_offset, in
     mn[1] = (int)((a1 >> 8) & 0xFFu);
 }
 
-// One partial of a row: block `blk`, its q8_1 blocks from x0, part iqs.  Integer sums are exact; the float steps
-// are the reference's, one rounding each (no contraction).
+// The activations of one 32-value block as the partials read them: the int8 words and the scale.  In memory a q8_1
+// block (fp16 scale first), in LDS eight words and then the scale in f32 (kXlDw dwords per block: an odd pitch).
+constexpr int kXlDw = 9;
+struct XMem {
+    const uint8_t* p;
+    __device__ __forceinline__ XMem at(int block) const { return {p + (size_t)block * 36}; }
+    __device__ __forceinline__ int32_t word(int w) const { return qword(p, w); }
+    __device__ __forceinline__ float scale() const { return rdh(p); }
+};
+struct XLds {
+    const uint32_t* p;
+    __device__ __forceinline__ XLds at(int block) const { return {p + kXlDw * block}; }
+    __device__ __forceinline__ int32_t word(int w) const { return (int32_t)p[w]; }
+    __device__ __forceinline__ float scale() const { return __uint_as_float(p[8]); }
+};
+
+// One partial of a row (part iqs of a block), decoded once: signed bytes whose integer dots are the reference's (an
+// offset it subtracts after the dot is subtracted from each byte: the same integer).  dot(x): the partial against a
+// column's activations of the block (x its first 32-value block); the float steps are the reference's, one rounding
+// each (no contraction).
 template <int TYPE>
-__device__ __forceinline__ float native_part(const uint8_t* __restrict__ blk, const uint8_t* __restrict__ x0, int iqs) {
-    if constexpr (TYPE == 8) {  // Q8_0
+struct NativePart;
+
+template <>
+struct NativePart<8> {  // Q8_0
+    int32_t w[8];
+    float d;
+    __device__ __forceinline__ void decode(const uint8_t* blk, int) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j] = rd32(blk + 2 + 4 * j);
+        d = rdh(blk);
+    }
+    template <class X>
+    __device__ __forceinline__ float dot(const X& x, int) const {
         int32_t s = 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) s = dot4(rd32(blk + 2 + 4 * (iqs + j)), qword(x0, iqs + j), s);
-        return (rdh(blk) * rdh(x0)) * (float)s;
-    } else if constexpr (TYPE == 2 || TYPE == 6) {  // Q4_0: nibble - 8; Q5_0: (nibble | high bit << 4) - 16
-        const uint8_t* qs = blk + (TYPE == 2 ? 2 : 6);
-        int32_t s = 0, a = 0;
+        for (int j = 0; j < 8; ++j) s = dot4(w[j], x.word(j), s);
+        return (d * x.scale()) * (float)s;
+    }
+};
+
+template <int TYPE>
+struct NativePart16 {  // Q4_0, Q5_0, IQ4_NL: 16 values of a 32-value block, words iqs, iqs + 1 and 4 words on
+    int32_t lo[2], hi[2];
+    float d;
+    __device__ __forceinline__ void decode(const uint8_t* blk, int iqs) {
+        const uint8_t* qs = blk + (TYPE == 6 ? 6 : 2);
+        uint32_t h = 0;
+        if constexpr (TYPE == 6) h = (uint32_t)rd32(blk + 2);
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int32_t v = rd32(qs + 4 * (iqs + i));
-            int32_t lo = v & 0x0F0F0F0F, hi = (v >> 4) & 0x0F0F0F0F;
-            if constexpr (TYPE == 6) {
-                const uint32_t h = (uint32_t)rd32(blk + 2) >> (4 * (iqs + i));
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    lo |= (int32_t)(((h >> b) & 1u) << (8 * b + 4));
-                    hi |= (int32_t)(((h >> (16 + b)) & 1u) << (8 * b + 4));
-                }
+            const uint32_t v = (uint32_t)rd32(qs + 4 * (iqs + i));
+            uint32_t a = v & 0x0F0F0F0Fu, b = (v >> 4) & 0x0F0F0F0Fu;
+            if constexpr (TYPE == 20) {
+                lo[i] = nl4_bytes(a);
+                hi[i] = nl4_bytes(b);
+                continue;
             }
-            const int32_t u0 = qword(x0, iqs + i), u1 = qword(x0, iqs + i + 4);
-            s = dot4(lo, u0, s);
-            s = dot4(hi, u1, s);
-            a = dot4(0x01010101, u0, a);
-            a = dot4(0x01010101, u1, a);
+            if constexpr (TYPE == 6) {  // value - 16: with the high bit the nibble, else the nibble | 0xF0
+                const uint32_t hs = h >> (4 * (iqs + i));
+                uint32_t ha = 0, hb = 0;  // 1 where the high bit is clear
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    ha |= ((~hs >> k) & 1u) << (8 * k);
+                    hb |= ((~hs >> (16 + k)) & 1u) << (8 * k);
+                }
+                a |= ha * 0xF0u;
+                b |= hb * 0xF0u;
+            } else {  // nibble - 8: bytes of n ^ 8, sign-extended from bit 3
+                a ^= 0x08080808u;
+                b ^= 0x08080808u;
+                a |= ((a >> 3) & 0x01010101u) * 0xF0u;
+                b |= ((b >> 3) & 0x01010101u) * 0xF0u;
+            }
+            lo[i] = (int32_t)a;
+            hi[i] = (int32_t)b;
         }
-        return (rdh(blk) * rdh(x0)) * (float)(s - (TYPE == 2 ? 8 : 16) * a);
-    } else if constexpr (TYPE == 20) {  // IQ4_NL
+        d = rdh(blk);
+    }
+    template <class X>
+    __device__ __forceinline__ float dot(const X& x, int iqs) const {
         int32_t s = 0;
 #pragma unroll
-        for (int l = 0; l < 2; ++l) {
-            int32_t lo, hi;
-            nl_bytes(rd32(blk + 2 + 4 * (iqs + l)), lo, hi);
-            s = dot4(lo, qword(x0, iqs + l), s);
-            s = dot4(hi, qword(x0, iqs + l + 4), s);
+        for (int i = 0; i < 2; ++i) {
+            s = dot4(lo[i], x.word(iqs + i), s);
+            s = dot4(hi[i], x.word(iqs + i + 4), s);
         }
-        return (rdh(blk) * rdh(x0)) * (float)s;
-    } else if constexpr (TYPE == 23) {  // IQ4_XS: 32-value group iqs / 4, its 6-bit scale - 32
-        const uint8_t* x = x0 + (size_t)(iqs / 4) * 36;
+        return (d * x.scale()) * (float)s;
+    }
+};
+template <> struct NativePart<2> : NativePart16<2> {};
+template <> struct NativePart<6> : NativePart16<6> {};
+template <> struct NativePart<20> : NativePart16<20> {};
+
+template <>
+struct NativePart<23> {  // IQ4_XS: 32-value group iqs / 4, its 6-bit scale - 32
+    int32_t lo[4], hi[4], ls;
+    float d;
+    __device__ __forceinline__ void decode(const uint8_t* blk, int iqs) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t v = (uint32_t)rd32(blk + 8 + 4 * (iqs + j));
+            lo[j] = nl4_bytes(v & 0x0F0F0F0Fu);
+            hi[j] = nl4_bytes((v >> 4) & 0x0F0F0F0Fu);
+        }
+        ls = (((blk[4 + iqs / 8] >> (iqs & 4)) & 15) | (int)(((rd16(blk + 2) >> (iqs / 2)) & 3u) << 4)) - 32;
+        d = rdh(blk);
+    }
+    template <class X>
+    __device__ __forceinline__ float dot(const X& x0, int iqs) const {
+        const X x = x0.at(iqs / 4);
         int32_t s = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            int32_t lo, hi;
-            nl_bytes(rd32(blk + 8 + 4 * (iqs + j)), lo, hi);
-            s = dot4(lo, qword(x, j), s);
-            s = dot4(hi, qword(x, j + 4), s);
+            s = dot4(lo[j], x.word(j), s);
+            s = dot4(hi[j], x.word(j + 4), s);
         }
-        const int ls = ((blk[4 + iqs / 8] >> (iqs & 4)) & 15) | (int)(((rd16(blk + 2) >> (iqs / 2)) & 3u) << 4);
-        s *= ls - 32;
-        return (rdh(blk) * rdh(x)) * (float)s;
-    } else if constexpr (TYPE == 12 || TYPE == 13) {  // Q4_K, Q5_K
+        return (d * x.scale()) * (float)(s * ls);
+    }
+};
+
+template <int TYPE>
+struct NativePartK {  // Q4_K, Q5_K: 8 values of two 32-value groups
+    int32_t p[2][2];
+    int sc[2], mn[2];
+    float d, dmin;
+    __device__ __forceinline__ void decode(const uint8_t* blk, int iqs) {
         constexpr bool q5 = TYPE == 13;
         const int bq8_offset = 2 * ((iqs / 2) / 4), qoff = (iqs / 2) % 4;
         const uint8_t* ql = blk + (q5 ? 48 : 16);
@@ -132,83 +205,145 @@ __device__ __forceinline__ float native_part(const uint8_t* __restrict__ blk, co
             vh0 = rd32(blk + 16 + 4 * qoff) >> bq8_offset;
             vh1 = rd32(blk + 32 + 4 * qoff) >> bq8_offset;
         }
-        int sc[2], mn[2];
         k_scale_min(blk + 4, bq8_offset, sc, mn);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            p[i][0] = (v0 >> (4 * i)) & 0x0F0F0F0F;
+            p[i][1] = (v1 >> (4 * i)) & 0x0F0F0F0F;
+            if constexpr (q5) {
+                p[i][0] |= ((vh0 >> i) << 4) & 0x10101010;
+                p[i][1] |= ((vh1 >> i) << 4) & 0x10101010;
+            }
+        }
+        d = rdh(blk);
+        dmin = rdh(blk + 2);
+    }
+    template <class X>
+    __device__ __forceinline__ float dot(const X& x0, int iqs) const {
+        const int bq8_offset = 2 * ((iqs / 2) / 4), qoff = (iqs / 2) % 4;
         float sum_d = 0.0f, sum_m = 0.0f;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const uint8_t* b8 = x0 + (size_t)(bq8_offset + i) * 36;
-            const float d8 = rdh(b8);
-            const int32_t u0 = qword(b8, qoff), u1 = qword(b8, qoff + 4);
-            int32_t p0 = (v0 >> (4 * i)) & 0x0F0F0F0F, p1 = (v1 >> (4 * i)) & 0x0F0F0F0F;
-            if constexpr (q5) {
-                p0 |= ((vh0 >> i) << 4) & 0x10101010;
-                p1 |= ((vh1 >> i) << 4) & 0x10101010;
-            }
-            const int32_t dq = dot4(p1, u1, dot4(p0, u0, 0));
+            const X x = x0.at(bq8_offset + i);
+            const float d8 = x.scale();
+            const int32_t u0 = x.word(qoff), u1 = x.word(qoff + 4);
+            const int32_t dq = dot4(p[i][1], u1, dot4(p[i][0], u0, 0));
             const int32_t da = dot4(0x01010101, u1, dot4(0x01010101, u0, 0));
             sum_d = sum_d + d8 * (float)(dq * sc[i]);
             sum_m = sum_m + d8 * (float)(da * mn[i]);
         }
-        return rdh(blk) * sum_d - rdh(blk + 2) * sum_m;
-    } else if constexpr (TYPE == 11) {  // Q3_K: 2 low bits, - 4 where the high bit is clear; scale - 32
+        return d * sum_d - dmin * sum_m;
+    }
+};
+template <> struct NativePart<12> : NativePartK<12> {};
+template <> struct NativePart<13> : NativePartK<13> {};
+
+template <>
+struct NativePart<11> {  // Q3_K: 2 low bits, - 4 where the high bit is clear; scale - 32
+    int32_t v[4];
+    int sc[4];
+    float d;
+    __device__ __forceinline__ void decode(const uint8_t* blk, int iqs) {
         const int bq8_offset = 4 * (iqs / 8), scale_offset = iqs - (iqs % 8) + (iqs % 8) / 4;
-        const uint8_t* sc8 = blk + 96;
-        const int32_t vl = rd32(blk + 32 + 4 * iqs);
+        const uint32_t vl = (uint32_t)rd32(blk + 32 + 4 * iqs);
         const uint32_t vh = (~(uint32_t)rd32(blk + 4 * (iqs % 8))) >> bq8_offset;
+        // scale j = scale_offset + 2 i: its low nibble in byte j % 8 (the high half of the byte from j = 8 on), its high
+        // bits 2 (j / 4) of byte 8 + j % 4; scale_offset is 0, 1, 8 or 9
+        const uint32_t sl[2] = {(uint32_t)rd32(blk + 96), (uint32_t)rd32(blk + 100)};
+        const uint32_t sh = (uint32_t)rd32(blk + 104);
+        const int odd = scale_offset & 1, half = scale_offset >> 3;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t lo = sl[i >> 1] >> (8 * (odd + 2 * (i & 1)) + 4 * half);
+            const uint32_t hi = sh >> (8 * (odd + 2 * (i & 1)) + 2 * (2 * half + (i >> 1)));
+            sc[i] = (int)((lo & 15u) | ((hi & 3u) << 4)) - 32;
+            v[i] = (int32_t)(((vl >> (2 * i)) & 0x03030303u) | ((vh >> i) & 0x01010101u) * 0xFCu);
+        }
+        d = rdh(blk + 108);
+    }
+    template <class X>
+    __device__ __forceinline__ float dot(const X& x0, int iqs) const {
+        const X x = x0.at(4 * (iqs / 8));
         float sumf = 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int isc = scale_offset + 2 * i;
-            const int sc = (((sc8[isc % 8] >> (4 * (isc / 8))) & 15) | (((sc8[8 + (isc % 4)] >> (2 * (isc / 4))) & 3) << 4)) -
-                           32;
-            const uint8_t* b8 = x0 + (size_t)(bq8_offset + i) * 36;
-            const int32_t u = qword(b8, iqs % 8);
-            // the byte-wise difference (low - 4 * clear) dotted with u, as two exact dots
-            const int32_t dl = dot4((vl >> (2 * i)) & 0x03030303, u, 0);
-            const int32_t dh = dot4((int32_t)(((vh >> i) << 2) & 0x04040404u), u, 0);
-            sumf = sumf + rdh(b8) * (float)((dl - dh) * sc);
+            const X xi = x.at(i);
+            sumf = sumf + xi.scale() * (float)(dot4(v[i], xi.word(iqs % 8), 0) * sc[i]);
         }
-        return rdh(blk + 108) * sumf;
-    } else {  // Q6_K (14): (low nibble | 2 high bits << 4) - 32 times an int8 scale
-        static_assert(TYPE == 14, "native_part: unknown type");
-        const int bq8_offset = 4 * (iqs / 16) + (iqs % 16) / 8, scale_offset = 8 * (iqs / 16) + (iqs % 16) / 4;
-        const int vh_shift = 2 * ((iqs % 16) / 8);
-        const int32_t vl = rd32(blk + 4 * iqs);
+        return d * sumf;
+    }
+};
+
+template <>
+struct NativePart<14> {  // Q6_K: (low nibble | 2 high bits << 4) - 32 times an int8 scale
+    int32_t v[2];
+    int sc[2];
+    float d;
+    __device__ __forceinline__ void decode(const uint8_t* blk, int iqs) {
+        const int scale_offset = 8 * (iqs / 16) + (iqs % 16) / 4, vh_shift = 2 * ((iqs % 16) / 8);
+        const uint32_t vl = (uint32_t)rd32(blk + 4 * iqs);
         const uint32_t vh = (uint32_t)rd32(blk + 128 + 4 * (8 * (iqs / 16) + (iqs % 8))) >> vh_shift;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            sc[i] = (int)(int8_t)blk[192 + scale_offset + 4 * i];
+            // six bits - 32: bytes of v ^ 32, sign-extended from bit 5
+            const uint32_t q = (((vl >> (4 * i)) & 0x0F0F0F0Fu) | (((vh >> (4 * i)) << 4) & 0x30303030u)) ^ 0x20202020u;
+            v[i] = (int32_t)(q | ((q >> 5) & 0x01010101u) * 0xC0u);
+        }
+        d = rdh(blk + 208);
+    }
+    template <class X>
+    __device__ __forceinline__ float dot(const X& x0, int iqs) const {
+        const X x = x0.at(4 * (iqs / 16) + (iqs % 16) / 8);
         float sumf = 0.0f;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const int sc = (int)(int8_t)blk[192 + scale_offset + 4 * i];
-            const int32_t v = ((vl >> (4 * i)) & 0x0F0F0F0F) | (int32_t)(((vh >> (4 * i)) << 4) & 0x30303030u);
-            const uint8_t* b8 = x0 + (size_t)(bq8_offset + 2 * i) * 36;
-            const int32_t u = qword(b8, iqs % 8);
-            const int32_t d = dot4(v, u, 0) - dot4(0x20202020, u, 0);
-            sumf = sumf + rdh(b8) * (float)(d * sc);
+            const X xi = x.at(2 * i);
+            sumf = sumf + xi.scale() * (float)(dot4(v[i], xi.word(iqs % 8), 0) * sc[i]);
         }
-        return rdh(blk + 208) * sumf;
+        return d * sumf;
     }
-}
+};
 
 // y[c * ldy + r] = row r . column c (times sigmoid(sg[c]) when sg is given).  Grid (ceil(n_out / 8), column
-// groups); a 32-lane half wave per row; a work-group takes columns blockIdx.y, + gridDim.y, ...
+// groups, matrices: w into y, then w2 into y2); a 32-lane half wave per row; a work-group takes columns blockIdx.y,
+// + gridDim.y, ...
 template <int TYPE>
-__global__ __launch_bounds__(256) void k_mmvq_native(const uint8_t* __restrict__ w, int n_in, int n_out, int n_col,
-                                                     const uint8_t* __restrict__ xq, float* __restrict__ y, int ldy,
+__global__ __launch_bounds__(256) void k_mmvq_native(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
+                                                     int n_in, int n_out, int n_col, const uint8_t* __restrict__ xq,
+                                                     float* __restrict__ y, float* __restrict__ y2, int ldy,
                                                      const float* __restrict__ sg) {
     using NT = NativeType<TYPE>;
+    if (blockIdx.z) {
+        w = w2;
+        y = y2;
+    }
     const int hw = threadIdx.x >> 5, l = threadIdx.x & 31;
     const int r = blockIdx.x * 8 + hw;
     const size_t rb = (size_t)(n_in / NT::qk) * NT::bytes, xb = (size_t)(n_in / 32) * 36;
     const uint8_t* row = w + (size_t)(r < n_out ? r : n_out - 1) * rb;  // a dead half wave reads the last row
     const int npart = (n_in / NT::qk) * NT::ipb;
     for (int c = blockIdx.y; c < n_col; c += gridDim.y) {
-        const uint8_t* col = xq + (size_t)c * xb;
+        const XMem col{xq + (size_t)c * xb};
         float acc = 0.0f;
-        for (int k = l; k < npart; k += 32) {
-            const int kb = k / NT::ipb;
-            acc = acc + native_part<TYPE>(row + (size_t)kb * NT::bytes, col + (size_t)kb * (NT::qk / 32) * 36,
-                                          NT::step * (k % NT::ipb));
+        int k = l;
+        // four partials at a time: their loads are in flight together, their sums added in order (not the wider partials
+        // of Q4_K and Q5_K, 3.3 us against 3.9 for 512 rows of 2048)
+        for (; TYPE != 12 && TYPE != 13 && k + 96 < npart; k += 128) {
+            NativePart<TYPE> p[4];
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) p[j].decode(row + (size_t)((k + 32 * j) / NT::ipb) * NT::bytes, NT::step * ((k + 32 * j) % NT::ipb));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = p[j].dot(col.at((k + 32 * j) / NT::ipb * (NT::qk / 32)), NT::step * ((k + 32 * j) % NT::ipb));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc = acc + v[j];
+        }
+        for (; k < npart; k += 32) {
+            NativePart<TYPE> p;
+            p.decode(row + (size_t)(k / NT::ipb) * NT::bytes, NT::step * (k % NT::ipb));
+            acc = acc + p.dot(col.at(k / NT::ipb * (NT::qk / 32)), NT::step * (k % NT::ipb));
         }
         acc = acc + xor_swap<16>(acc);
         acc = acc + xor_swap<8>(acc);
@@ -216,6 +351,108 @@ __global__ __launch_bounds__(256) void k_mmvq_native(const uint8_t* __restrict__
         acc = acc + xor_swap<2>(acc);
         acc = acc + xor_swap<1>(acc);
         if (r < n_out && l == 0) y[(size_t)c * ldy + r] = sg ? acc * sigmoid(sg[c]) : acc;
+    }
+}
+
+// One exchange step of the scattering butterfly below: N values per lane become N / 2, each lane keeping the half its
+// lane bit D names, summed with lane ^ D's (the butterfly's addition: commutative, so the same bits in either lane).
+template <int D, int N>
+__device__ __forceinline__ void scatter_step(float* v, int lane) {
+    if constexpr (N == 1) {
+        v[0] = v[0] + __uint_as_float(xor_lane<D>(__float_as_uint(v[0])));
+    } else {
+        const bool up = (lane & D) != 0;
+#pragma unroll
+        for (int j = 0; j < N / 2; ++j) {
+            if constexpr (D == 16) {  // rows of 16 lanes: the swap leaves each output's two halves in the lanes that add them
+                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(v[j]), __float_as_int(v[j + N / 2]), false, false);
+                v[j] = __int_as_float(r[0]) + __int_as_float(r[1]);
+            } else {
+                const float keep = up ? v[j + N / 2] : v[j], send = up ? v[j] : v[j + N / 2];
+                v[j] = keep + __uint_as_float(xor_lane<D>(__float_as_uint(send)));
+            }
+        }
+    }
+}
+
+// The same product for C columns at a time: a half wave owns kRw rows; x of the column tile in LDS, kXlChunk values of
+// K at a time (a multiple of 32 partials of every type, so the order of a lane's partials is k_mmvq_native's); a partial
+// is decoded once and taken against the C columns.  The butterflies of the kRw * C sums run as one scattering butterfly
+// (each step halves the values a lane holds, 31 exchanges for 32 sums instead of 160), and the results go out through
+// LDS as whole runs of a column's rows.  On 1000 columns, a work-group per column decoding the rows again and this: Q3_K
+// 512 x 2048 232 and 58 us, IQ4_NL 2048 x 512 609 and 36 us.  Bound by the VALU: about nine instructions per 16 products
+// for IQ4_NL, 22 for Q3_K.
+constexpr int kRw = 2, kXlChunk = 2048;
+template <int TYPE, int C>
+__global__ __launch_bounds__(256) void k_mmvq_native_cols(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
+                                                          int n_in, int n_out, int n_col,
+                                                          const uint8_t* __restrict__ xq, float* __restrict__ y,
+                                                          float* __restrict__ y2, int ldy, const float* __restrict__ sg) {
+    using NT = NativeType<TYPE>;
+    constexpr int N = kRw * C;
+    static_assert(N <= 32 && (N & (N - 1)) == 0, "a scattering butterfly over 32 lanes");
+    extern __shared__ __align__(16) uint32_t xl[];  // [C][chunk blocks][kXlDw]
+    __shared__ float ot[C][8 * kRw + 1];
+    if (blockIdx.z) {
+        w = w2;
+        y = y2;
+    }
+    const int hw = threadIdx.x >> 5, l = threadIdx.x & 31;
+    const int r0 = blockIdx.x * 8 * kRw, c0 = blockIdx.y * C;
+    const size_t rb = (size_t)(n_in / NT::qk) * NT::bytes;
+    const uint8_t* row[kRw];
+#pragma unroll
+    for (int j = 0; j < kRw; ++j) row[j] = w + (size_t)min(r0 + hw * kRw + j, n_out - 1) * rb;  // dead rows read the last
+    const uint32_t* xd = reinterpret_cast<const uint32_t*>(xq);  // 36-byte blocks: whole dwords
+    const int xb = n_in / 32 * 9;                                // dwords of a column
+    float acc[N];
+#pragma unroll
+    for (int o = 0; o < N; ++o) acc[o] = 0.0f;
+    for (int v0 = 0; v0 < n_in; v0 += kXlChunk) {
+        const int vals = min(kXlChunk, n_in - v0), nb = vals / 32;  // 32-value blocks of this chunk
+        const int npart = vals / NT::qk * NT::ipb, kb0 = v0 / NT::qk;
+        if (v0) __syncthreads();
+        for (int p = threadIdx.x; p < C * nb; p += 256) {  // a block per thread: its words, then its scale
+            const int c = p / nb;
+            const uint32_t* src = xd + (size_t)min(c0 + c, n_col - 1) * xb + (size_t)(v0 / 32 + p - c * nb) * 9;
+            uint32_t v[9];
+#pragma unroll
+            for (int m = 0; m < 9; ++m) v[m] = src[m];
+#pragma unroll
+            for (int m = 1; m < 9; ++m) xl[p * kXlDw + m - 1] = v[m];
+            xl[p * kXlDw + 8] = __float_as_uint((float)__builtin_bit_cast(_Float16, (uint16_t)(v[0] & 0xFFFFu)));
+        }
+        __syncthreads();
+        for (int k = l; k < npart; k += 32) {
+            const int kb = k / NT::ipb, iqs = NT::step * (k % NT::ipb);
+            NativePart<TYPE> part[kRw];
+#pragma unroll
+            for (int j = 0; j < kRw; ++j) part[j].decode(row[j] + (size_t)(kb0 + kb) * NT::bytes, iqs);
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const XLds x{xl + (c * nb + kb * (NT::qk / 32)) * kXlDw};
+#pragma unroll
+                for (int j = 0; j < kRw; ++j) acc[j * C + c] = acc[j * C + c] + part[j].dot(x, iqs);
+            }
+        }
+    }
+    scatter_step<16, N>(acc, l);
+    scatter_step<8, (N > 2 ? N / 2 : 1)>(acc, l);
+    scatter_step<4, (N > 4 ? N / 4 : 1)>(acc, l);
+    scatter_step<2, (N > 8 ? N / 8 : 1)>(acc, l);
+    scatter_step<1, (N > 16 ? N / 16 : 1)>(acc, l);
+    constexpr int kDup = 32 / N;  // lanes that end with the same sum
+    if (l % kDup == 0) {
+        const int o = l / kDup, j = o / C, c = o % C;
+        ot[c][hw * kRw + j] = acc[0];
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < C * 8 * kRw; p += 256) {
+        const int c = p / (8 * kRw), r = p % (8 * kRw);
+        if (c0 + c < n_col && r0 + r < n_out) {
+            const float v = ot[c][r];
+            y[(size_t)(c0 + c) * ldy + r0 + r] = sg ? v * sigmoid(sg[c0 + c]) : v;
+        }
     }
 }
 
@@ -267,12 +504,38 @@ int64_t native_row_bytes(int type, int64_t n) {
     return (n <= 0 || n % qk) ? -1 : n / qk * bytes;
 }
 
+// Columns per work-group: the most of 16, 8 and 4 that leaves the chip two work-groups per CU, else 4.  Below
+// kColsGroupsMin work-groups of 4 columns, a work-group per column and eight rows: a tile's chain of columns is then the
+// longer one (by type, 512 x 2048 at 16 columns: 3.9 to 6.6 us against 5.0 to 8.5 in tiles, at 32 columns 5.8 to 10.9
+// against 4.1 to 8.4; 2048 x 512 at 4 columns 2.9 against 3.5, at 8 columns 3.8 to 4.3 against 3.1).
+constexpr int kColsGroups = 512, kColsGroupsMin = 224;
+
 hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y,
-                              int ldy, const float* sg, hipStream_t s) {
+                              int ldy, const float* sg, hipStream_t s, const uint8_t* w2, float* y2) {
     if (!native_type(type) || n_in % native_block_values(type)) return hipErrorInvalidValue;
+    const unsigned nz = w2 ? 2 : 1;
+    const int rg = (n_out + 8 * kRw - 1) / (8 * kRw);
+    int cols = 1;
+    if ((int64_t)rg * ((n_col + 3) / 4) * nz >= kColsGroupsMin && n_col >= 4 && n_col / 4 < 65535) {
+        cols = 4;
+        for (int c = 16; c > 4; c /= 2)
+            if ((int64_t)rg * ((n_col + c - 1) / c) * nz >= kColsGroups) {
+                cols = c;
+                break;
+            }
+    }
     const int cg = n_col < 64 ? n_col : 64;
-    dim3 grid((unsigned)((n_out + 7) / 8), (unsigned)cg);
-#define SMOE_NAT(T) hipLaunchKernelGGL(k_mmvq_native<T>, grid, dim3(256), 0, s, w, n_in, n_out, n_col, xq, y, ldy, sg)
+    const dim3 grid1((unsigned)((n_out + 7) / 8), (unsigned)cg, nz);
+    const dim3 gridc((unsigned)rg, (unsigned)((n_col + cols - 1) / cols), nz);
+    const size_t lds = (size_t)cols * (n_in < kXlChunk ? n_in : kXlChunk) / 32 * kXlDw * 4;
+#define SMOE_NATC(T, C) \
+    hipLaunchKernelGGL((k_mmvq_native_cols<T, C>), gridc, dim3(256), lds, s, w, w2, n_in, n_out, n_col, xq, y, y2, ldy, sg)
+#define SMOE_NAT(T)                                                                                                  \
+    if (cols == 16) SMOE_NATC(T, 16);                                                                                \
+    else if (cols == 8) SMOE_NATC(T, 8);                                                                             \
+    else if (cols == 4) SMOE_NATC(T, 4);                                                                             \
+    else                                                                                                             \
+        hipLaunchKernelGGL(k_mmvq_native<T>, grid1, dim3(256), 0, s, w, w2, n_in, n_out, n_col, xq, y, y2, ldy, sg)
     switch (type) {
         case 8: SMOE_NAT(8); break;
         case 2: SMOE_NAT(2); break;
@@ -285,6 +548,7 @@ hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int
         default: SMOE_NAT(14); break;
     }
 #undef SMOE_NAT
+#undef SMOE_NATC
     return hipGetLastError();
 }
 

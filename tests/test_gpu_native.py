@@ -66,6 +66,25 @@ def test_mmvq_native_bitwise(torch, t):
         assert np.array_equal(bits(host(torch, y)), bits(want)), (n_in, n_out, n_col)
 
 
+@pytest.mark.parametrize("t", TYPES)
+def test_mmvq_native_column_tiles_bitwise(torch, t):
+    """Column tiles of 4, 8 and 16 (by rows and columns: smoe_native.hip's rule) with remainders of rows, columns and
+    of the 2048 values of K staged at a time."""
+    qk = O.NATIVE[t][0]
+    for n_in, n_out, n_col in [(qk, 895, 16), (2048 + qk, 1031, 15), (4096 + qk, 512, 29), (256, 2047, 30), (256, 2048, 50),
+                               (2304, 1025, 131), (256, 16, 900)]:
+        print(f"case: mmvq type {t} n_in={n_in} n_out={n_out} n_col={n_col}", flush=True)
+        w = O.gen_native_blocks(t, 8, n_in + n_out, n_in * n_out)
+        xq = O.quant_q8_1(O.gen_normal(t, n_in, n_col * n_in).reshape(n_col, n_in))
+        y = torch.full((n_col * n_out + 16,), 7.0, dtype=torch.float32, device="cuda")
+        wd, xd = dev(torch, w), dev(torch, xq)
+        S._check(S.lib().smoe_mmvq(t, wd.data_ptr(), 0, xd.data_ptr(), n_in, n_out, n_col, y.data_ptr(), S._stream()))
+        got = host(torch, y)
+        assert (got[n_col * n_out:] == 7.0).all(), "guard words written"
+        want = O.native_gemv(t, w, xq, n_in, n_out, n_col)
+        assert np.array_equal(bits(got[:n_col * n_out].reshape(n_col, n_out)), bits(want)), (n_in, n_out, n_col)
+
+
 def test_mmvq_native_refusals(torch):
     say("case: mmvq native refusals")
     w = torch.zeros(1024, dtype=torch.uint8, device="cuda")
