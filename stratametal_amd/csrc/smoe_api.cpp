@@ -58,6 +58,10 @@ constexpr int kFusedRouteTokens = 4;
 constexpr int kDispatchMultiPairs = 2048;
 // SMOE_PATH_AUTO runs the MFMA (prefill) contract from this many tokens on.
 constexpr int kMfmaTokens = 128;
+// The decode path runs the junction as a kernel of its own from this many tokens on: before, its fusion into the router
+// kernel saves the launch; from here on the tiled router gains more (junction and router, 512 experts of 2048: 9.9 us fused
+// and 10.0 apart at 8 tokens, 10.3 and 9.7 at 12, 14.6 and 9.8 at 16, 28.8 and 12.0 at 48).
+constexpr int kJunctionApartTokens = 12;
 // The MFMA kernels' buffer offsets into the activation and h records are 31-bit.
 constexpr size_t kMfmaRecordLimit = (size_t)1 << 31;
 // The prefill path's Y (f32 per-pair rows) from this size on is stored and read with streaming accesses (half the
@@ -453,7 +457,8 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
         if (_m != SMOE_OK) return _m;        \
     } while (0)
     SMOE_MARK();
-    const bool fused_norm = x_prev && !mfma;
+    // the junction is fused into the router kernel of few tokens; more tokens take it as a kernel of its own
+    const bool fused_norm = x_prev && !mfma && n_tokens < kJunctionApartTokens;
     // the expert stages of the trace: the decode path's unfused kernels, so that every stage lands in memory
     const bool stages = trace && (trace->xq || trace->hq || trace->parts || trace->shared || trace->egate ||
                                   trace->eup || trace->sgu || trace->shq);
@@ -474,6 +479,8 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
     if (x_prev && mfma)
         SMOE_TRY(smoe::launch_junction_records(x_prev, r_prev, T, H, eps, x_io, ximg, xbf, st, xflags),
                  "junction records");
+    if (x_prev && !mfma && !fused_norm)
+        SMOE_TRY(smoe::launch_residual_rmsnorm(x_prev, r_prev, T, H, eps, x_io, st), "junction");
     if (mfma && !x_prev)
         SMOE_TRY(smoe::launch_act_records(x, (int64_t)T * (H / 64), ximg, xbf, st, xflags), "activation records");
     // the f32 router (router_dtype 1) reads f32 x on the row-per-wave path, also for many tokens

@@ -595,6 +595,169 @@ __global__ __launch_bounds__(256) void k_router(int H, int E, int T, int tok_til
     SMOE_STAMP(0, 10);
 }
 
+// The same logits for many tokens, bit for bit: a wave takes RR rows against a tile of TT tokens, so that a staged x
+// chunk serves RR rows and a weight chunk TT tokens.  K runs in stages of 512 values: x of the tile (bf16, or f32 for
+// the f32 router) through two LDS buffers, the next stage's x and weights in flight in registers, one barrier per
+// stage.  A (row, token)'s chain is k_router's: lane l adds the chunks l, l + 64, ... in element order (past the row's
+// end zeros: no sum that starts at +0 changes), then the butterfly 32 .. 1, here one scattering butterfly of the RR * TT
+// sums (63 exchanges for 64 sums instead of 384).  The shared gate row goes one wave per token (n_gate work-groups behind
+// the tiles), then the q8_1 images, eight blocks per work-group.  k_router re-reads and re-stages x for every four rows
+// and reduces every sum by itself: 512 experts of 2048 bf16 values 20 us at 64 tokens and 126 at 600, of 2560 f32 values
+// 84 us at 77; bound by the VALU here (an fma per product, a quarter more to unpack bf16).
+constexpr int kRtStage = 512;
+// Two f32 to bf16 (round to nearest even) by the hardware's packed conversion: f32_to_bf16's bits but for the payload of
+// a NaN, which makes a NaN of every sum either way.
+__device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
+template <bool F32, int RR, int TT>
+__global__ __launch_bounds__(256) void k_router_tile(int H, int E, int T, int n_tiles, const void* __restrict__ W,
+                                                      const float* __restrict__ xf, const uint16_t* __restrict__ xb,
+                                                      int n_rb, int n_tb, int by_tok, int n_gate,
+                                                      const uint16_t* __restrict__ w_inp,
+                                                      const float* __restrict__ bias, float* __restrict__ logits,
+                                                      int ld_logits, float* __restrict__ sg,
+                                                      uint32_t* __restrict__ ximg, int img_natural) {
+    constexpr int CH = F32 ? 4 : 8;               // values of a 16-byte weight piece
+    constexpr int JS = kRtStage / (64 * CH);      // a lane's pieces per stage
+    constexpr int XP = kRtStage / CH;             // 16-byte LDS pieces of a token's stage
+    constexpr int XU = TT * XP / 256;             // a thread's pieces
+    constexpr int N = RR * TT;
+    static_assert(N <= 64 && (N & (N - 1)) == 0 && TT * XP % 256 == 0, "a scattering butterfly over the wave");
+    __shared__ __align__(16) uint4 xs[2][TT * XP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int id = blockIdx.x;
+    if (id >= n_tiles) {
+        id -= n_tiles;
+        if (id < n_gate) {  // the shared gate: bf16(x) . w_inp, k_router's order
+            const int t = id * 4 + wave;
+            if (t >= T) return;
+            float acc = 0.0f;
+            for (int c = lane; c < H >> 3; c += 64) {
+                const uint4 wv = reinterpret_cast<const uint4*>(w_inp)[c];
+                const float4* src = reinterpret_cast<const float4*>(xf + (size_t)t * H) + 2 * c;
+                const float4 a = src[0], b = src[1];
+                const uint32_t wq[4] = {wv.x, wv.y, wv.z, wv.w};
+                const float x8[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    acc = __builtin_fmaf(u2f(f32_to_bf16(x8[2 * q]) << 16), u2f(wq[q] << 16), acc);
+                    acc = __builtin_fmaf(u2f(f32_to_bf16(x8[2 * q + 1]) << 16), u2f(wq[q] & 0xFFFF0000u), acc);
+                }
+            }
+            acc = wave_sum_xor_fast(acc);
+            if (lane == 0) sg[t] = acc;
+            return;
+        }
+        const int64_t blk = (int64_t)(id - n_gate) * 8 + (tid >> 5);
+        const bool live = blk < (int64_t)T * (H >> 5);
+        const float v = xf[(live ? blk : 0) * 32 + (tid & 31)];
+        uint8_t* sc = reinterpret_cast<uint8_t*>(xs) + 32 * (tid >> 5);
+        q8_image_store(v, live, sc, ximg + (live ? blk : 0) * kImgDw, img_natural != 0);
+        return;
+    }
+    // the tiles of one row group (or, by_tok, of one token tile) on one XCD
+    const int o = id >> 3, m = by_tok ? n_rb : n_tb;
+    const int hi = (o / m) * 8 + (id & 7), lo = o % m;
+    const int rb = by_tok ? lo : hi, tb = by_tok ? hi : lo;
+    if (rb >= n_rb || tb >= n_tb) return;  // (the padding of hi to whole groups of 8)
+    const int t0 = tb * TT, row0 = (rb * 4 + wave) * RR;
+    const uint8_t* wr[RR];
+#pragma unroll
+    for (int i = 0; i < RR; ++i)
+        wr[i] = static_cast<const uint8_t*>(W) + (size_t)min(row0 + i, E - 1) * H * (F32 ? 4 : 2);
+    uint4 wn[JS][RR], xn[XU];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < JS; ++j) {
+            const int c = k0 + (lane + 64 * j) * CH;
+#pragma unroll
+            for (int i = 0; i < RR; ++i)
+                wn[j][i] = c < H ? *reinterpret_cast<const uint4*>(wr[i] + (size_t)c * (F32 ? 4 : 2)) : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < XU; ++u) {
+            const int p = tid + 256 * u, t = min(t0 + p / XP, T - 1), c = k0 + (p % XP) * CH;
+            uint4 v = make_uint4(0, 0, 0, 0);
+            if (c < H) {
+                if constexpr (F32) {
+                    v = *reinterpret_cast<const uint4*>(xf + (size_t)t * H + c);
+                } else if (xf) {
+                    const float4* src = reinterpret_cast<const float4*>(xf + (size_t)t * H + c);
+                    const float4 a = src[0], b = src[1];
+                    v = make_uint4(pk_bf16(a.x, a.y), pk_bf16(a.z, a.w), pk_bf16(b.x, b.y), pk_bf16(b.z, b.w));
+                } else {
+                    v = *reinterpret_cast<const uint4*>(xb + (size_t)t * H + c);
+                }
+            }
+            xn[u] = v;
+        }
+    };
+    load(0);
+    float acc[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = 0.0f;
+    int buf = 0;
+    for (int k0 = 0; k0 < H; k0 += kRtStage, buf ^= 1) {
+        uint4 w[JS][RR];
+#pragma unroll
+        for (int j = 0; j < JS; ++j)
+#pragma unroll
+            for (int i = 0; i < RR; ++i) w[j][i] = wn[j][i];
+#pragma unroll
+        for (int u = 0; u < XU; ++u) xs[buf][tid + 256 * u] = xn[u];
+        __syncthreads();  // (the buffer written next was read two barriers ago)
+        if (k0 + kRtStage < H) load(k0 + kRtStage);
+#pragma unroll
+        for (int j = 0; j < JS; ++j) {
+            float wv[RR][CH];
+#pragma unroll
+            for (int i = 0; i < RR; ++i) {
+                const uint32_t q[4] = {w[j][i].x, w[j][i].y, w[j][i].z, w[j][i].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (F32) {
+                        wv[i][e] = u2f(q[e]);
+                    } else {
+                        wv[i][2 * e] = u2f(q[e] << 16);
+                        wv[i][2 * e + 1] = u2f(q[e] & 0xFFFF0000u);
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const uint4 xv = xs[buf][t * XP + lane + 64 * j];
+                const uint32_t q[4] = {xv.x, xv.y, xv.z, xv.w};
+                float x[CH];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (F32) {
+                        x[e] = u2f(q[e]);
+                    } else {
+                        x[2 * e] = u2f(q[e] << 16);
+                        x[2 * e + 1] = u2f(q[e] & 0xFFFF0000u);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < RR; ++i)
+#pragma unroll
+                    for (int e = 0; e < CH; ++e) acc[t * RR + i] = __builtin_fmaf(x[e], wv[i][e], acc[t * RR + i]);
+            }
+        }
+    }
+    scatter_step<32, N>(acc, lane);
+    scatter_step<16, (N > 2 ? N / 2 : 1)>(acc, lane);
+    scatter_step<8, (N > 4 ? N / 4 : 1)>(acc, lane);
+    scatter_step<4, (N > 8 ? N / 8 : 1)>(acc, lane);
+    scatter_step<2, (N > 16 ? N / 16 : 1)>(acc, lane);
+    scatter_step<1, (N > 32 ? N / 32 : 1)>(acc, lane);
+    constexpr int kDup = 64 / N;  // lanes that end with the same sum
+    if (lane % kDup) return;
+    const int out = lane / kDup, row = row0 + out % RR, t = t0 + out / RR;
+    if (row < E && t < T) logits[(size_t)t * ld_logits + row] = bias ? acc[0] + bias[row] : acc[0];
+}
 
 // One stage of a reduce-scatter over per-lane values v[0 .. N): at distance D a lane keeps the half of its items
 // selected by its bit D and adds the partner's copy of them, so every item's sum is formed by exactly the additions
@@ -2684,6 +2847,28 @@ static unsigned router_grid_x(int blocks, int T, int tile) {
     return (unsigned)(T > tile ? (blocks + 7) / 8 * 8 : blocks);
 }
 
+// From kRouterTileTokens tokens a call without the fused junction runs k_router_tile: 512 rows of 2048, k_router and the
+// tiles, bf16 6.3 and 6.3 us at 5 tokens, 8.4 and 6.4 at 16, 19.8 and 7.7 at 64, 126 and 38 at 600; f32 7.8 and 5.9 at 5,
+// 27 and 7.1 at 64, 204 and 41 at 600.  The tile: few tokens need the work-groups (bf16 4 rows by 4 tokens, f32 2 by 8),
+// from kRouterTileWide on 4 by 8 re-reads less (bf16 9.6 against 10.4 us at 100 tokens, 11.4 against 10.7 at 127).
+constexpr int kRouterTileTokens = 5, kRouterTileWide = 112;
+
+template <bool F32, int RR, int TT>
+static hipError_t launch_router_tile(const float* xf, const uint16_t* xb, const void* W, const uint16_t* w_inp,
+                                     const float* bias, int H, int E, int T, float* logits, int ld_logits, float* sg,
+                                     uint32_t* ximg, int img_natural, hipStream_t s) {
+    const int n_rb = (E + 4 * RR - 1) / (4 * RR), n_tb = (T + TT - 1) / TT;
+    // the smaller of x and W is what every XCD reads
+    const int by_tok = (int64_t)T * 4 > (int64_t)E * (F32 ? 4 : 2) ? 1 : 0;
+    const int64_t tiles = by_tok ? (int64_t)(n_tb + 7) / 8 * 8 * n_rb : (int64_t)(n_rb + 7) / 8 * 8 * n_tb;
+    const int64_t gate = w_inp ? (T + 3) / 4 : 0, img = ximg ? ((int64_t)T * (H / 32) + 7) / 8 : 0;
+    if (tiles + gate + img > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_router_tile<F32, RR, TT>), dim3((unsigned)(tiles + gate + img)), dim3(256), 0, s, H, E, T,
+                       (int)tiles, W, xf, xb, n_rb, n_tb, by_tok, (int)gate, w_inp, bias, logits, ld_logits, sg, ximg,
+                       img_natural);
+    return hipGetLastError();
+}
+
 hipError_t launch_router(const float* xf, const uint16_t* xb, const void* W, const uint16_t* w_inp,
                          const float* bias, int H, int E, int rows_total, int T, float* logits, int ld_logits, float* sg,
                          uint32_t* ximg, int tile_rows, int img_natural, hipStream_t s, const float* rprev, float eps,
@@ -2695,6 +2880,14 @@ hipError_t launch_router(const float* xf, const uint16_t* xb, const void* W, con
     if (clear_n16 && (tile_rows || !clear)) return hipErrorInvalidValue;
     // the f32 router runs on the row-per-wave path from f32 x
     if (w_f32 && (tile_rows || !xf || H % 4 || H > 4096)) return hipErrorInvalidValue;
+    const bool x16 = xf ? (reinterpret_cast<uintptr_t>(xf) & 15) == 0 : (reinterpret_cast<uintptr_t>(xb) & 15) == 0;
+    if (!tile_rows && !rprev && !clear_n16 && T >= kRouterTileTokens && x16 && H % 8 == 0 && (xf || !w_inp)) {
+#define SMOE_ROUTER_TILE(F, RR, TT) \
+    launch_router_tile<F, RR, TT>(xf, xb, W, w_inp, bias, H, E, T, logits, ld_logits, sg, ximg, img_natural, s)
+        if (T >= kRouterTileWide) return w_f32 ? SMOE_ROUTER_TILE(true, 4, 8) : SMOE_ROUTER_TILE(false, 4, 8);
+        return w_f32 ? SMOE_ROUTER_TILE(true, 2, 8) : SMOE_ROUTER_TILE(false, 4, 4);
+#undef SMOE_ROUTER_TILE
+    }
     if (w_f32) {
         const int maxc4 = (H / 4 + 63) / 64;
         int tile = T <= 64 ? 4 : 16384 / H;  // f32 tile in LDS: at most 64 KiB

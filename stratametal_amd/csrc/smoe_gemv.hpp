@@ -141,6 +141,33 @@ __device__ __forceinline__ void wave_sum_xor_fast_n(float (&v)[N]) {
     for (int i = 0; i < N; ++i) v[i] = v[i] + t[i];
 }
 
+// One exchange step of the scattering butterfly: N values per lane become N / 2, each lane keeping the half its
+// lane bit D names, summed with lane ^ D's (the butterfly's addition: commutative, so the same bits in either lane).
+template <int D, int N>
+__device__ __forceinline__ void scatter_step(float* v, int lane) {
+    if constexpr (N == 1) {
+        v[0] = v[0] + __uint_as_float(xor_lane<D>(__float_as_uint(v[0])));
+    } else {
+        const bool up = (lane & D) != 0;
+#pragma unroll
+        for (int j = 0; j < N / 2; ++j) {
+            if constexpr (D >= 16) {  // the swap leaves each value's two halves in the lanes that add them
+                const int a = __float_as_int(v[j]), b = __float_as_int(v[j + N / 2]);
+                if constexpr (D == 16) {
+                    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+                    v[j] = __int_as_float(r[0]) + __int_as_float(r[1]);
+                } else {
+                    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+                    v[j] = __int_as_float(r[0]) + __int_as_float(r[1]);
+                }
+            } else {
+                const float keep = up ? v[j + N / 2] : v[j], send = up ? v[j] : v[j + N / 2];
+                v[j] = keep + __uint_as_float(xor_lane<D>(__float_as_uint(send)));
+            }
+        }
+    }
+}
+
 // Wave maxima for order-free reductions: row rotations by DPP (8, 4, 2, 1), then the four row results read
 // into scalars.  The result is uniform.
 __device__ __forceinline__ uint32_t wave_max_u32_fast(uint32_t v) {

@@ -354,27 +354,6 @@ __global__ __launch_bounds__(256) void k_mmvq_native(const uint8_t* __restrict__
     }
 }
 
-// One exchange step of the scattering butterfly below: N values per lane become N / 2, each lane keeping the half its
-// lane bit D names, summed with lane ^ D's (the butterfly's addition: commutative, so the same bits in either lane).
-template <int D, int N>
-__device__ __forceinline__ void scatter_step(float* v, int lane) {
-    if constexpr (N == 1) {
-        v[0] = v[0] + __uint_as_float(xor_lane<D>(__float_as_uint(v[0])));
-    } else {
-        const bool up = (lane & D) != 0;
-#pragma unroll
-        for (int j = 0; j < N / 2; ++j) {
-            if constexpr (D == 16) {  // rows of 16 lanes: the swap leaves each output's two halves in the lanes that add them
-                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(v[j]), __float_as_int(v[j + N / 2]), false, false);
-                v[j] = __int_as_float(r[0]) + __int_as_float(r[1]);
-            } else {
-                const float keep = up ? v[j + N / 2] : v[j], send = up ? v[j] : v[j + N / 2];
-                v[j] = keep + __uint_as_float(xor_lane<D>(__float_as_uint(send)));
-            }
-        }
-    }
-}
-
 // The same product for C columns at a time: a half wave owns kRw rows; x of the column tile in LDS, kXlChunk values of
 // K at a time (a multiple of 32 partials of every type, so the order of a lane's partials is k_mmvq_native's); a partial
 // is decoded once and taken against the C columns.  The butterflies of the kRw * C sums run as one scattering butterfly
