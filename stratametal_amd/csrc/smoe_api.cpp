@@ -371,14 +371,16 @@ bool recall_flags(const void* ws, FlagWords& f) {
 }
 
 // The native shared expert (its projections in their own types): q8_1 of x, gate and up, SwiGLU + q8_1, down
-// times sigmoid(sg[t]) into out[t] (T rows of n_embd), in the workspace's native-chain slots.
+// times sigmoid(sg[t]) into out[t] (T rows of n_embd), in the workspace's native-chain slots.  `stages`: every stage is
+// wanted in memory (a trace).  `add_to`: the rows are added to it (a combine that left them out: its own last addition),
+// and out need not hold them.
 smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float* x, int T, uint8_t* ws,
-                          const Layout& L, float* out, const float* sg, hipStream_t st) {
+                          const Layout& L, float* out, const float* sg, hipStream_t st, bool stages = false,
+                          float* add_to = nullptr) {
     const int H = g.n_embd, Fn = g.n_ff_shared;
     uint8_t* nxq = ws + L.nxq;
     float* ngu = reinterpret_cast<float*>(ws + L.ngu);
     uint8_t* nhq = ws + L.nhq;
-    SMOE_TRY(smoe::launch_prep(x, (int64_t)T * H, nxq, nullptr, st), "shared q8_1");
     auto gemv = [&](int type, const void* wt, const uint8_t* xq, int n_in, int n_out, float* y,
                     const float* gate) -> hipError_t {
         const uint8_t* wb = static_cast<const uint8_t*>(wt);
@@ -388,16 +390,27 @@ smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float
         if (e == hipSuccess && gate) e = smoe::launch_sigmoid_rows(y, T, n_out, gate, st);
         return e;
     };
-    if (smoe::native_type(sh_gate_t(g)) && sh_gate_t(g) == sh_up_t(g)) {  // gate and up in one launch
-        SMOE_TRY(smoe::launch_mmvq_native(sh_gate_t(g), static_cast<const uint8_t*>(w->gate_sh), nxq, H, Fn, T, ngu, Fn,
-                                          nullptr, st, static_cast<const uint8_t*>(w->up_sh), ngu + (size_t)T * Fn),
+    const int tg = sh_gate_t(g), td = sh_down_t(g);
+    const uint8_t* gw = static_cast<const uint8_t*>(w->gate_sh);
+    const uint8_t* uw = static_cast<const uint8_t*>(w->up_sh);
+    const bool pair = tg == sh_up_t(g) && smoe::native_type(tg);  // gate and up in one launch
+    if (pair && !stages && smoe::native_few_ok(tg, td, T, H, Fn)) {
+        SMOE_TRY(smoe::launch_native_few(tg, td, x, gw, uw, static_cast<const uint8_t*>(w->down_sh), T, H, Fn, ngu, sg,
+                                         add_to ? 1 : 0, add_to ? add_to : out, st),
+                 "shared expert");
+        return SMOE_OK;
+    }
+    SMOE_TRY(smoe::launch_prep(x, (int64_t)T * H, nxq, nullptr, st), "shared q8_1");
+    if (pair) {
+        SMOE_TRY(smoe::launch_mmvq_native(tg, gw, nxq, H, Fn, T, ngu, Fn, nullptr, st, uw, ngu + (size_t)T * Fn),
                  "shared gate/up");
     } else {
-        SMOE_TRY(gemv(sh_gate_t(g), w->gate_sh, nxq, H, Fn, ngu, nullptr), "shared gate");
-        SMOE_TRY(gemv(sh_up_t(g), w->up_sh, nxq, H, Fn, ngu + (size_t)T * Fn, nullptr), "shared up");
+        SMOE_TRY(gemv(tg, gw, nxq, H, Fn, ngu, nullptr), "shared gate");
+        SMOE_TRY(gemv(sh_up_t(g), uw, nxq, H, Fn, ngu + (size_t)T * Fn, nullptr), "shared up");
     }
     SMOE_TRY(smoe::launch_swiglu_q8(ngu, ngu + (size_t)T * Fn, (int64_t)T * Fn, nhq, st), "shared swiglu");
-    SMOE_TRY(gemv(sh_down_t(g), w->down_sh, nhq, Fn, H, out, sg), "shared down");
+    SMOE_TRY(gemv(td, w->down_sh, nhq, Fn, H, out, sg), "shared down");
+    if (add_to) SMOE_TRY(smoe::launch_add_rows(add_to, out, T, H, st), "shared add");
     return SMOE_OK;
 }
 
@@ -569,13 +582,14 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
             SMOE_TRY(smoe::launch_q2_down(de, ds, himg, L.h_blocks, sg, items, H, F, Fs, n_items, Y, st), "down");
     }
     SMOE_MARK();
-    if (nat) SMOE_TRY_S(native_shared(*g, w, x_io, T, ws, L, Y + (size_t)P * H, sg, st));
+    // a native shared expert's rows into Y for the combine, or added to y after the fused combine, which left them out
+    if (nat)
+        SMOE_TRY_S(native_shared(*g, w, x_io, T, ws, L, Y + (size_t)P * H, sg, st, stages,
+                                 small_down && add_shared ? y : nullptr));
     if (!small_down)
         SMOE_TRY(smoe::launch_combine(Y, slot, wts, K, H, P, T, (has_sh && add_shared) ? 1 : 0, y, st,
                                       y_stream ? 1 : 0),
                  "combine");
-    else if (nat && add_shared)  // the fused combine left the shared rows out: the same last addition, after it
-        SMOE_TRY(smoe::launch_add_rows(y, Y + (size_t)P * H, T, H, st), "shared add");
     SMOE_MARK();
 #undef SMOE_MARK
     FlagWords flags;
@@ -667,8 +681,8 @@ hipError_t hc_read(const smoe_hc& h, int n_embd, const float* R, int T, float* m
         return smoe::launch_hc_read_mm(R, h.norm, h.down, h.up, h.inject, T, n_embd, h.hc, h.hc_lr, h.eps, rs,
                                        reinterpret_cast<uint16_t*>(ws + L.act), reinterpret_cast<float*>(ws + L.part),
                                        reinterpret_cast<uint16_t*>(ws + L.lq), mixed, inject, st);
-    return smoe::launch_hc_read(const_cast<float*>(R), h.norm, h.down, h.up, h.inject, T, n_embd, h.hc, h.hc_lr, h.eps,
-                                reinterpret_cast<float*>(ws + L.proj), rs, mixed, inject, nullptr, nullptr, nullptr, st);
+    return smoe::launch_hc_read(R, h.norm, h.down, h.up, h.inject, T, n_embd, h.hc, h.hc_lr, h.eps,
+                                reinterpret_cast<float*>(ws + L.proj), rs, mixed, inject, st);
 }
 
 smoe_status check_hc(const smoe_hc* h, int32_t n_embd) {

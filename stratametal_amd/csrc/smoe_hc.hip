@@ -55,15 +55,14 @@ __device__ __forceinline__ void stream_scales(const float (&v)[HC][NM], int hc, 
 // k_hc_proj: grid (ceil((hc_lr + hc) / 4), T), 256 threads; block (b, t) takes rows 4b .. 4b + 3 of [down; inj] for
 // token t, one row per wave (lane l adds the 8-element chunks l, l + 64, ... in element order, then the xor butterfly
 // 32..1, as the router).  Every block forms the token's scales and stages act = bf16((R * rs) * w_norm) in LDS; block
-// (0, t) also writes rs[t][c] for k_hc_mix.  With `rprev` the layer's streams are first formed from the layer before,
-// R = rprev + y_prev * 2 sigmoid(inj_prev / hc) (the stacked call's write, fused), and block (0, t) stores them to R.
+// (0, t) also writes rs[t][c] for k_hc_mix.  Bound by latency at one token (81 work-groups): every load it needs (its
+// streams, norm and weight row) is issued up front, unconditionally (indices clamped into the row), so that one memory
+// round trip covers them all (with the loads under their bounds' branches 13.1 us, of which the bytes take 1.2).
 template <int HC, int NM, int MAXC>
-__global__ __launch_bounds__(256) void k_hc_proj(float* __restrict__ R, const float* __restrict__ norm,
+__global__ __launch_bounds__(256) void k_hc_proj(const float* __restrict__ R, const float* __restrict__ norm,
                                                   const uint16_t* __restrict__ down, const uint16_t* __restrict__ inj,
                                                   int n, int hc, int hc_lr, float eps, float* __restrict__ proj,
-                                                  float* __restrict__ inject, float* __restrict__ rs_out,
-                                                  const float* __restrict__ rprev, const float* __restrict__ yprev,
-                                                  const float* __restrict__ injprev) {
+                                                  float* __restrict__ inject, float* __restrict__ rs_out) {
     extern __shared__ __align__(16) uint16_t act_s[];  // hc * n bf16
     __shared__ float wsum[HC][4];
     __shared__ float rs_s[HC];
@@ -73,39 +72,20 @@ __global__ __launch_bounds__(256) void k_hc_proj(float* __restrict__ R, const fl
     const int row = min((int)blockIdx.x * 4 + (tid >> 6), rows - 1);  // clamped: every load in bounds
     const uint16_t* wr = row < hc_lr ? down + (size_t)row * hd : inj + (size_t)(row - hc_lr) * hd;
     const int chunks = hd >> 3;
+    const float* Rt = R + (size_t)t * hd;
+    float v[HC][NM], nv[HC][NM];
     uint4 wv[MAXC];
 #pragma unroll
-    for (int j = 0; j < MAXC; ++j) {  // the wave's weight row first: in flight while the scales are formed
-        const int c = lane + 64 * j;
-        wv[j] = c < chunks ? *reinterpret_cast<const uint4*>(wr + 8 * c) : make_uint4(0, 0, 0, 0);
-    }
-    float* Rt = R + (size_t)t * hd;
-    float v[HC][NM];
+    for (int c = 0; c < HC; ++c)
 #pragma unroll
-    for (int c = 0; c < HC; ++c) {
+        for (int m = 0; m < NM; ++m) v[c][m] = Rt[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            const int d = tid + 256 * m;
-            float x = 0.0f;
-            if (c < hc && d < n) {
-                const size_t i = (size_t)c * n + d;
-                if (rprev) {
-                    const float s = sigmoid(injprev[(size_t)t * hc + c] / (float)hc);
-                    x = rprev[(size_t)t * hd + i] + yprev[(size_t)t * n + d] * (2.0f * s);
-                } else {
-                    x = Rt[i];
-                }
-            }
-            v[c][m] = x;
-        }
-    }
-    if (rprev && blockIdx.x == 0) {
+    for (int c = 0; c < HC; ++c)
 #pragma unroll
-        for (int c = 0; c < HC; ++c)
+        for (int m = 0; m < NM; ++m) nv[c][m] = norm[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
 #pragma unroll
-            for (int m = 0; m < NM; ++m)
-                if (c < hc && tid + 256 * m < n) Rt[(size_t)c * n + tid + 256 * m] = v[c][m];
-    }
+    for (int j = 0; j < MAXC; ++j) wv[j] = *reinterpret_cast<const uint4*>(wr + 8 * min(lane + 64 * j, chunks - 1));
+    __builtin_amdgcn_sched_barrier(0);
     stream_scales<HC, NM>(v, hc, n, eps, wsum, rs_s);
     if (blockIdx.x == 0 && tid < hc) rs_out[(size_t)t * hc + tid] = rs_s[tid];
 #pragma unroll
@@ -113,10 +93,7 @@ __global__ __launch_bounds__(256) void k_hc_proj(float* __restrict__ R, const fl
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             const int d = tid + 256 * m;
-            if (c < hc && d < n) {
-                const size_t i = (size_t)c * n + d;
-                act_s[i] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * norm[i]);
-            }
+            if (c < hc && d < n) act_s[c * n + d] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * nv[c][m]);
         }
     }
     __syncthreads();
@@ -166,8 +143,7 @@ __global__ __launch_bounds__(256) void k_hc_mix(const float* __restrict__ R, con
         const uint16_t* wr = up + ((size_t)c * n + d0 + g) * hc_lr;
 #pragma unroll
         for (int j = 0; j < LQC; ++j) {
-            const int ch = l + 8 * j;
-            wv[j] = ch < lchunks ? *reinterpret_cast<const uint4*>(wr + 8 * ch) : make_uint4(0, 0, 0, 0);
+            wv[j] = *reinterpret_cast<const uint4*>(wr + 8 * min(l + 8 * j, lchunks - 1));  // clamped: no branch
         }
     }
     for (int i = tid; i < hc_lr; i += 256) {
@@ -181,8 +157,7 @@ __global__ __launch_bounds__(256) void k_hc_mix(const float* __restrict__ R, con
             const uint16_t* wr = up + i * hc_lr;
 #pragma unroll
             for (int j = 0; j < LQC; ++j) {
-                const int ch = l + 8 * j;
-                wv[j] = ch < lchunks ? *reinterpret_cast<const uint4*>(wr + 8 * ch) : make_uint4(0, 0, 0, 0);
+                wv[j] = *reinterpret_cast<const uint4*>(wr + 8 * min(l + 8 * j, lchunks - 1));
             }
         }
         float acc = 0.0f;
@@ -229,6 +204,23 @@ __global__ __launch_bounds__(256) void k_hc_write(const float* R, const float* _
     out[i] = R[i] + y[t * n + d] * (2.0f * s);
 }
 
+// The same with R, y and out as 16-byte vectors (n % 4 == 0): block (p, t) takes 256 four-value pieces of y of token t
+// through every stream, so y is read once (few tokens: a block per stream).  hc 4, n 2048, a value per thread and this: 1000
+// tokens (73 MB) 20.9 and 11.5 us, 4096 tokens 99 and 48.
+__global__ __launch_bounds__(256) void k_hc_write4(const float* R, const float* __restrict__ y,
+                                                    const float* __restrict__ inject, int n4, int hc, int parts,
+                                                    float* out) {
+    const int t = blockIdx.x / parts, d = (blockIdx.x % parts) * 256 + threadIdx.x;
+    if (d >= n4) return;
+    const float4 yv = reinterpret_cast<const float4*>(y)[(size_t)t * n4 + d];
+    for (int c = blockIdx.y; c < hc; c += gridDim.y) {
+        const float s = sigmoid(inject[(size_t)t * hc + c] / (float)hc), g = 2.0f * s;
+        const size_t i = ((size_t)t * hc + c) * n4 + d;
+        const float4 r = reinterpret_cast<const float4*>(R)[i];
+        reinterpret_cast<float4*>(out)[i] = make_float4(r.x + yv.x * g, r.y + yv.y * g, r.z + yv.z * g, r.w + yv.w * g);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ many tokens
 // The read as two bf16 matrix products: every bf16 product is exact in f32 and the sums are the matrix core's f32
 // accumulation, in the hardware's order and over the K slices below, so proj, inject and the gates are the exact dots
@@ -250,14 +242,16 @@ __global__ __launch_bounds__(256) void k_hc_act(const float* __restrict__ R, con
     const int t = blockIdx.x, tid = threadIdx.x;
     const int hd = hc * n;
     const float* Rt = R + (size_t)t * hd;
-    float v[HC][NM];
+    float v[HC][NM], nv[HC][NM];
 #pragma unroll
     for (int c = 0; c < HC; ++c)
 #pragma unroll
-        for (int m = 0; m < NM; ++m) {
-            const int d = tid + 256 * m;
-            v[c][m] = (c < hc && d < n) ? Rt[(size_t)c * n + d] : 0.0f;
-        }
+        for (int m = 0; m < NM; ++m) v[c][m] = Rt[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
+#pragma unroll
+    for (int c = 0; c < HC; ++c)
+#pragma unroll
+        for (int m = 0; m < NM; ++m) nv[c][m] = norm[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
+    __builtin_amdgcn_sched_barrier(0);
     stream_scales<HC, NM>(v, hc, n, eps, wsum, rs_s);
     if (tid < hc) rs_out[(size_t)t * hc + tid] = rs_s[tid];
 #pragma unroll
@@ -265,10 +259,7 @@ __global__ __launch_bounds__(256) void k_hc_act(const float* __restrict__ R, con
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             const int d = tid + 256 * m;
-            if (c < hc && d < n) {
-                const size_t i = (size_t)c * n + d;
-                act_s[i] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * norm[i]);
-            }
+            if (c < hc && d < n) act_s[c * n + d] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * nv[c][m]);
         }
     __syncthreads();
     u32x4* dst = reinterpret_cast<u32x4*>(act + (size_t)t * hd);
@@ -456,30 +447,39 @@ __global__ __launch_bounds__(256) void k_hc_mix_mm(const float* __restrict__ R, 
             }
         }
     };
+    // lane (q, i) ends with the gates of d .. d + 3 of token i of each tile; R of a token tile is loaded a tile ahead (the
+    // first before the products)
+    const int d = d0 + 4 * q;
+    f32x4 xr[2][HC], nv[HC];
+    auto load_r = [&](f32x4(&x)[HC], int b) {
+        const float* p = R + (size_t)min(t0 + 16 * b + i, T - 1) * hd + d;
+#pragma unroll
+        for (int c = 0; c < HC; ++c) x[c] = *reinterpret_cast<const f32x4*>(p + (size_t)min(c, hc - 1) * n);
+    };
+#pragma unroll
+    for (int c = 0; c < HC; ++c) nv[c] = *reinterpret_cast<const f32x4*>(norm + (size_t)min(c, hc - 1) * n + d);
+    load_r(xr[0], 0);
     int k0 = 0;
     for (; k0 + 64 < kp; k0 += 128) {
         chunk(k0, Zero{});
         chunk(k0 + 64, One{});
     }
     if (k0 < kp) chunk(k0, Zero{});
-    const int d = d0 + 4 * q;  // lane (q, i): the gates of d .. d + 3 of token i of each tile
 #pragma unroll
     for (int b = 0; b < NT; ++b) {
+        if (b + 1 < NT) load_r(xr[(b + 1) & 1], b + 1);
         const int t = t0 + 16 * b + i;
-        if (t >= T) continue;
         f32x4 m = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int c = 0; c < HC; ++c) {
             if (c >= hc) break;
-            const f32x4 x = *reinterpret_cast<const f32x4*>(R + (size_t)t * hd + (size_t)c * n + d);
-            const f32x4 nv = *reinterpret_cast<const f32x4*>(norm + (size_t)c * n + d);
-            const float sc = rs[(size_t)t * hc + c];
+            const float sc = rs[(size_t)min(t, T - 1) * hc + c];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) m[r] = m[r] + ((x[r] * sc) * nv[r]) * sigmoid(acc[c][b][r]);
+            for (int r = 0; r < 4; ++r) m[r] = m[r] + ((xr[b & 1][c][r] * sc) * nv[c][r]) * sigmoid(acc[c][b][r]);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) m[r] = m[r] / (float)hc;
-        *reinterpret_cast<f32x4*>(mixed + (size_t)t * n + d) = m;
+        if (t < T) *reinterpret_cast<f32x4*>(mixed + (size_t)t * n + d) = m;
     }
 }
 
@@ -539,7 +539,8 @@ hipError_t launch_hc_read_mm(const float* R, const float* norm, const uint16_t* 
     hipLaunchKernelGGL(k_hc_proj_mm, dim3((unsigned)(splits * n_tb * n_rb)), dim3(256), 0, s, act, down, inj, hd, hc_lr,
                        rows, ld, T, splits, per, n_rb, part);
     hipLaunchKernelGGL(k_hc_lq, dim3((unsigned)T), dim3(256), 0, s, part, T, splits, ld, hc, hc_lr, kp, lq, inject);
-    const int nt = T > 32 && hc <= 4 && kp <= 448 ? 4 : 2;
+    // 64-token tiles where they fill the chip (T 64, n 2048: 35.2 against 30.1 us the whole read; T 1000: 64.9 against 73.1)
+    const int nt = (int64_t)((T + 63) / 64) * (n / 64) >= 256 && hc <= 4 && kp <= 448 ? 4 : 2;
     const unsigned grid = (unsigned)((T + 16 * nt - 1) / (16 * nt)) * (unsigned)(n / 64);
     const size_t tile = (size_t)16 * nt * (kp * 2 + 16);
 #define SMOE_HCM(HCv, NTv)                                                                                         \
@@ -564,9 +565,9 @@ bool hc_shape_ok(int n, int hc, int hc_lr) {
     return (int64_t)hc * n <= 16384;  // the activations in LDS: 32 KiB of bf16
 }
 
-hipError_t launch_hc_read(float* R, const float* norm, const uint16_t* down, const uint16_t* up, const uint16_t* inj,
+hipError_t launch_hc_read(const float* R, const float* norm, const uint16_t* down, const uint16_t* up, const uint16_t* inj,
                           int n_tok, int n, int hc, int hc_lr, float eps, float* proj, float* rs, float* mixed,
-                          float* inject, const float* rprev, const float* yprev, const float* injprev, hipStream_t s) {
+                          float* inject, hipStream_t s) {
     if (!hc_shape_ok(n, hc, hc_lr) || n_tok <= 0) return hipErrorInvalidValue;
     const int hd = hc * n;
     const int maxc = (hd / 8 + 63) / 64;
@@ -575,7 +576,7 @@ hipError_t launch_hc_read(float* R, const float* norm, const uint16_t* down, con
     const size_t lds = (size_t)hd * 2;
 #define SMOE_HCP(HCv, NMv, C)                                                                                       \
     hipLaunchKernelGGL((k_hc_proj<HCv, NMv, C>), g1, dim3(256), lds, s, R, norm, down, inj, n, hc, hc_lr, eps, proj, \
-                       inject, rs, rprev, yprev, injprev)
+                       inject, rs)
 #define SMOE_HCP_C(HCv, NMv)             \
     if (maxc <= 8) SMOE_HCP(HCv, NMv, 8);  \
     else if (maxc <= 16) SMOE_HCP(HCv, NMv, 16); \
@@ -604,6 +605,13 @@ hipError_t launch_hc_write(const float* R, const float* y, const float* inject, 
                            hipStream_t s) {
     const int64_t total = (int64_t)n_tok * hc * n;
     if (total <= 0) return hipErrorInvalidValue;
+    const int parts = (n / 4 + 255) / 256;
+    const uintptr_t al = reinterpret_cast<uintptr_t>(R) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out);
+    if (n % 4 == 0 && (al & 15) == 0 && (int64_t)n_tok * parts <= INT32_MAX) {
+        hipLaunchKernelGGL(k_hc_write4, dim3((unsigned)((int64_t)n_tok * parts), n_tok < 64 ? (unsigned)hc : 1u), dim3(256), 0, s, R, y, inject, n / 4, hc,
+                           parts, out);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_hc_write, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, R, y, inject, n, hc, total,
                        out);
     return hipGetLastError();

@@ -105,6 +105,11 @@ int64_t native_row_bytes(int type, int64_t n);  // -1: not native, or n not a wh
 // (with w2, a second matrix of the same type and shape into y2 by the same launch)
 hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y,
                               int ldy, const float* sg, hipStream_t s, const uint8_t* w2 = nullptr, float* y2 = nullptr);
+// a native shared expert of a few tokens in two launches (h: T * F floats of scratch; y rows written, or with add added to)
+bool native_few_ok(int gu_type, int d_type, int T, int H, int F);
+hipError_t launch_native_few(int gu_type, int d_type, const float* x, const uint8_t* gate, const uint8_t* up,
+                             const uint8_t* down, int T, int H, int F, float* h, const float* sg, int add, float* y,
+                             hipStream_t s);
 hipError_t launch_sigmoid_rows(float* y, int T, int n, const float* sg, hipStream_t s);  // y[t][.] *= sigmoid(sg[t])
 hipError_t launch_add_rows(float* y, const float* r, int T, int n, hipStream_t s);       // y[t][.] += r[t][.]
 hipError_t launch_q2_mmvq(const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y, hipStream_t s);
@@ -143,12 +148,11 @@ hipError_t launch_mm_down(const uint8_t* down_exps, const uint8_t* down_sh, cons
                           int h_rec, const float* sg, const int4* items, int H, int F, int Fs, int max_items, float* Y,
                           int nt, hipStream_t s);  // nt: streaming stores of Y
 
-// the hyper-connection ends (smoe_hc.hip): gr_read (two launches; proj [T][hc_lr] and rs [T][hc] are scratch; with
-// rprev, R = rprev + yprev * 2 sigmoid(injprev / hc) is formed and stored first) and gr_write
+// the hyper-connection ends (smoe_hc.hip): gr_read (two launches; proj [T][hc_lr] and rs [T][hc] are scratch) and gr_write
 bool hc_shape_ok(int n, int hc, int hc_lr);
-hipError_t launch_hc_read(float* R, const float* norm, const uint16_t* down, const uint16_t* up, const uint16_t* inj,
+hipError_t launch_hc_read(const float* R, const float* norm, const uint16_t* down, const uint16_t* up, const uint16_t* inj,
                           int n_tok, int n, int hc, int hc_lr, float eps, float* proj, float* rs, float* mixed,
-                          float* inject, const float* rprev, const float* yprev, const float* injprev, hipStream_t s);
+                          float* inject, hipStream_t s);
 // the read of a batch of tokens on the matrix cores, where hc_mm_shape says so: its scratch (hc_mm_bytes: act, the K
 // slices' sums, lq) and launches; R, norm and mixed 16-byte aligned
 bool hc_mm_shape(int64_t T, int n, int hc, int hc_lr);

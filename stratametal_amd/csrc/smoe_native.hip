@@ -87,7 +87,7 @@ struct XLds {
 // One partial of a row (part iqs of a block), decoded once: signed bytes whose integer dots are the reference's (an
 // offset it subtracts after the dot is subtracted from each byte: the same integer).  dot(x): the partial against a
 // column's activations of the block (x its first 32-value block); the float steps are the reference's, one rounding
-// each (no contraction).
+// each (no contraction).  A dot times its scale is a 24-bit multiply: every dot is below 2^20, every scale below 2^8.
 template <int TYPE>
 struct NativePart;
 
@@ -185,7 +185,7 @@ struct NativePart<23> {  // IQ4_XS: 32-value group iqs / 4, its 6-bit scale - 32
             s = dot4(lo[j], x.word(j), s);
             s = dot4(hi[j], x.word(j + 4), s);
         }
-        return (d * x.scale()) * (float)(s * ls);
+        return (d * x.scale()) * (float)__mul24(s, ls);
     }
 };
 
@@ -229,8 +229,8 @@ struct NativePartK {  // Q4_K, Q5_K: 8 values of two 32-value groups
             const int32_t u0 = x.word(qoff), u1 = x.word(qoff + 4);
             const int32_t dq = dot4(p[i][1], u1, dot4(p[i][0], u0, 0));
             const int32_t da = dot4(0x01010101, u1, dot4(0x01010101, u0, 0));
-            sum_d = sum_d + d8 * (float)(dq * sc[i]);
-            sum_m = sum_m + d8 * (float)(da * mn[i]);
+            sum_d = sum_d + d8 * (float)__mul24(dq, sc[i]);
+            sum_m = sum_m + d8 * (float)__mul24(da, mn[i]);
         }
         return d * sum_d - dmin * sum_m;
     }
@@ -268,7 +268,7 @@ struct NativePart<11> {  // Q3_K: 2 low bits, - 4 where the high bit is clear; s
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const X xi = x.at(i);
-            sumf = sumf + xi.scale() * (float)(dot4(v[i], xi.word(iqs % 8), 0) * sc[i]);
+            sumf = sumf + xi.scale() * (float)__mul24(dot4(v[i], xi.word(iqs % 8), 0), sc[i]);
         }
         return d * sumf;
     }
@@ -299,11 +299,107 @@ struct NativePart<14> {  // Q6_K: (low nibble | 2 high bits << 4) - 32 times an 
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const X xi = x.at(2 * i);
-            sumf = sumf + xi.scale() * (float)(dot4(v[i], xi.word(iqs % 8), 0) * sc[i]);
+            sumf = sumf + xi.scale() * (float)__mul24(dot4(v[i], xi.word(iqs % 8), 0), sc[i]);
         }
         return d * sumf;
     }
 };
+
+// A row against one column by 32 lanes: lane l (k = l) adds partials l, l + 32, ... in order, then the butterfly 16
+// .. 1; every lane returns the sum.  (`acc`: the sum of the partials before k.)
+template <int TYPE, class X>
+__device__ __forceinline__ float native_row(const uint8_t* row, int npart, const X& col, float acc, int k) {
+    using NT = NativeType<TYPE>;
+    // four partials at a time: their loads are in flight together, their sums added in order (not the wider partials
+    // of Q4_K and Q5_K, 3.3 us against 3.9 for 512 rows of 2048)
+    for (; TYPE != 12 && TYPE != 13 && k + 96 < npart; k += 128) {
+        NativePart<TYPE> p[4];
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j].decode(row + (size_t)((k + 32 * j) / NT::ipb) * NT::bytes, NT::step * ((k + 32 * j) % NT::ipb));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            v[j] = p[j].dot(col.at((k + 32 * j) / NT::ipb * (NT::qk / 32)), NT::step * ((k + 32 * j) % NT::ipb));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = acc + v[j];
+    }
+    for (; k < npart; k += 32) {
+        NativePart<TYPE> p;
+        p.decode(row + (size_t)(k / NT::ipb) * NT::bytes, NT::step * (k % NT::ipb));
+        acc = acc + p.dot(col.at(k / NT::ipb * (NT::qk / 32)), NT::step * (k % NT::ipb));
+    }
+    acc = acc + xor_swap<16>(acc);
+    acc = acc + xor_swap<8>(acc);
+    acc = acc + xor_swap<4>(acc);
+    acc = acc + xor_swap<2>(acc);
+    acc = acc + xor_swap<1>(acc);
+    return acc;
+}
+
+// n values of x (n % 32 == 0) as q8_1 blocks in LDS, by the whole work-group (NTH threads): q8_1_value's int8 and scale,
+// without the block sum, which no partial reads.
+template <int NTH>
+__device__ __forceinline__ void quantise_lds(const float* __restrict__ x, int n, uint32_t* xl) {
+    uint8_t* xb = reinterpret_cast<uint8_t*>(xl);
+    const int l = threadIdx.x & 31;
+    for (int i0 = threadIdx.x; i0 < n; i0 += NTH * 4) {
+        float v[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) v[m] = x[min(i0 + NTH * m, n - 32 + l)];  // past the end: the last block again
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const float a = half_max(__builtin_fabsf(v[m]));
+            float d = a / 127.0f;
+            if (d > 65504.0f) d = 65504.0f;
+            float r = __builtin_roundf(v[m] / d);
+            r = r > 127.0f ? 127.0f : r;
+            r = r < -127.0f ? -127.0f : r;
+            const int q = (a != 0.0f && r == r) ? (int)r : 0;
+            const int i = i0 + NTH * m;
+            if (i < n) {
+                xb[(i >> 5) * (4 * kXlDw) + l] = (uint8_t)(int8_t)q;
+                if (l == 0) xl[(i >> 5) * kXlDw + 8] = __float_as_uint((float)(_Float16)d);
+            }
+        }
+    }
+}
+
+// A shared expert of native types for a few tokens, in two launches: h = silu(gate) * up of x in q8_1 (k_native_gu: grid
+// (ceil(ff / 8), T), a half wave per row of each plane), then down rows of h in q8_1 (k_native_down: grid (ceil(n / 8),
+// T)), each work-group quantising its token's row into LDS as the stage kernels form it.  Bound by launches and latency:
+// one token of Q3_K gate and up, IQ4_NL down, 512 wide, took 4.0 + 7.8 + 7.0 + 2.4 + 3.3 us in five.
+template <int TYPE>
+__global__ __launch_bounds__(512) void k_native_gu(const float* __restrict__ x, const uint8_t* __restrict__ gate,
+                                                   const uint8_t* __restrict__ up, int H, int F, float* __restrict__ h) {
+    using NT = NativeType<TYPE>;
+    extern __shared__ __align__(16) uint32_t xl[];  // [H / 32][kXlDw]
+    __shared__ float rowv[16];                      // eight gate rows, the same up rows
+    const int l = threadIdx.x & 31, hw = threadIdx.x >> 5, r = blockIdx.x * 8 + (hw & 7), t = blockIdx.y;
+    quantise_lds<512>(x + (size_t)t * H, H, xl);
+    __syncthreads();
+    const float v = native_row<TYPE>((hw < 8 ? gate : up) + (size_t)min(r, F - 1) * (H / NT::qk) * NT::bytes,
+                                     (H / NT::qk) * NT::ipb, XLds{xl}, 0.0f, l);
+    if (l == 0) rowv[hw] = v;
+    __syncthreads();
+    if (hw < 8 && l == 0 && r < F) h[(size_t)t * F + r] = silu_mul(rowv[hw], rowv[hw + 8]);
+}
+
+template <int TYPE>
+__global__ __launch_bounds__(256) void k_native_down(const float* __restrict__ h, const uint8_t* __restrict__ down, int F,
+                                                     int H, const float* __restrict__ sg, int add, float* __restrict__ y) {
+    using NT = NativeType<TYPE>;
+    extern __shared__ __align__(16) uint32_t xl[];  // [F / 32][kXlDw]
+    const int l = threadIdx.x & 31, r = blockIdx.x * 8 + (threadIdx.x >> 5), t = blockIdx.y;
+    quantise_lds<256>(h + (size_t)t * F, F, xl);
+    __syncthreads();
+    const float acc = native_row<TYPE>(down + (size_t)min(r, H - 1) * (F / NT::qk) * NT::bytes, (F / NT::qk) * NT::ipb,
+                                       XLds{xl}, 0.0f, l);
+    if (r < H && l == 0) {
+        const float v = acc * sigmoid(sg[t]);
+        float* dst = y + (size_t)t * H + r;
+        *dst = add ? *dst + v : v;
+    }
+}
 
 // y[c * ldy + r] = row r . column c (times sigmoid(sg[c]) when sg is given).  Grid (ceil(n_out / 8), column
 // groups, matrices: w into y, then w2 into y2); a 32-lane half wave per row; a work-group takes columns blockIdx.y,
@@ -324,32 +420,7 @@ __global__ __launch_bounds__(256) void k_mmvq_native(const uint8_t* __restrict__
     const uint8_t* row = w + (size_t)(r < n_out ? r : n_out - 1) * rb;  // a dead half wave reads the last row
     const int npart = (n_in / NT::qk) * NT::ipb;
     for (int c = blockIdx.y; c < n_col; c += gridDim.y) {
-        const XMem col{xq + (size_t)c * xb};
-        float acc = 0.0f;
-        int k = l;
-        // four partials at a time: their loads are in flight together, their sums added in order (not the wider partials
-        // of Q4_K and Q5_K, 3.3 us against 3.9 for 512 rows of 2048)
-        for (; TYPE != 12 && TYPE != 13 && k + 96 < npart; k += 128) {
-            NativePart<TYPE> p[4];
-            float v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) p[j].decode(row + (size_t)((k + 32 * j) / NT::ipb) * NT::bytes, NT::step * ((k + 32 * j) % NT::ipb));
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                v[j] = p[j].dot(col.at((k + 32 * j) / NT::ipb * (NT::qk / 32)), NT::step * ((k + 32 * j) % NT::ipb));
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc = acc + v[j];
-        }
-        for (; k < npart; k += 32) {
-            NativePart<TYPE> p;
-            p.decode(row + (size_t)(k / NT::ipb) * NT::bytes, NT::step * (k % NT::ipb));
-            acc = acc + p.dot(col.at(k / NT::ipb * (NT::qk / 32)), NT::step * (k % NT::ipb));
-        }
-        acc = acc + xor_swap<16>(acc);
-        acc = acc + xor_swap<8>(acc);
-        acc = acc + xor_swap<4>(acc);
-        acc = acc + xor_swap<2>(acc);
-        acc = acc + xor_swap<1>(acc);
+        const float acc = native_row<TYPE>(row, npart, XMem{xq + (size_t)c * xb}, 0.0f, l);
         if (r < n_out && l == 0) y[(size_t)c * ldy + r] = sg ? acc * sigmoid(sg[c]) : acc;
     }
 }
@@ -528,6 +599,42 @@ hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int
     }
 #undef SMOE_NAT
 #undef SMOE_NATC
+    return hipGetLastError();
+}
+
+// A native shared expert of up to kNativeFewTokens tokens whose gate and up have one type and whose down is native.
+// (Every work-group quantises its whole row, so more tokens are better served by the stage kernels' column tiles.)
+constexpr int kNativeFewTokens = 4;
+bool native_few_ok(int gu_type, int d_type, int T, int H, int F) {
+    return T <= kNativeFewTokens && native_row_bytes(gu_type, H) > 0 && native_row_bytes(d_type, F) > 0 && H <= 4096 &&
+           F <= 4096;
+}
+
+hipError_t launch_native_few(int gu_type, int d_type, const float* x, const uint8_t* gate, const uint8_t* up,
+                             const uint8_t* down, int T, int H, int F, float* h, const float* sg, int add, float* y,
+                             hipStream_t s) {
+    if (!native_few_ok(gu_type, d_type, T, H, F) || T < 1) return hipErrorInvalidValue;
+    const dim3 g1((unsigned)((F + 7) / 8), (unsigned)T), g2((unsigned)((H + 7) / 8), (unsigned)T);
+    const size_t l1 = (size_t)(H / 32) * kXlDw * 4, l2 = (size_t)(F / 32) * kXlDw * 4;
+#define SMOE_EACH_NATIVE(type, CALL) \
+    switch (type) {                  \
+        case 8: CALL(8); break;      \
+        case 2: CALL(2); break;      \
+        case 6: CALL(6); break;      \
+        case 20: CALL(20); break;    \
+        case 23: CALL(23); break;    \
+        case 11: CALL(11); break;    \
+        case 12: CALL(12); break;    \
+        case 13: CALL(13); break;    \
+        default: CALL(14); break;    \
+    }
+#define SMOE_GU(T_) hipLaunchKernelGGL(k_native_gu<T_>, g1, dim3(512), l1, s, x, gate, up, H, F, h)
+#define SMOE_DN(T_) hipLaunchKernelGGL(k_native_down<T_>, g2, dim3(256), l2, s, h, down, F, H, sg, add, y)
+    SMOE_EACH_NATIVE(gu_type, SMOE_GU)
+    SMOE_EACH_NATIVE(d_type, SMOE_DN)
+#undef SMOE_DN
+#undef SMOE_GU
+#undef SMOE_EACH_NATIVE
     return hipGetLastError();
 }
 
