@@ -155,11 +155,11 @@ def _need(t, name: str, dtype, shape=None, numel=None):
         raise SmoeError(-1, f"{name} is {t.dtype}, needs {dtype}")
     if not t.is_contiguous():
         raise SmoeError(-5, f"{name} is not contiguous")
-    if shape is not None and tuple(t.shape) != tuple(shape):
+    if shape is not None and t.shape != tuple(shape):
         raise SmoeError(-2, f"{name} has shape {tuple(t.shape)}, needs {tuple(shape)}")
     if numel is not None and t.numel() < numel:
         raise SmoeError(-2, f"{name} has {t.numel()} elements, needs {numel}")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise SmoeError(-1, f"{name} is on {t.device}, not a GPU")
     return t
 
@@ -168,6 +168,15 @@ def _stream(stream=None) -> int:
     import torch
     s = torch.cuda.current_stream() if stream is None else stream
     return s.cuda_stream
+
+
+def _parts(buf, *sizes):
+    """Consecutive views of `buf`, one per size."""
+    out, at = [], 0
+    for n in sizes:
+        out.append(buf[at:at + n])
+        at += n
+    return out
 
 
 # the other native GGUF types (smoe.h): type -> (values per block, bytes per block)
@@ -816,14 +825,12 @@ def expert_group(ids, k_per_tok: int, n_expert: int, table, stream=None) -> Dict
     _need(table, "table", torch.int64, numel=n_expert)
     n = ids.numel()
     G = max(1, min(n, n_expert))
-    dev = ids.device
-    out = dict(grp_ptr=torch.zeros(G, dtype=torch.int64, device=dev),
-               grp_expert=torch.full((G,), -1, dtype=torch.int32, device=dev),
-               grp_start=torch.zeros(G + 1, dtype=torch.int32, device=dev),
-               ent_dst=torch.full((max(n, 1),), -1, dtype=torch.int32, device=dev),
-               ent_tok=torch.full((max(n, 1),), -1, dtype=torch.int32, device=dev),
-               miss_dst=torch.full((max(n, 1),), -1, dtype=torch.int32, device=dev),
-               counts=torch.zeros(4, dtype=torch.int32, device=dev))
+    dev, m = ids.device, max(n, 1)
+    # two fills, not one per list: the lists that start as zeros and those that start as -1
+    ptr, start, counts = _parts(torch.zeros(2 * G + G + 1 + 4, dtype=torch.int32, device=dev), 2 * G, G + 1, 4)
+    expert, dst, tok, miss = _parts(torch.full((G + 3 * m,), -1, dtype=torch.int32, device=dev), G, m, m, m)
+    out = dict(grp_ptr=ptr.view(torch.int64), grp_expert=expert, grp_start=start, ent_dst=dst, ent_tok=tok,
+               miss_dst=miss, counts=counts)
     _check(lib().smoe_expert_group(ids.data_ptr(), n, k_per_tok, n_expert, table.data_ptr(),
                                    out["grp_ptr"].data_ptr(), out["grp_start"].data_ptr(),
                                    out["grp_expert"].data_ptr(), out["ent_dst"].data_ptr(), out["ent_tok"].data_ptr(),
@@ -850,9 +857,10 @@ def expert_grouped(g: Geom, groups: Dict, x_q8, n_tokens: int, out, cap_groups: 
         _need(groups[key], key, dtype, numel=n)
     _need(x_q8, "x_q8", torch.uint8, numel=n_tokens * (g.n_embd // 32) * 36)
     _need(out, "out", torch.float32)
-    nb = int(lib().smoe_expert_grouped_workspace_bytes(C.byref(g.c()), n_tokens, cg, ce))
+    gc = C.byref(g.c())
+    nb = int(lib().smoe_expert_grouped_workspace_bytes(gc, n_tokens, cg, ce))
     ws = torch.empty(max(nb, 1), dtype=torch.uint8, device=out.device)
-    _check(lib().smoe_expert_grouped(C.byref(g.c()), groups["grp_ptr"].data_ptr(), groups["grp_start"].data_ptr(),
+    _check(lib().smoe_expert_grouped(gc, groups["grp_ptr"].data_ptr(), groups["grp_start"].data_ptr(),
                                      groups["ent_dst"].data_ptr(), groups["ent_tok"].data_ptr(),
                                      groups["counts"].data_ptr(), cg, ce, x_q8.data_ptr(), n_tokens, out.data_ptr(),
                                      out.shape[0], ws.data_ptr(), nb, _stream(stream)))
@@ -883,12 +891,13 @@ class VerifyWindow:
         if T > self.max_tokens:
             raise SmoeError(-1, f"{T} tokens exceed the window's {self.max_tokens}")
         _need(table, "table", torch.int64, numel=self.g.n_expert)
-        dev = x.device
-        r = dict(rows=torch.zeros((T * K + T, H), dtype=torch.float32, device=dev),
+        dev, n = x.device, (T * K + T) * H
+        rows, counts = _parts(torch.zeros(n + 4, dtype=torch.float32, device=dev), n, 4)  # one fill of zeros
+        r = dict(rows=rows.view(T * K + T, H),
                  ids=torch.empty((T, K), dtype=torch.int32, device=dev),
                  weights=torch.empty((T, K), dtype=torch.float32, device=dev),
                  miss_dst=torch.full((max(T * K, 1),), -1, dtype=torch.int32, device=dev),
-                 counts=torch.zeros(4, dtype=torch.int32, device=dev))
+                 counts=counts.view(torch.int32))
         _check(lib().smoe_verify_begin(C.byref(self._gc), C.byref(self._wc), table.data_ptr(), x.data_ptr(), T,
                                        r["rows"].data_ptr(), r["ids"].data_ptr(), r["weights"].data_ptr(),
                                        r["miss_dst"].data_ptr(), r["counts"].data_ptr(), self.ws.data_ptr(),

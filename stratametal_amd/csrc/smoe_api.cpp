@@ -1153,10 +1153,10 @@ GroupedLayout grouped_layout(const smoe_geom& g, int64_t T, int64_t cap_groups, 
 }
 
 // The verify window's workspace: the router's outputs, the group lists, the item table (groups, then the shared
-// chunks of a fused shared expert), the h images of every entry and shared token, the combine's slots, and the
-// native shared expert's chain (in `nat`, whose other offsets are unused).
+// chunks of a fused shared expert), the h images of every entry and shared token, and the native shared expert's
+// chain (in `nat`, whose other offsets are unused).
 struct VerifyLayout {
-    size_t ximg, logits, sg, grp_ptr, grp_start, ent_dst, ent_tok, items, himg, slot, total;
+    size_t ximg, logits, sg, grp_ptr, grp_start, ent_dst, ent_tok, items, himg, total;
     int cap_groups, n_items, h_blocks;
     Layout nat;
 };
@@ -1182,7 +1182,6 @@ VerifyLayout verify_layout(const smoe_geom& g, int64_t T) {
     L.ent_tok = take((size_t)P * 4);
     L.items = take((size_t)L.n_items * 32);
     L.himg = take(smoe::img_bytes((P + T) * L.h_blocks));
-    L.slot = take((size_t)P * 4);
     if (sh_native(g)) {
         const int64_t Fs = g.n_ff_shared;
         L.nat.nxq = take((size_t)T * (H / 32) * 36);
@@ -1231,7 +1230,7 @@ smoe_status smoe_expert_group(const int32_t* ids, int32_t n, int32_t k_per_tok, 
         return fail(SMOE_ENULL, "expert_group: NULL buffer");
     if (!aligned(expert_ptr, 8) || !aligned(grp_ptr, 8)) return fail(SMOE_EALIGN, "expert_group: pointer tables must be 8-byte aligned");
     SMOE_TRY(smoe::launch_expert_group(ids, n, k_per_tok, n_expert, expert_ptr, grp_ptr, grp_start, grp_expert, ent_dst,
-                                       ent_tok, miss_dst, counts, nullptr, 0, 0, n, 0, nullptr, stream_of(hip_stream)),
+                                       ent_tok, miss_dst, counts, nullptr, 0, 0, n, 0, stream_of(hip_stream)),
              "expert_group");
     return ok();
 }
@@ -1272,10 +1271,10 @@ smoe_status smoe_expert_grouped(const smoe_geom* g, const uint64_t* grp_ptr, con
     uint32_t* himg = reinterpret_cast<uint32_t*>(ws + L.himg);
     const int hb = F / 32;
     const hipStream_t st = stream_of(hip_stream);
-    SMOE_TRY(smoe::launch_q8_images(x_q8_1, (int64_t)n_tokens * (H / 32), iq2 ? 1 : 0, ximg, st), "grouped images");
-    SMOE_TRY(smoe::launch_group_items(grp_ptr, grp_start, ent_tok, ent_dst, counts, cap_groups, cap_entries, n_tokens,
-                                      n_out_rows, items, etok, edst, st),
-             "grouped items");
+    SMOE_TRY(smoe::launch_grouped_prep(x_q8_1, (int64_t)n_tokens * (H / 32), iq2 ? 1 : 0, ximg, grp_ptr, grp_start, ent_tok,
+                                       ent_dst, counts, cap_groups, cap_entries, n_tokens, n_out_rows, items, etok, edst,
+                                       st),
+             "grouped images and items");
     if (iq2) {
         SMOE_TRY(smoe::launch_iq2_gu(nullptr, nullptr, nullptr, nullptr, ximg, items, etok, 1, H, F, 0, 0, cap_groups,
                                      himg, hb, st, nullptr, grp_ptr),
@@ -1343,8 +1342,7 @@ smoe_status smoe_verify_begin(const smoe_geom* g, const smoe_weights* w, const u
              "verify router");
     SMOE_TRY(smoe::launch_topk(logits, E, T, E, K, ids, weights, st), "verify topk");
     SMOE_TRY(smoe::launch_expert_group(ids, P, K, E, expert_ptr, grp_ptr, grp_start, nullptr, ent_dst, ent_tok,
-                                       miss_dst, counts, items, L.cap_groups, L.n_items - L.cap_groups, P, T, nullptr,
-                                       st),
+                                       miss_dst, counts, items, L.cap_groups, L.n_items - L.cap_groups, P, T, st),
              "verify split");
     const uint8_t* gs = static_cast<const uint8_t*>(w->gate_sh);
     const uint8_t* us = static_cast<const uint8_t*>(w->up_sh);
@@ -1385,10 +1383,8 @@ smoe_status smoe_verify_end(const smoe_geom* g, int32_t n_tokens, const float* r
     const int T = n_tokens, H = g->n_embd, K = g->top_k, P = T * K;
     if (overlaps_n(y, (size_t)T * H * 4, rows, (size_t)(P + T) * H * 4))
         return fail(SMOE_EINVAL, "verify_end: y overlaps rows");
-    int32_t* slot = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + L.slot);
     const hipStream_t st = stream_of(hip_stream);
-    SMOE_TRY(smoe::launch_iota(slot, P, st), "verify slots");
-    SMOE_TRY(smoe::launch_combine(rows, slot, weights, K, H, P, T, (g->sh_type >= 0 && add_shared) ? 1 : 0, y, st),
+    SMOE_TRY(smoe::launch_combine(rows, nullptr, weights, K, H, P, T, (g->sh_type >= 0 && add_shared) ? 1 : 0, y, st),
              "verify combine");
     return ok();
 }

@@ -37,13 +37,12 @@ struct GroupLds {
 // i: an entry's rank among the earlier entries of its expert in the pass comes from the pass's ids in LDS, the
 // misses' positions from a scan.  With `items`, the work-item table of the expert kernels as well: slot g < cap_groups
 // is group g (e = g, so that the kernels read the blob at grp_ptr[g]), the rest empty, then the shared expert's
-// token chunks (rows P + t); and `slot_id` = i for the combine of the rows in entry order.
+// token chunks (rows P + t).
 __global__ __launch_bounds__(kGroupThreads) void k_expert_group(
     const int32_t* __restrict__ ids, int n, int kpt, int E, const uint64_t* __restrict__ eptr,
     uint64_t* __restrict__ grp_ptr, int32_t* __restrict__ grp_start, int32_t* __restrict__ grp_expert,
     int32_t* __restrict__ ent_dst, int32_t* __restrict__ ent_tok, int32_t* __restrict__ miss_dst,
-    int32_t* __restrict__ counts, int4* __restrict__ items, int cap_groups, int n_sh_items, int P, int T,
-    int32_t* __restrict__ slot_id) {
+    int32_t* __restrict__ counts, int4* __restrict__ items, int cap_groups, int n_sh_items, int P, int T) {
     __shared__ GroupLds s;
     const int tid = threadIdx.x;
     // every expert's blob flag and count (E <= 1024 = one thread each)
@@ -120,7 +119,6 @@ __global__ __launch_bounds__(kGroupThreads) void k_expert_group(
         items[2 * wi] = a;
         items[2 * wi + 1] = b;
     }
-    for (int i = tid; slot_id && i < n; i += kGroupThreads) slot_id[i] = i;
 }
 
 // The work-item table of caller-made group lists (counts[0] groups; group g's blob at grp_ptr[g], its entries
@@ -129,14 +127,12 @@ __global__ __launch_bounds__(kGroupThreads) void k_expert_group(
 // clipped to [0, cap_entries), a group without a blob is empty, and an entry whose token is not below n_tok or
 // whose row is not below n_rows gets token 0 and row -1 (computed, not written).  The checked tokens and rows go
 // to etok / edst, which the kernels read instead of the caller's.
-__global__ __launch_bounds__(256) void k_group_items(const uint64_t* __restrict__ grp_ptr,
-                                                      const int32_t* __restrict__ grp_start,
-                                                      const int32_t* __restrict__ ent_tok,
-                                                      const int32_t* __restrict__ ent_dst,
-                                                      const int32_t* __restrict__ counts, int cap_groups,
-                                                      int cap_entries, int n_tok, int n_rows, int4* __restrict__ items,
-                                                      int32_t* __restrict__ etok, int32_t* __restrict__ edst) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ void group_items(int i, const uint64_t* __restrict__ grp_ptr,
+                                            const int32_t* __restrict__ grp_start,
+                                            const int32_t* __restrict__ ent_tok, const int32_t* __restrict__ ent_dst,
+                                            const int32_t* __restrict__ counts, int cap_groups, int cap_entries,
+                                            int n_tok, int n_rows, int4* __restrict__ items,
+                                            int32_t* __restrict__ etok, int32_t* __restrict__ edst) {
     auto checked_tok = [&](int j) {
         const int t = ent_tok[j], d = ent_dst[j];
         return (t >= 0 && t < n_tok && d >= 0 && d < n_rows) ? t : 0;
@@ -168,10 +164,8 @@ __global__ __launch_bounds__(256) void k_group_items(const uint64_t* __restrict_
 // q8_1 blocks (36 bytes: fp16 d, fp16 s, 32 int8) -> activation images (kImgDw dwords: the 32 values split into
 // nibbles, or in natural byte order, then f32 of d and the integer sum of the values), one thread per block.  The
 // image equals the one the router kernel writes for the same activation row (both come from the same quantiser).
-__global__ __launch_bounds__(256) void k_q8_images(const uint8_t* __restrict__ xq, int64_t n_blocks, int natural,
-                                                    uint32_t* __restrict__ img) {
-    const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (b >= n_blocks) return;
+__device__ __forceinline__ void q8_image(int64_t b, const uint8_t* __restrict__ xq, int natural,
+                                         uint32_t* __restrict__ img) {
     const uint8_t* p = xq + b * 36;
     const uint32_t d16 = (uint32_t)p[0] | ((uint32_t)p[1] << 8);
     int q[32];
@@ -205,40 +199,47 @@ __global__ __launch_bounds__(256) void k_q8_images(const uint8_t* __restrict__ x
     o[2] = make_uint4(f2u(f16_to_f32(d16)), (uint32_t)sum, 0u, 0u);
 }
 
-// p[i] = i (the combine's slots of rows kept in entry order)
-__global__ __launch_bounds__(256) void k_iota(int32_t* __restrict__ p, int n) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = i;
+// What the grouped expert kernels read, in one launch: the images of the x blocks (the first img_blocks work-groups),
+// then the item table of the group lists.
+__global__ __launch_bounds__(256) void k_grouped_prep(const uint8_t* __restrict__ xq, int64_t n_blocks, int natural,
+                                                       uint32_t* __restrict__ img, int img_blocks,
+                                                       const uint64_t* __restrict__ grp_ptr,
+                                                       const int32_t* __restrict__ grp_start,
+                                                       const int32_t* __restrict__ ent_tok,
+                                                       const int32_t* __restrict__ ent_dst,
+                                                       const int32_t* __restrict__ counts, int cap_groups,
+                                                       int cap_entries, int n_tok, int n_rows, int4* __restrict__ items,
+                                                       int32_t* __restrict__ etok, int32_t* __restrict__ edst) {
+    if ((int)blockIdx.x < img_blocks) {
+        const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (b < n_blocks) q8_image(b, xq, natural, img);
+    } else {
+        group_items(((int)blockIdx.x - img_blocks) * 256 + (int)threadIdx.x, grp_ptr, grp_start, ent_tok, ent_dst, counts,
+                    cap_groups, cap_entries, n_tok, n_rows, items, etok, edst);
+    }
 }
 
 }  // namespace
 
-hipError_t launch_iota(int32_t* p, int n, hipStream_t s) {
-    hipLaunchKernelGGL(k_iota, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, p, n);
-    return hipGetLastError();
-}
-
 hipError_t launch_expert_group(const int32_t* ids, int n, int kpt, int E, const uint64_t* eptr, uint64_t* grp_ptr,
                                int32_t* grp_start, int32_t* grp_expert, int32_t* ent_dst, int32_t* ent_tok,
                                int32_t* miss_dst, int32_t* counts, int4* items, int cap_groups, int n_sh_items, int P,
-                               int T, int32_t* slot_id, hipStream_t s) {
+                               int T, hipStream_t s) {
     hipLaunchKernelGGL(k_expert_group, dim3(1), dim3(kGroupThreads), 0, s, ids, n, kpt, E, eptr, grp_ptr, grp_start,
-                       grp_expert, ent_dst, ent_tok, miss_dst, counts, items, cap_groups, n_sh_items, P, T, slot_id);
+                       grp_expert, ent_dst, ent_tok, miss_dst, counts, items, cap_groups, n_sh_items, P, T);
     return hipGetLastError();
 }
 
-hipError_t launch_group_items(const uint64_t* grp_ptr, const int32_t* grp_start, const int32_t* ent_tok,
-                              const int32_t* ent_dst, const int32_t* counts, int cap_groups, int cap_entries, int n_tok,
-                              int n_rows, int4* items, int32_t* etok, int32_t* edst, hipStream_t s) {
+hipError_t launch_grouped_prep(const uint8_t* xq, int64_t n_blocks, int natural, uint32_t* img, const uint64_t* grp_ptr,
+                               const int32_t* grp_start, const int32_t* ent_tok, const int32_t* ent_dst,
+                               const int32_t* counts, int cap_groups, int cap_entries, int n_tok, int n_rows,
+                               int4* items, int32_t* etok, int32_t* edst, hipStream_t s) {
     const int n = cap_groups > cap_entries ? cap_groups : cap_entries;
-    hipLaunchKernelGGL(k_group_items, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, grp_ptr, grp_start, ent_tok,
-                       ent_dst, counts, cap_groups, cap_entries, n_tok, n_rows, items, etok, edst);
-    return hipGetLastError();
-}
-
-hipError_t launch_q8_images(const uint8_t* xq, int64_t n_blocks, int natural, uint32_t* img, hipStream_t s) {
-    hipLaunchKernelGGL(k_q8_images, dim3((unsigned)((n_blocks + 255) / 256)), dim3(256), 0, s, xq, n_blocks, natural,
-                       img);
+    const int64_t ib = (n_blocks + 255) / 256;
+    if (ib + (n + 255) / 256 > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_grouped_prep, dim3((unsigned)(ib + (n + 255) / 256)), dim3(256), 0, s, xq, n_blocks, natural,
+                       img, (int)ib, grp_ptr, grp_start, ent_tok, ent_dst, counts, cap_groups, cap_entries, n_tok, n_rows,
+                       items, etok, edst);
     return hipGetLastError();
 }
 

@@ -2617,6 +2617,8 @@ __global__ __launch_bounds__(256) void k_q2_mmvq(const uint8_t* __restrict__ w, 
 
 // ------------------------------------------------------------------------------------------------ combine
 // y[t][j] = w0 * Y[slot0][j], then fma in selection order, then + shared (include/strata/kernels/native_moe.hpp:10-15).
+// SL false: the pair rows are in entry order (row t * k + i), without slots.
+template <bool SL>
 __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ Y, const int32_t* __restrict__ slot,
                                                   const float* __restrict__ wts, int k, int H, int P, int add_shared,
                                                   float* __restrict__ y) {
@@ -2630,7 +2632,7 @@ __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ Y, co
     float wt16[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        sl16[i] = sl[min(i, k - 1)];
+        sl16[i] = SL ? sl[min(i, k - 1)] : t * k + min(i, k - 1);
         wt16[i] = wt[min(i, k - 1)];
     }
     for (int j = blockIdx.y * 256 + threadIdx.x; j < H; j += gridDim.y * 256) {
@@ -2641,7 +2643,7 @@ __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ Y, co
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int s = min(s0 + i, k - 1);
-                const int r = s0 == 0 ? sl16[i] : sl[s];
+                const int r = s0 == 0 ? sl16[i] : SL ? sl[s] : t * k + s;
                 v[i] = Y[(size_t)r * H + j];
                 wv[i] = s0 == 0 ? wt16[i] : wt[s];
             }
@@ -2660,7 +2662,7 @@ __global__ __launch_bounds__(256) void k_combine(const float* __restrict__ Y, co
 // The same combine four neighbouring elements per thread (16-byte loads and stores; every element's sum is
 // formed exactly as above), NB pair rows per batch (NB >= k where k <= 16, so that no batch reloads rows).
 // H % 4 == 0, y 16-byte aligned.  NT: Y read and y written with streaming accesses (a Y larger than the caches).
-template <int NB, bool NT>
+template <int NB, bool NT, bool SL = true>
 __global__ __launch_bounds__(256) void k_combine4(const float* __restrict__ Y, const int32_t* __restrict__ slot,
                                                    const float* __restrict__ wts, int k, int H, int P, int add_shared,
                                                    float* __restrict__ y) {
@@ -2681,7 +2683,7 @@ __global__ __launch_bounds__(256) void k_combine4(const float* __restrict__ Y, c
     float wtb[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-        slb[i] = sl[min(i, k - 1)];
+        slb[i] = SL ? sl[min(i, k - 1)] : t * k + min(i, k - 1);
         wtb[i] = wt[min(i, k - 1)];
     }
     const int H4 = H >> 2;
@@ -2693,7 +2695,7 @@ __global__ __launch_bounds__(256) void k_combine4(const float* __restrict__ Y, c
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
                 const int s = min(s0 + i, k - 1);
-                const int r = s0 == 0 ? slb[i] : sl[s];
+                const int r = s0 == 0 ? slb[i] : SL ? sl[s] : t * k + s;
                 v[i] = ld(Y + (size_t)r * H + 4 * j);
                 wv[i] = s0 == 0 ? wtb[i] : wt[s];
             }
@@ -3196,7 +3198,9 @@ hipError_t launch_combine(const float* Y, const int32_t* slot, const float* wts,
         dim3 grid((unsigned)T, (unsigned)(ychunks < 8 ? ychunks : 8));
 #define SMOE_C4(NB)                                                                                                   \
     do {                                                                                                               \
-        if (nt) hipLaunchKernelGGL((k_combine4<NB, true>), grid, dim3(256), 0, s, Y, slot, wts, k, H, P, add_shared, y); \
+        if (!slot) hipLaunchKernelGGL((k_combine4<NB, false, false>), grid, dim3(256), 0, s, Y, slot, wts, k, H, P,    \
+                                      add_shared, y);                                                                  \
+        else if (nt) hipLaunchKernelGGL((k_combine4<NB, true>), grid, dim3(256), 0, s, Y, slot, wts, k, H, P, add_shared, y); \
         else hipLaunchKernelGGL((k_combine4<NB, false>), grid, dim3(256), 0, s, Y, slot, wts, k, H, P, add_shared, y);  \
     } while (0)
         if (k <= 4) SMOE_C4(4);
@@ -3209,7 +3213,8 @@ hipError_t launch_combine(const float* Y, const int32_t* slot, const float* wts,
     }
     const int ychunks = (H + 255) / 256;
     dim3 grid((unsigned)T, (unsigned)(ychunks < 8 ? ychunks : 8));
-    hipLaunchKernelGGL(k_combine, grid, dim3(256), 0, s, Y, slot, wts, k, H, P, add_shared, y);
+    if (slot) hipLaunchKernelGGL(k_combine<true>, grid, dim3(256), 0, s, Y, slot, wts, k, H, P, add_shared, y);
+    else hipLaunchKernelGGL(k_combine<false>, grid, dim3(256), 0, s, Y, slot, wts, k, H, P, add_shared, y);
     return hipGetLastError();
 }
 

@@ -165,19 +165,18 @@ hipError_t launch_hc_write(const float* R, const float* y, const float* inject, 
 
 // the expert tier (smoe_cache.hip): routed entries grouped by a table of one blob pointer per expert (at most
 // kMaxGroupExperts experts and kMaxGroupEntries entries), with the expert kernels' item table (group g = item g,
-// then n_sh_items shared chunks) and the identity slots of the rows' combine when asked; caller-made lists checked
-// into an item table; q8_1 blocks into activation images
+// then n_sh_items shared chunks) when asked; caller-made lists checked into an item table and q8_1 blocks into
+// activation images, in one launch
 constexpr int kMaxGroupExperts = 1024;
 constexpr int kMaxGroupEntries = 4096;
 hipError_t launch_expert_group(const int32_t* ids, int n, int kpt, int E, const uint64_t* eptr, uint64_t* grp_ptr,
                                int32_t* grp_start, int32_t* grp_expert, int32_t* ent_dst, int32_t* ent_tok,
                                int32_t* miss_dst, int32_t* counts, int4* items, int cap_groups, int n_sh_items, int P,
-                               int T, int32_t* slot_id, hipStream_t s);
-hipError_t launch_group_items(const uint64_t* grp_ptr, const int32_t* grp_start, const int32_t* ent_tok,
-                              const int32_t* ent_dst, const int32_t* counts, int cap_groups, int cap_entries, int n_tok,
-                              int n_rows, int4* items, int32_t* etok, int32_t* edst, hipStream_t s);
-hipError_t launch_q8_images(const uint8_t* xq, int64_t n_blocks, int natural, uint32_t* img, hipStream_t s);
-hipError_t launch_iota(int32_t* p, int n, hipStream_t s);
+                               int T, hipStream_t s);
+hipError_t launch_grouped_prep(const uint8_t* xq, int64_t n_blocks, int natural, uint32_t* img, const uint64_t* grp_ptr,
+                               const int32_t* grp_start, const int32_t* ent_tok, const int32_t* ent_dst,
+                               const int32_t* counts, int cap_groups, int cap_entries, int n_tok, int n_rows,
+                               int4* items, int32_t* etok, int32_t* edst, hipStream_t s);
 
 hipError_t launch_synth_blocks(int type, uint64_t seed, uint64_t stream_id, int64_t n_blocks, float sigma, uint8_t* out,
                                hipStream_t s);
