@@ -383,10 +383,12 @@ __device__ __forceinline__ void load_act_std(const uint8_t* __restrict__ blk, Ac
 // which the caller's LDS holds beyond its cap_cols columns), so the loads are not serialised behind branches;
 // a j with no live piece in the whole work-group is skipped.
 typedef __attribute__((ext_vector_type(4))) uint32_t img_u32x4;  // a native vector: stays in registers
-struct StagePieces {
-    img_u32x4 v[4];
-    int dst[4];
+template <int R>
+struct StageRounds {  // R rounds of one piece per thread
+    img_u32x4 v[R];
+    int dst[R];
 };
+using StagePieces = StageRounds<4>;
 template <int NT>
 __device__ __forceinline__ void stage_issue(StagePieces& sp, const uint32_t* __restrict__ img, int qb, int c0, int nc,
                                             int cap_cols, int base, const Item& it, const int32_t* perm, int k,
@@ -419,18 +421,18 @@ __device__ __forceinline__ void stage_commit(const StagePieces& sp, uint32_t* ac
     for (int j = 0; j < 4; ++j)
         if (base + j * nt < total) reinterpret_cast<img_u32x4*>(act)[lds_piece(sp.dst[j])] = sp.v[j];
 }
-// Round `base` with rows that need no memory read (see stage_issue) as straight-line code: all four loads
+// Round `base` with rows that need no memory read (see stage_issue) as straight-line code: all R loads
 // unconditional (a piece past the end, or a whole j past the end, reloads the last piece and is stored to the
 // dead slot), so that the compiler counts the loads in flight exactly and a later store waits for its own load
 // alone.
-template <int NT>
-__device__ __forceinline__ void stage_issue_direct(StagePieces& sp, const uint32_t* __restrict__ img, int qb, int c0,
+template <int NT, int R>
+__device__ __forceinline__ void stage_issue_direct(StageRounds<R>& sp, const uint32_t* __restrict__ img, int qb, int c0,
                                                    int nc, int cap_cols, int base, const Item& it, bool by_token) {
     const int per_col = qb * (kImgDw / 4);
     const int total = nc * per_col, dead = cap_cols * per_col;
     constexpr int nt = NT;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < R; ++j) {
         const int raw = base + j * nt + (int)threadIdx.x;
         const int idx = min(raw, total - 1);
         const int c = idx / per_col;
@@ -439,9 +441,10 @@ __device__ __forceinline__ void stage_issue_direct(StagePieces& sp, const uint32
         sp.dst[j] = raw < total ? raw : dead;
     }
 }
-__device__ __forceinline__ void stage_commit_direct(const StagePieces& sp, uint32_t* act) {
+template <int R>
+__device__ __forceinline__ void stage_commit_direct(const StageRounds<R>& sp, uint32_t* act) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) reinterpret_cast<img_u32x4*>(act)[lds_piece(sp.dst[j])] = sp.v[j];
+    for (int j = 0; j < R; ++j) reinterpret_cast<img_u32x4*>(act)[lds_piece(sp.dst[j])] = sp.v[j];
 }
 // True when stage_issue_direct can serve columns c0 .. c0 + nc.
 __device__ __forceinline__ bool stage_direct(const Item& it, int c0, int nc, bool by_token) {

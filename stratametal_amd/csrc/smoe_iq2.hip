@@ -102,6 +102,10 @@ __device__ __forceinline__ uint32_t load_block_raw(const uint8_t* row, int b, ui
     return (b & 1) ? 0u : 2u;
 }
 
+// The kernels are bound by VALU issue, of which this is the larger part (IQ2_S batch 64: two thirds of a wave's
+// instructions before its one or two columns): per group of 8 weights a table read, four instructions for its index and
+// two nibble multiplies, merges and permutes for its signs (with field extracts per group and the staging's indices not
+// constant, k_iq2_gu of 64 tokens took 107 us and k_iq2_down 46, against 95 and 40).
 __device__ __forceinline__ void decode_block(const uint32_t (&raw)[21], uint32_t sh, const uint2* __restrict__ tab,
                                              Iq2Block& B) {
     // field dword m (m = 0 .. 19 from byte 2: qs 0-7, signs 8-15, qh 16-17, scales 18-19)
@@ -113,16 +117,23 @@ __device__ __forceinline__ void decode_block(const uint32_t (&raw)[21], uint32_t
     B.sc[1] = fd(19);
 #pragma unroll
     for (int ib = 0; ib < 8; ++ib) {
-        const uint32_t qsd = fd(ib);
-        const uint32_t sgd = fd(8 + ib);
-        const uint32_t qhd = ib < 4 ? qh0 : qh1;
+        const uint32_t qsd = fd(ib), sgd = fd(8 + ib);
+        // the groups' sign nibbles as bytes (opaque, so that a nibble is a byte operand of its multiply, not a field extract)
+        uint32_t slo = sgd & 0x0F0F0F0Fu, shi = (sgd >> 4) & 0x0F0F0F0Fu;
+        asm("" : "+v"(slo), "+v"(shi));
+        // the groups' high index bits (2 each) spread to one byte each, then the 10-bit indices as 16-bit halves, as byte
+        // offsets of the 8-byte entries
+        const uint32_t qhb = ((ib < 4 ? qh0 : qh1) >> (8 * (ib & 3))) & 0xFFu;
+        const uint32_t hi2 = (qhb | (qhb << 12)) & 0x000F000Fu, hi = (hi2 | (hi2 << 6)) & 0x03030303u;
+        const uint32_t i01 = __builtin_amdgcn_perm(hi, qsd, 0x05010400u) << 3;
+        const uint32_t i23 = __builtin_amdgcn_perm(hi, qsd, 0x07030602u) << 3;
 #pragma unroll
         for (int grp = 0; grp < 4; ++grp) {
-            const uint32_t idx = ((qsd >> (8 * grp)) & 0xFFu) | (((qhd >> (8 * (ib & 3) + 2 * grp)) & 3u) << 8);
-            const uint2 e = tab[idx];
-            const uint32_t sb = (sgd >> (8 * grp)) & 0xFFu;
-            B.w[2 * (4 * ib + grp)] = signed_mags(e.x, sb & 15u);
-            B.w[2 * (4 * ib + grp) + 1] = signed_mags(e.y, sb >> 4);
+            const uint32_t ip = grp < 2 ? i01 : i23;
+            const uint2 e = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint8_t*>(tab) +
+                                                            ((grp & 1) ? ip >> 16 : ip & 0xFFFFu));
+            B.w[2 * (4 * ib + grp)] = signed_mags(e.x, (slo >> (8 * grp)) & 0xFFu);
+            B.w[2 * (4 * ib + grp) + 1] = signed_mags(e.y, (shi >> (8 * grp)) & 0xFFu);
         }
     }
 }
@@ -195,6 +206,7 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
                                                      const uint8_t* __restrict__ up_sh, const int32_t* __restrict__ perm,
                                                      uint32_t* __restrict__ himg, int h_blocks, const StageOut so) {
     constexpr int kCols = 2 * NW;
+    constexpr int kDirect = 2;  // staging rounds of 64 NW pieces that hold four columns of 24 NW
     extern __shared__ __align__(16) uint32_t smem[];
     __shared__ uint2 tab[kIq2sTabEntries];
     __shared__ float rowv[kCols][64];
@@ -204,7 +216,7 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
     const int hb = blockIdx.x;
     const int Fe = item.shared ? Fs : F;
     if (hb * 32 >= Fe) return;
-    const int nb = H >> 8;  // == NW
+    constexpr int nb = NW, qb = 8 * NW;  // blocks and 32-value images of a row: H = 256 NW
     const size_t rb = (size_t)nb * 82;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int rho = wave * (64 / nb) + lane / nb, b = lane % nb;
@@ -216,7 +228,6 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
     const uint8_t* base = (rho < 32 ? (item.shared ? gate_sh : gate_exps + (size_t)item.e * F * rb)
                                     : (item.shared ? up_sh : up_exps + (size_t)item.e * F * rb));
     const uint8_t* rowp = base + (size_t)(32 * hb + (rho & 31)) * rb;
-    const int qb = H >> 5;
     // loads in the order their data is needed: the grid codes, the first column batch's images (when their rows
     // need no memory read), then the weights; the table store waits for the codes alone, the image commit for
     // the images alone
@@ -226,7 +237,7 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
     uint32_t raw[21];
     uint32_t off;
     if (stage_direct(item, 0, nc0, true)) {  // straight-line inside each branch, so no wait lands between the loads
-        StagePieces sp;
+        StageRounds<kDirect> sp;
         stage_issue_direct<64 * NW>(sp, ximg, qb, 0, nc0, kCols, 0, item, true);
         __builtin_amdgcn_sched_barrier(0);
         off = load_block_raw(rowp, b, raw);
@@ -236,9 +247,10 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
     } else {
         off = load_block_raw(rowp, b, raw);
         grid_table_store<64 * NW>(codes, tab);
-        stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, 0, 4 * 64 * NW);
+        stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, 0, kDirect * 64 * NW);
     }
-    stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, 4 * 64 * NW);  // rounds beyond the first
+    if (nc0 > 4)  // columns beyond those rounds
+        stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, kDirect * 64 * NW);
     __syncthreads();
     Iq2Block B[1];
     decode_block(raw, off, tab, B[0]);
@@ -274,24 +286,24 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
 // Grid (H / (4 * 64 / nbf), work items); nbf = F / 256 lanes per row, 64 / nbf rows per wave.  The item's h
 // images are copied to LDS `cps` columns at a time; each group leader writes Y[first + c][row] (the shared
 // rows times sigmoid(sg[t])).
-// (Arguments ordered as k_iq2_gu's.)
+// (Arguments ordered as k_iq2_gu's.)  NB = F / 256 (a shared expert is as wide as the routed ones).
+template <int NB>
 __global__ __launch_bounds__(256) void k_iq2_down(const int4* __restrict__ items, const uint32_t* __restrict__ himg,
                                                    const uint8_t* __restrict__ down_exps,
-                                                   const uint64_t* __restrict__ eptr, int H, int F, int Fs,
-                                                   int h_blocks, int cps, const uint8_t* __restrict__ down_sh,
+                                                   const uint64_t* __restrict__ eptr, int H, int cps,
+                                                   const uint8_t* __restrict__ down_sh,
                                                    const float* __restrict__ sg, float* __restrict__ Y,
                                                    const int32_t* __restrict__ dmap) {
     extern __shared__ __align__(16) uint32_t smem[];
     __shared__ uint2 tab[kIq2sTabEntries];
     Item item;
     if (!work_item(items, blockIdx.y, item)) return;
-    const int Fe = item.shared ? Fs : F;
-    const int nb = Fe >> 8;
-    const size_t rb = (size_t)nb * 82;
+    constexpr int nb = NB, h_blocks = 8 * NB;
+    constexpr size_t rb = (size_t)nb * 82;
     const uint8_t* base =
         item.shared ? down_sh
-        : eptr      ? reinterpret_cast<const uint8_t*>(eptr[item.e]) + (size_t)2 * F * ((size_t)(H >> 8) * 82)
-                    : down_exps + (size_t)item.e * H * ((size_t)(F >> 8) * 82);
+        : eptr      ? reinterpret_cast<const uint8_t*>(eptr[item.e]) + (size_t)2 * (256 * NB) * ((size_t)(H >> 8) * 82)
+                    : down_exps + (size_t)item.e * H * rb;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int rpw = 64 / nb, grp = lane / nb, b = lane - grp * nb;
     const int r = blockIdx.x * 4 * rpw + wave * rpw + grp;
@@ -301,7 +313,7 @@ __global__ __launch_bounds__(256) void k_iq2_down(const int4* __restrict__ items
     uint4 codes[kTabRounds<256>];
     grid_codes_load<256>(codes);
     const int nc0 = min(cps, item.ncol);
-    StagePieces sp;
+    StageRounds<1> sp;
     stage_issue_direct<256>(sp, himg, h_blocks, 0, nc0, cps, 0, item, false);
     __builtin_amdgcn_sched_barrier(0);
     uint32_t raw[21];
@@ -310,7 +322,8 @@ __global__ __launch_bounds__(256) void k_iq2_down(const int4* __restrict__ items
     __builtin_amdgcn_sched_barrier(0);
     grid_table_store<256>(codes, tab);
     stage_commit_direct(sp, smem);
-    stage_images<256>(smem, himg, h_blocks, 0, nc0, cps, item, nullptr, 1, false, 4 * 256);  // rounds beyond the first
+    if (nc0 * 24 * NB > 256)  // rounds beyond the first
+        stage_images<256>(smem, himg, h_blocks, 0, nc0, cps, item, nullptr, 1, false, 256);
     __syncthreads();
     Iq2Block B[1];
     decode_block(raw, off, tab, B[0]);
@@ -393,13 +406,20 @@ hipError_t launch_iq2_gu(const uint8_t* gate_exps, const uint8_t* up_exps, const
 hipError_t launch_iq2_down(const uint8_t* down_exps, const uint8_t* down_sh, const uint32_t* himg, int h_blocks,
                            const float* sg, const int4* items, int H, int F, int Fs, int max_items, float* Y,
                            hipStream_t s, const uint64_t* eptr, const int32_t* dmap) {
-    const int rpw = 64 / (F / 256);  // the caller guarantees the shared width has the same row shape
+    // the shared expert of an IQ2_S layer is as wide as the routed ones, and h rows are that wide
+    if ((F != 512 && F != 1024 && F != 2048) || h_blocks != F / 32 || (Fs != 0 && Fs != F)) return hipErrorInvalidValue;
+    const int rpw = 64 / (F / 256);
     dim3 grid((unsigned)((H + 4 * rpw - 1) / (4 * rpw)), (unsigned)max_items);
     const size_t col_bytes = (size_t)h_blocks * kImgLdsDw * 4;
     int cps = (int)(24576 / col_bytes);
     cps = cps < 1 ? 1 : cps > 16 ? 16 : cps;
-    hipLaunchKernelGGL(k_iq2_down, grid, dim3(256), (size_t)cps * col_bytes + 16, s, items, himg, down_exps, eptr, H, F,
-                       Fs, h_blocks, cps, down_sh, sg, Y, dmap);
+#define SMOE_IQ2_DOWN(NB)                                                                                            \
+    hipLaunchKernelGGL((k_iq2_down<NB>), grid, dim3(256), (size_t)cps * col_bytes + 16, s, items, himg, down_exps, eptr, H, \
+                       cps, down_sh, sg, Y, dmap)
+    if (F == 512) SMOE_IQ2_DOWN(2);
+    else if (F == 1024) SMOE_IQ2_DOWN(4);
+    else SMOE_IQ2_DOWN(8);
+#undef SMOE_IQ2_DOWN
     return hipGetLastError();
 }
 
