@@ -139,6 +139,12 @@ int max_items_mfma(const smoe_geom& g, int64_t T) {
     const int64_t P = T * g.top_k, C = smoe::mfma_chunk();
     return (int)((P < g.n_expert ? P : g.n_expert) + P / C + (sh_fused(g) ? (T + C - 1) / C : 0));
 }
+// The IQ2_S products on the matrix cores take chunks of columns of their own.
+bool iq2_mm(const smoe_geom& g, int64_t T) { return g.w_type == SMOE_IQ2_S && smoe::iq2_mm_batch(T * g.top_k, g.n_expert); }
+int max_items_iq2_mm(const smoe_geom& g, int64_t T) {
+    const int64_t P = T * g.top_k, S = smoe::iq2_mm_shared_chunk();
+    return (int)((P < g.n_expert ? P : g.n_expert) + P / smoe::iq2_mm_chunk() + (sh_fused(g) ? (T + S - 1) / S : 0));
+}
 
 Layout layout(const smoe_geom& g, int64_t T) {
     Layout L{};
@@ -167,7 +173,7 @@ Layout layout(const smoe_geom& g, int64_t T) {
     L.slot = take((size_t)P * 4);
     L.elist = take((size_t)(E + 1) * 4);
     L.nlist = take(16);
-    L.items = take((size_t)most(max_items_gemv(g, T), max_items_mfma(g, T)) * 32);
+    L.items = take(most(most(max_items_gemv(g, T), max_items_mfma(g, T)), max_items_iq2_mm(g, T)) * 32);
     L.himg = take(most(smoe::img_bytes((P + T) * L.h_blocks), smoe::act_rec_bytes((P + T) * L.h_rec)));
     L.Y = take((size_t)(P + T) * H * 4);
     L.dwork = take(smoe::dispatch_work_bytes(P, (int)E));  // chunk histograms of the many-pair dispatch
@@ -287,6 +293,7 @@ smoe_status check_forward(const smoe_geom* g, const smoe_weights* w, const float
     if (n_tokens > kMaxGridY)
         return fail(SMOE_EINVAL, std::to_string(n_tokens) + " tokens exceed " + std::to_string(kMaxGridY) +
                                      " per call; split the batch");
+    // (a traced call runs the kernels whose grid takes the items on its y dimension, whatever the batch)
     const int64_t n_items = mfma ? max_items_mfma(*g, n_tokens) : max_items_gemv(*g, n_tokens);
     if (n_items > kMaxGridY)
         return fail(SMOE_EINVAL, std::to_string(n_items) + " expert work items exceed " + std::to_string(kMaxGridY) +
@@ -448,14 +455,18 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
     uint32_t* himg = reinterpret_cast<uint32_t*>(ws + L.himg);
     float* Y = reinterpret_cast<float*>(ws + L.Y);
     const hipStream_t st = stream_of(hip_stream);
-    const int n_items = mfma ? max_items_mfma(*g, T) : max_items_gemv(*g, T);
-    const int chunk = mfma ? smoe::mfma_chunk() : (1 << 30);
+    // the expert stages of the trace: the decode path's unfused kernels, so that every stage lands in memory
+    const bool stages = trace && (trace->xq || trace->hq || trace->parts || trace->shared || trace->egate ||
+                                  trace->eup || trace->sgu || trace->shq);
+    const bool imm = iq2_mm(*g, T) && !stages;  // the IQ2_S products on the matrix cores
+    const int n_items = mfma ? max_items_mfma(*g, T) : imm ? max_items_iq2_mm(*g, T) : max_items_gemv(*g, T);
+    const int chunk = mfma ? smoe::mfma_chunk() : imm ? smoe::iq2_mm_chunk() : (1 << 30);
     // the prefill path's per-pair rows Y past kYStreamBytes: the down kernels store them and the combine reads them
     // (and writes y) with streaming accesses, which keep them out of the XCDs' L2 (measured at 4096 tokens of the
     // benchmark's layer, 369 MB of Y: 50 us less per layer; at 512 tokens, 46 MB, the combine reads Y back from the
     // Infinity Cache and the streaming loads cost it 1.5 us)
     const bool y_stream = mfma && (size_t)(P + T) * (size_t)H * sizeof(float) > kYStreamBytes;
-    const int sh_chunk = mfma ? smoe::mfma_chunk() : smoe::gemv_shared_chunk();
+    const int sh_chunk = mfma ? smoe::mfma_chunk() : imm ? smoe::iq2_mm_shared_chunk() : smoe::gemv_shared_chunk();
 
     void* const* ev = trace ? trace->stage_events : nullptr;
     int ev_i = 0;
@@ -472,9 +483,6 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
     SMOE_MARK();
     // the junction is fused into the router kernel of few tokens; more tokens take it as a kernel of its own
     const bool fused_norm = x_prev && !mfma && n_tokens < kJunctionApartTokens;
-    // the expert stages of the trace: the decode path's unfused kernels, so that every stage lands in memory
-    const bool stages = trace && (trace->xq || trace->hq || trace->parts || trace->shared || trace->egate ||
-                                  trace->eup || trace->sgu || trace->shq);
     // the prefill path's per-work-group flags of its fp16 operand limits (folded by a trace or smoe_forward_status)
     int32_t* xflags = mfma ? reinterpret_cast<int32_t*>(ws + L.oflags) : nullptr;
     int32_t* hflags = xflags ? xflags + L.n_xflags : nullptr;
@@ -551,6 +559,11 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
         SMOE_TRY(smoe::launch_mm_down(de, ds, himg, (int64_t)(P + T) * L.h_rec, L.h_rec, sg, items, H, F, Fs, n_items,
                                       Y, y_stream ? 1 : 0, st),
                  "down");
+    } else if (imm) {
+        SMOE_TRY(smoe::launch_iq2_mm_gu(ge, ue, gs, us, ximg, items, perm, K, H, F, n_items, himg, L.h_blocks, st),
+                 "gate/up");
+        SMOE_MARK();
+        SMOE_TRY(smoe::launch_iq2_mm_down(de, ds, himg, L.h_blocks, sg, items, H, F, n_items, Y, st), "down");
     } else if (iq2) {
         SMOE_TRY(smoe::launch_iq2_gu(ge, ue, gs, us, ximg, items, perm, K, H, F, Fs, shf ? 1 : 0, n_items, himg,
                                      L.h_blocks, st, &so),

@@ -347,6 +347,18 @@ __device__ __forceinline__ void load_act_img(const uint32_t* __restrict__ img, A
     }
 }
 
+// IQ2_S block b of a row (rows are a whole number of block pairs, 164 bytes, so dword aligned).  Every field after the
+// scale (qs @2, signs @34, qh @66, scales @74) starts at byte 2 modulo 4, so the block is loaded so that each
+// field dword is one alignbyte of two raw dwords with a per-lane shift: an even block's 80 bytes from its first
+// byte (shift 2), an odd block's from its byte 2 (shift 0, the pair's bytes 84 .. 163); raw[20] is the pair's
+// dword 20 for both (the even block's bytes 80-83, the odd block's scale in its high half).  Returns the shift.
+__device__ __forceinline__ uint32_t load_block_raw(const uint8_t* row, int b, uint32_t (&raw)[21]) {
+    const uint8_t* pair = row + (size_t)(b >> 1) * 164;
+    __builtin_memcpy(raw, __builtin_assume_aligned(pair + ((b & 1) ? 84 : 0), 4), 80);
+    raw[20] = *reinterpret_cast<const uint32_t*>(__builtin_assume_aligned(pair + 80, 4));
+    return (b & 1) ? 0u : 2u;
+}
+
 __device__ __forceinline__ void transpose4x4(uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3, uint32_t* o) {
     const uint32_t t0 = __builtin_amdgcn_perm(a1, a0, 0x05010400u);
     const uint32_t u0 = __builtin_amdgcn_perm(a3, a2, 0x05010400u);

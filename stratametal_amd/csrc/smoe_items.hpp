@@ -66,4 +66,19 @@ __device__ __forceinline__ int item_token(const Item& it, const int32_t* perm, i
     return perm[it.first + c] / k;
 }
 
+// The expert GEMMs' 1-D grids: work-group id -> (work item y, row block rb).  The dispatcher deals linear ids round
+// robin over the 8 XCDs, so the n_rb row blocks of item y are given the ids 8 (n_rb (y / 8) + rb) + y % 8: one XCD,
+// dispatched back to back, reading the item's activation records from memory once and then from that XCD's L2 (a 2-D
+// grid of (row block, item) put each row block of an item on another XCD).  The grid holds n_rb * (max_items rounded
+// up to 8) work-groups; false past max_items.
+__device__ __forceinline__ bool xcd_item(int n_rb, int max_items, int& y, int& rb) {
+    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3, g = slot / n_rb;
+    y = 8 * g + xcd;
+    rb = slot - n_rb * g;
+    return y < max_items;
+}
+__host__ __device__ inline unsigned xcd_grid(int n_rb, int max_items) {
+    return (unsigned)(n_rb * ((max_items + 7) / 8) * 8);
+}
+
 }  // namespace smoe

@@ -480,21 +480,6 @@ __device__ __forceinline__ float silu_mul_fast(float g, float u) {
     return (g * __builtin_amdgcn_rcpf(1.0f + e)) * u;
 }
 
-// The expert GEMMs' 1-D grids: work-group id -> (work item y, row block rb).  The dispatcher deals linear ids round
-// robin over the 8 XCDs, so the n_rb row blocks of item y are given the ids 8 (n_rb (y / 8) + rb) + y % 8: one XCD,
-// dispatched back to back, reading the item's activation records from memory once and then from that XCD's L2 (a 2-D
-// grid of (row block, item) put each row block of an item on another XCD).  The grid holds n_rb * (max_items rounded
-// up to 8) work-groups; false past max_items.
-__device__ __forceinline__ bool xcd_item(int n_rb, int max_items, int& y, int& rb) {
-    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3, g = slot / n_rb;
-    y = 8 * g + xcd;
-    rb = slot - n_rb * g;
-    return y < max_items;
-}
-__host__ __device__ inline unsigned xcd_grid(int n_rb, int max_items) {
-    return (unsigned)(n_rb * ((max_items + 7) / 8) * 8);
-}
-
 template <int MODE>
 __device__ __forceinline__ void mm_gu_body(uint8_t* lds, const int* rowidx, const Item& item, int ncol, int rt,
                                            const uint8_t* g0, const uint8_t* u0, const uint32_t* xrec,
