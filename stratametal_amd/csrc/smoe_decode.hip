@@ -2981,13 +2981,19 @@ int shared_items(int T) { return (T + kShCols - 1) / kShCols; }
 int gemv_shared_chunk() { return kShCols; }
 
 
+// Passes per wave and units per lane as constants: the unit loads are unconditional, so a kernel with more slots than the
+// row has units reloads the first in the others.  Odd unit counts have kernels of their own (2560 values are five units of
+// four lanes): with eight slots the gate/up and down of 77 tokens, 512 experts of 2560 by 640, took 115 and 68 us, the
+// whole call 198; with five the call takes 171.
 #define SMOE_SHAPE_DISPATCH(KERNEL_MACRO)              \
     if (nit == 4 && upl == 1) KERNEL_MACRO(4, 1);      \
     else if (nit == 4) KERNEL_MACRO(4, 2);             \
     else if (nit == 2 && upl == 1) KERNEL_MACRO(2, 1); \
     else if (nit == 2) KERNEL_MACRO(2, 4);             \
     else if (upl <= 2) KERNEL_MACRO(1, 2);             \
-    else if (upl <= 4) KERNEL_MACRO(1, 4);             \
+    else if (upl == 3) KERNEL_MACRO(1, 3);             \
+    else if (upl == 4) KERNEL_MACRO(1, 4);             \
+    else if (upl == 5) KERNEL_MACRO(1, 5);             \
     else KERNEL_MACRO(1, 8);
 
 hipError_t launch_q2_gu(const uint8_t* gate_exps, const uint8_t* up_exps, const uint8_t* gate_sh, const uint8_t* up_sh,
