@@ -380,10 +380,10 @@ bool recall_flags(const void* ws, FlagWords& f) {
 // The native shared expert (its projections in their own types): q8_1 of x, gate and up, SwiGLU + q8_1, down
 // times sigmoid(sg[t]) into out[t] (T rows of n_embd), in the workspace's native-chain slots.  `stages`: every stage is
 // wanted in memory (a trace).  `add_to`: the rows are added to it (a combine that left them out: its own last addition),
-// and out need not hold them.
+// and out need not hold them.  `mm`: the prefill contract, whose products may run on the matrix cores.
 smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float* x, int T, uint8_t* ws,
                           const Layout& L, float* out, const float* sg, hipStream_t st, bool stages = false,
-                          float* add_to = nullptr) {
+                          float* add_to = nullptr, bool mm = false) {
     const int H = g.n_embd, Fn = g.n_ff_shared;
     uint8_t* nxq = ws + L.nxq;
     float* ngu = reinterpret_cast<float*>(ws + L.ngu);
@@ -391,6 +391,7 @@ smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float
     auto gemv = [&](int type, const void* wt, const uint8_t* xq, int n_in, int n_out, float* y,
                     const float* gate) -> hipError_t {
         const uint8_t* wb = static_cast<const uint8_t*>(wt);
+        if (mm && smoe::native_mm_ok(type, n_out)) return smoe::launch_native_mm(type, wb, xq, n_in, n_out, T, y, n_out, gate, st);
         if (smoe::native_type(type)) return smoe::launch_mmvq_native(type, wb, xq, n_in, n_out, T, y, n_out, gate, st);
         hipError_t e = type == SMOE_IQ2_S ? smoe::launch_iq2_mmvq(wb, xq, n_in, n_out, T, y, st)
                                           : smoe::launch_q2_mmvq(wb, xq, n_in, n_out, T, y, st);
@@ -409,8 +410,8 @@ smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float
     }
     SMOE_TRY(smoe::launch_prep(x, (int64_t)T * H, nxq, nullptr, st), "shared q8_1");
     if (pair) {
-        SMOE_TRY(smoe::launch_mmvq_native(tg, gw, nxq, H, Fn, T, ngu, Fn, nullptr, st, uw, ngu + (size_t)T * Fn),
-                 "shared gate/up");
+        const auto gu = mm && smoe::native_mm_ok(tg, Fn) ? smoe::launch_native_mm : smoe::launch_mmvq_native;
+        SMOE_TRY(gu(tg, gw, nxq, H, Fn, T, ngu, Fn, nullptr, st, uw, ngu + (size_t)T * Fn), "shared gate/up");
     } else {
         SMOE_TRY(gemv(tg, gw, nxq, H, Fn, ngu, nullptr), "shared gate");
         SMOE_TRY(gemv(sh_up_t(g), uw, nxq, H, Fn, ngu + (size_t)T * Fn, nullptr), "shared up");
@@ -598,7 +599,7 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
     // a native shared expert's rows into Y for the combine, or added to y after the fused combine, which left them out
     if (nat)
         SMOE_TRY_S(native_shared(*g, w, x_io, T, ws, L, Y + (size_t)P * H, sg, st, stages,
-                                 small_down && add_shared ? y : nullptr));
+                                 small_down && add_shared ? y : nullptr, mfma));
     if (!small_down)
         SMOE_TRY(smoe::launch_combine(Y, slot, wts, K, H, P, T, (has_sh && add_shared) ? 1 : 0, y, st,
                                       y_stream ? 1 : 0),
