@@ -60,10 +60,11 @@ struct MmLds {
 static_assert(sizeof(float) * kCols * kHPitch <= sizeof(uint8_t) * kCols * kXPitch, "the h tile fits the x tile");
 
 // Column tile `c0` of the item against two row sets: wave w, lane (q, i) returns rows 16 w + 4 q .. + 3 of set s and
-// column i in out[s].  row0 / row1: the lane's row i of the wave in each set; rowidx: image row of each column.
+// column i in out[s].  row0 / row1: the lane's row i of the wave in each set; rowidx: image row of each column.  With
+// `staged` the tile's x is in LDS from the call before (one phase: rows of at most four blocks).
 template <int NB>
 __device__ __forceinline__ void mm_tile(MmLds& s, const uint8_t* row0, const uint8_t* row1, const uint32_t* img,
-                                        const int* rowidx, f32x4 (&out)[2]) {
+                                        const int* rowidx, f32x4 (&out)[2], bool staged = false) {
     constexpr int PB = NB < kPhaseBlocks ? NB : kPhaseBlocks, PH = NB / PB;
     const int tid = threadIdx.x, lane = tid & 63, i = lane & 15, q = lane >> 4;
     // block of step k in phase ph: the order whose pairwise sums are the butterfly's
@@ -75,7 +76,7 @@ __device__ __forceinline__ void mm_tile(MmLds& s, const uint8_t* row0, const uin
     for (int ph = 0; ph < PH; ++ph) {
         if (ph) __syncthreads();  // the phase before is done with s.x
         // x of the phase's blocks as fp16 in the weights' pair order, one group of 8 values per piece
-        for (int p = tid; p < kCols * PB * 32; p += kThreads) {
+        for (int p = staged ? kCols * PB * 32 : tid; p < kCols * PB * 32; p += kThreads) {
             const int c = p / (PB * 32), g = p % (PB * 32), k = g >> 5, sub = (g >> 2) & 7;
             const uint32_t* src = img + ((size_t)rowidx[c] * (8 * NB) + 8 * block_of(ph, k) + sub) * kImgDw;
             const uint2 w = *reinterpret_cast<const uint2*>(src + 2 * (g & 3));
@@ -90,7 +91,7 @@ __device__ __forceinline__ void mm_tile(MmLds& s, const uint8_t* row0, const uin
             *reinterpret_cast<u32x4*>(s.x + c * kXPitch + 16 * g) = o;
             if ((g & 3) == 0) s.dx[c][g >> 2] = u2f(src[8]);
         }
-        __syncthreads();
+        if (!staged) __syncthreads();  // (uniform)
         f32x4 pair = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, tot = pair;
         // the steps of set 0, then of set 1 (not unrolled: one step's code is eight sub-blocks)
 #pragma clang loop unroll(disable)
@@ -217,9 +218,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
 }
 
-// Down: work-group (item y, row block rt) computes down rows [256 rt, 256 rt + 256) of the item's columns into Y[first + c]
-// (the shared expert's times sigmoid(sg[t])): wave w rows 32 w .. + 15 (set 0) and 32 w + 16 .. + 15 (set 1).
-template <int NB>
+// Down: work-group (item y, row block rt) computes down rows [256 RP rt, 256 RP rt + 256 RP) of the item's columns into
+// Y[first + c] (the shared expert's times sigmoid(sg[t])), 256 rows a pass: wave w rows 32 w .. + 15 (set 0) and 32 w + 16
+// .. + 15 (set 1).  The passes of a tile share its staged x, and the work-group its grid table.
+template <int NB, int RP>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_iq2_mm_down(
     const int4* __restrict__ items, int max_items, int n_rb, const uint32_t* __restrict__ himg,
     const uint8_t* __restrict__ down_exps, const uint8_t* __restrict__ down_sh, int H, const float* __restrict__ sg,
@@ -232,22 +234,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     if (!work_item(items, y, item)) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 15, q = lane >> 4;
     constexpr size_t rb = (size_t)NB * 82;
-    const int row = 256 * rt + 32 * wave;
+    static_assert(RP == 1 || NB <= kPhaseBlocks, "several passes: x staged in one phase");
+    const int row = 256 * RP * rt + 32 * wave;
     const uint8_t* d = (item.shared ? down_sh : down_exps + (size_t)item.e * H * rb) + (size_t)(row + i) * rb;
     load_table(s);
     for (int c0 = 0; c0 < item.ncol; c0 += kCols) {
         const int nc = min(kCols, item.ncol - c0);
         if (tid < kCols) rowidx[tid] = item.first + c0 + min(tid, nc - 1);
         __syncthreads();
-        f32x4 o[2];
-        mm_tile<NB>(s, d, d + 16 * rb, himg, rowidx, o);
-        if (i < nc) {
-            const float gs = item.shared ? sigmoid(sg[item.tok0 + c0 + i]) : 1.0f;
+        const float gs = item.shared && i < nc ? sigmoid(sg[item.tok0 + c0 + i]) : 1.0f;
+#pragma clang loop unroll(disable)
+        for (int pass = 0; pass < RP; ++pass) {
+            const uint8_t* dp = d + (size_t)(256 * pass) * rb;
+            f32x4 o[2];
+            mm_tile<NB>(s, dp, dp + 16 * rb, himg, rowidx, o, pass > 0);
+            if (i < nc) {
 #pragma unroll
-            for (int set = 0; set < 2; ++set) {
-                f32x4 v = o[set];
-                if (item.shared) v = f32x4{v[0] * gs, v[1] * gs, v[2] * gs, v[3] * gs};
-                *reinterpret_cast<f32x4*>(Y + (size_t)(item.first + c0 + i) * H + row + 16 * set + 4 * q) = v;
+                for (int set = 0; set < 2; ++set) {
+                    f32x4 v = o[set];
+                    if (item.shared) v = f32x4{v[0] * gs, v[1] * gs, v[2] * gs, v[3] * gs};
+                    *reinterpret_cast<f32x4*>(Y + (size_t)(item.first + c0 + i) * H + row + 256 * pass + 16 * set + 4 * q) = v;
+                }
             }
         }
         __syncthreads();  // every wave is done with s.x and rowidx
@@ -271,17 +278,23 @@ hipError_t launch_iq2_mm_gu(const uint8_t* gate_exps, const uint8_t* up_exps, co
     return hipGetLastError();
 }
 
+constexpr int kDownTwoPasses = 2048;
 hipError_t launch_iq2_mm_down(const uint8_t* down_exps, const uint8_t* down_sh, const uint32_t* himg, int h_blocks,
                               const float* sg, const int4* items, int H, int F, int max_items, float* Y, hipStream_t s) {
     if (!iq2_shape_ok(H) || !iq2_shape_ok(F) || h_blocks != F / 32) return hipErrorInvalidValue;
-    const int n_rb = H / 256;
+    // two passes where the halved grid still fills the chip (two work-groups per CU) four times
+    // (600 tokens of 512 experts, 2048 rows of 512: 165 us one by one, 155 in twos)
+    const int rp = F <= 1024 && H % 512 == 0 && (int64_t)max_items * (H / 512) >= kDownTwoPasses ? 2 : 1;
+    const int n_rb = H / (256 * rp);
     const dim3 grid(xcd_grid(n_rb, max_items));
-#define SMOE_MM_DOWN(NB)                                                                                           \
-    hipLaunchKernelGGL((k_iq2_mm_down<NB>), grid, dim3(kThreads), 0, s, items, max_items, n_rb, himg, down_exps, down_sh, \
-                       H, sg, Y)
-    if (F == 512) SMOE_MM_DOWN(2);
-    else if (F == 1024) SMOE_MM_DOWN(4);
-    else SMOE_MM_DOWN(8);
+#define SMOE_MM_DOWN(NB, RP)                                                                                       \
+    hipLaunchKernelGGL((k_iq2_mm_down<NB, RP>), grid, dim3(kThreads), 0, s, items, max_items, n_rb, himg, down_exps, \
+                       down_sh, H, sg, Y)
+    if (F == 512 && rp == 2) SMOE_MM_DOWN(2, 2);
+    else if (F == 512) SMOE_MM_DOWN(2, 1);
+    else if (F == 1024 && rp == 2) SMOE_MM_DOWN(4, 2);
+    else if (F == 1024) SMOE_MM_DOWN(4, 1);
+    else SMOE_MM_DOWN(8, 1);
 #undef SMOE_MM_DOWN
     return hipGetLastError();
 }

@@ -50,3 +50,16 @@ def test_forward_iq2_s_batches(torch, case):  # noqa: F811
     assert np.array_equal(bits(got), bits(want)), f"max rel {O.rel_l1_rows(got, want).max()}"
     y2, _ = ml.forward(dev(torch, x), add_shared=add_shared, trace=True, stages=True)
     assert np.array_equal(bits(host(torch, y2)), bits(want))
+
+
+@pytest.mark.parametrize("n_embd, n_ff", [(2048, 512), (2048, 1024)])
+def test_iq2_s_down_passes(torch, n_embd, n_ff):  # noqa: F811
+    """Enough items for the down kernel's two passes of 256 rows: the row kernels' bits (those of a traced call)."""
+    g = S.Geom(w_type=22, sh_type=22, n_embd=n_embd, n_ff=n_ff, n_ff_shared=n_ff, n_expert=512, top_k=10)
+    T = 311
+    print(f"case: IQ2_S down passes H={n_embd} F={n_ff} T={T}", flush=True)
+    ml = S.MoELayer(g, S.synth_layer(g, 7), max_tokens=T)
+    x = dev(torch, O.gen_normal(7, 100, T * n_embd).reshape(T, n_embd))
+    y = ml.forward(x)
+    y2, _ = ml.forward(x, trace=True, stages=True)
+    assert np.array_equal(bits(host(torch, y)), bits(host(torch, y2)))
