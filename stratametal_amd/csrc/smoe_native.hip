@@ -510,11 +510,12 @@ __global__ __launch_bounds__(256) void k_mmvq_native_cols(const uint8_t* __restr
 // per 32 values, or per 256) that fp16 holds exactly, as it holds q8_1's: a 32-value dot is then exact in f32 and only
 // fma(d_w d_x, dot, sum) rounds, once per 32 values (d_w d_x is exact: two fp16 values).  k_mmvq_native_cols spends 9 to
 // 22 VALU instructions per 16 products on the row kernels' order of partials, which a prompt's contract does not ask for.
-// A work-group takes 64 rows (16 per wave) by 32 columns, 256 values of K at a time through LDS as fp16; the sums run
-// 4 + 4 blocks, two chunks, then in order: short chains, for an error no larger than the row kernels'.  A word's four
-// values lie in the order 0, 2, 1, 3 on both sides.  1000 columns, gate and up of Q3_K 512 x 2048 and down of IQ4_NL
-// 2048 x 512: 124 and 37 us on the row kernels, 32 and 17 here; bound by the latency of a chunk's loads.
-constexpr int kNmRows = 64, kNmCols = 32, kNmPitch = 256 * 2 + 16;  // (the pad spreads 16 rows over the banks)
+// A work-group takes 64 rows (16 per wave) or 32 (16 rows by 16 columns per wave) by 32 columns, 256 values of K at a time
+// through LDS as fp16; the sums run 4 + 4 blocks, two chunks, then in order: short chains, for an error no larger than the
+// row kernels'.  A word's four values lie in the order 0, 2, 1, 3 on both sides.  1000 columns, gate and up of Q3_K
+// 512 x 2048 and down of IQ4_NL 2048 x 512: 124 and 37 us on the row kernels, 32 and 17 here; bound by the latency of a
+// chunk's loads.
+constexpr int kNmCols = 32, kNmPitch = 256 * 2 + 16;  // (the pad spreads 16 rows over the banks)
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -533,8 +534,8 @@ __device__ __forceinline__ uint2 word_bits(int32_t w) {
     return make_uint2(__builtin_bit_cast(uint32_t, o[0]), __builtin_bit_cast(uint32_t, o[1]));
 }
 
-// Partial k of a row's 256-value chunk into its fp16 row and its blocks' scales (dw: [8][kNmRows]).
-template <int TYPE>
+// Partial k of a row's 256-value chunk into its fp16 row and its blocks' scales (dw: [8][ROWS]).
+template <int TYPE, int ROWS>
 __device__ __forceinline__ void nm_put(const NativePart<TYPE>& p, int k, uint8_t* wrow, float* dw) {
     if constexpr (TYPE == 8) {
 #pragma unroll
@@ -542,7 +543,7 @@ __device__ __forceinline__ void nm_put(const NativePart<TYPE>& p, int k, uint8_t
             const uint2 a = word_bits(p.w[2 * j]), b = word_bits(p.w[2 * j + 1]);
             *reinterpret_cast<u32x4*>(wrow + 64 * k + 16 * j) = u32x4{a.x, a.y, b.x, b.y};
         }
-        dw[k * kNmRows] = p.d;
+        dw[k * ROWS] = p.d;
     } else if constexpr (TYPE == 11) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -553,40 +554,43 @@ __device__ __forceinline__ void nm_put(const NativePart<TYPE>& p, int k, uint8_t
             *reinterpret_cast<uint2*>(wrow + 64 * (4 * (k / 8) + i) + 8 * (k % 8)) =
                 make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
         }
-        if (k % 2 == 0) dw[k / 2 * kNmRows] = p.d;
+        if (k % 2 == 0) dw[k / 2 * ROWS] = p.d;
     } else {
         const int kb = k >> 1, iqs = 2 * (k & 1);
         const uint2 l0 = word_bits(p.lo[0]), l1 = word_bits(p.lo[1]), h0 = word_bits(p.hi[0]), h1 = word_bits(p.hi[1]);
         *reinterpret_cast<u32x4*>(wrow + 64 * kb + 8 * iqs) = u32x4{l0.x, l0.y, l1.x, l1.y};
         *reinterpret_cast<u32x4*>(wrow + 64 * kb + 8 * iqs + 32) = u32x4{h0.x, h0.y, h1.x, h1.y};
-        if (iqs == 0) dw[kb * kNmRows] = p.d;
+        if (iqs == 0) dw[kb * ROWS] = p.d;
     }
 }
 
-template <int TYPE>
+template <int TYPE, int ROWS>
 __global__ __launch_bounds__(256) void k_native_mm(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2, int n_in,
                                                    int n_out, int n_col, const uint8_t* __restrict__ xq,
                                                    float* __restrict__ y, float* __restrict__ y2, int ldy,
                                                    const float* __restrict__ sg) {
     using NT = NativeType<TYPE>;
     constexpr int NP = 256 / NT::qk * NT::ipb;  // partials of a row's chunk
-    constexpr int U = kNmRows * NP / 256;       // per thread
+    constexpr int U = ROWS * NP / 256;          // per thread
+    constexpr int CT = ROWS / 32;               // column tiles per wave
+    static_assert(ROWS == 64 || ROWS == 32, "four waves over the tile");
     static_assert(NP == 8 || NP == 16, "whole partials per thread");
-    __shared__ __align__(16) uint8_t ws[kNmRows * kNmPitch];
+    __shared__ __align__(16) uint8_t ws[ROWS * kNmPitch];
     __shared__ __align__(16) uint8_t xs[kNmCols * kNmPitch];
-    __shared__ __align__(16) float dw[8 * kNmRows];
+    __shared__ __align__(16) float dw[8 * ROWS];
     __shared__ float dx[8][kNmCols];
     if (blockIdx.z) {
         w = w2;
         y = y2;
     }
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, i = lane & 15, q = lane >> 4;
-    const int r0 = blockIdx.x * kNmRows, c0 = blockIdx.y * kNmCols;
+    const int r0 = blockIdx.x * ROWS, c0 = blockIdx.y * kNmCols;
     const size_t rb = (size_t)(n_in / NT::qk) * NT::bytes;
     const uint32_t* xd = reinterpret_cast<const uint32_t*>(xq) + (size_t)min(c0 + (tid >> 3), n_col - 1) * (n_in / 32 * 9);
-    f32x4 tot[2], hold[2];
+    const int wr = ROWS == 64 ? 16 * wave : 16 * (wave & 1), wc = ROWS == 64 ? 0 : 16 * (wave >> 1);
+    f32x4 tot[CT], hold[CT];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) tot[b] = hold[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int b = 0; b < CT; ++b) tot[b] = hold[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     for (int v0 = 0, ph = 0; v0 < n_in; v0 += 256, ph ^= 1) {
         const int nb = min(8, (n_in - v0) / 32);  // 32-value blocks of this chunk
         const int np = nb * 32 / NT::qk * NT::ipb;
@@ -615,26 +619,26 @@ __global__ __launch_bounds__(256) void k_native_mm(const uint8_t* __restrict__ w
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int p = tid + 256 * u, row = p / NP;
-            nm_put<TYPE>(part[u], p % NP, ws + row * kNmPitch, dw + row);
+            nm_put<TYPE, ROWS>(part[u], p % NP, ws + row * kNmPitch, dw + row);
         }
         __syncthreads();
-        f32x4 half[2][2];
+        f32x4 half[2][CT];
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b) half[hf][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int b = 0; b < CT; ++b) half[hf][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int blk = 4 * hf + j;
                 if (blk >= nb) break;  // (uniform)
                 const f16x8 a = __builtin_bit_cast(
-                    f16x8, *reinterpret_cast<const u32x4*>(ws + (16 * wave + i) * kNmPitch + 64 * blk + 16 * q));
-                const f32x4 d = *reinterpret_cast<const f32x4*>(dw + blk * kNmRows + 16 * wave + 4 * q);
+                    f16x8, *reinterpret_cast<const u32x4*>(ws + (wr + i) * kNmPitch + 64 * blk + 16 * q));
+                const f32x4 d = *reinterpret_cast<const f32x4*>(dw + blk * ROWS + wr + 4 * q);
 #pragma unroll
-                for (int b = 0; b < 2; ++b) {
+                for (int b = 0; b < CT; ++b) {
                     const f16x8 x = __builtin_bit_cast(
-                        f16x8, *reinterpret_cast<const u32x4*>(xs + (16 * b + i) * kNmPitch + 64 * blk + 16 * q));
-                    const float xsc = dx[blk][16 * b + i];
+                        f16x8, *reinterpret_cast<const u32x4*>(xs + (wc + 16 * b + i) * kNmPitch + 64 * blk + 16 * q));
+                    const float xsc = dx[blk][wc + 16 * b + i];
                     const f32x4 S =
                         __builtin_amdgcn_mfma_f32_16x16x32_f16(a, x, f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 #pragma unroll
@@ -643,7 +647,7 @@ __global__ __launch_bounds__(256) void k_native_mm(const uint8_t* __restrict__ w
             }
         }
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int b = 0; b < CT; ++b)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float v = half[0][b][e] + half[1][b][e];
@@ -656,10 +660,10 @@ __global__ __launch_bounds__(256) void k_native_mm(const uint8_t* __restrict__ w
             }
     }
     // lane (q, i) holds rows 4 q .. + 3 of column i of each tile
-    const int r = r0 + 16 * wave + 4 * q;
+    const int r = r0 + wr + 4 * q;
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-        const int c = c0 + 16 * b + i;
+    for (int b = 0; b < CT; ++b) {
+        const int c = c0 + wc + 16 * b + i;
         if (c >= n_col || r >= n_out) continue;
         const float g = sg ? sigmoid(sg[c]) : 1.0f;
         f32x4 v;
@@ -779,8 +783,16 @@ hipError_t launch_native_mm(int type, const uint8_t* w, const uint8_t* xq, int n
     const int cg = (n_col + kNmCols - 1) / kNmCols;
     if (!native_mm_ok(type, n_out) || native_row_bytes(type, n_in) <= 0 || n_col < 1 || cg > 65535 || ldy % 4 || (al & 15))
         return hipErrorInvalidValue;
-    const dim3 grid((unsigned)((n_out + kNmRows - 1) / kNmRows), (unsigned)cg, w2 ? 2 : 1);
-#define SMOE_NM(T) hipLaunchKernelGGL((k_native_mm<T>), grid, dim3(256), 0, s, w, w2, n_in, n_out, n_col, xq, y, y2, ldy, sg)
+    // 32 rows while 64 leave no second work-group per CU (the layer call at 128, 400 and 900 tokens: 221, 289 and 439 us
+    // in 32 rows, 227, 290 and 427 in 64)
+    const unsigned nz = w2 ? 2 : 1;
+    const int rows = (int64_t)((n_out + 63) / 64) * cg * nz <= 256 ? 32 : 64;
+    const dim3 grid((unsigned)((n_out + rows - 1) / rows), (unsigned)cg, nz);
+#define SMOE_NMR(T, R) \
+    hipLaunchKernelGGL((k_native_mm<T, R>), grid, dim3(256), 0, s, w, w2, n_in, n_out, n_col, xq, y, y2, ldy, sg)
+#define SMOE_NM(T)                        \
+    if (rows == 32) SMOE_NMR(T, 32);      \
+    else SMOE_NMR(T, 64)
     switch (type) {
         case 8: SMOE_NM(8); break;
         case 2: SMOE_NM(2); break;
@@ -789,6 +801,7 @@ hipError_t launch_native_mm(int type, const uint8_t* w, const uint8_t* xq, int n
         default: SMOE_NM(11); break;
     }
 #undef SMOE_NM
+#undef SMOE_NMR
     return hipGetLastError();
 }
 

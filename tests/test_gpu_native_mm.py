@@ -14,12 +14,13 @@ from test_gpu_native import dev, native_layer, say, torch  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # H, F, gate, up, down, T: column tiles of 32 and row tiles of 64 with remainders, an odd chunk count, a short chunk
+    # H, F, gate, up, down, T: column tiles of 32 and row tiles of 32 with remainders, an odd chunk count, a short chunk
     (2048, 512, O.Q3_K, O.Q3_K, O.IQ4_NL, 160),
     (2560, 640, O.Q3_K, O.Q3_K, O.IQ4_NL, 129),  # down: two chunks and a half
     (1024, 384, O.Q8_0, O.Q8_0, O.Q8_0, 33),     # down: a chunk and a half
     (1280, 512, O.Q4_0, O.Q4_0, O.Q5_0, 31),     # gate/up: five chunks
     (640, 128, O.Q5_0, O.IQ4_NL, O.Q4_0, 1),     # gate and up apart; down: half a chunk
+    (2048, 512, O.Q8_0, O.Q8_0, O.Q4_0, 545),    # row tiles of 64: more than 256 work-groups
     (1536, 768, O.Q4_K, O.Q8_0, O.Q3_K, 64),     # one projection keeps the row kernels
 ]
 
