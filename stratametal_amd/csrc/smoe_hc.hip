@@ -15,6 +15,7 @@
 #include "smoe_device.hpp"
 #include "smoe_gemv.hpp"
 #include "smoe_launch.hpp"
+#include "smoe_rules.hpp"
 
 #include <type_traits>
 
@@ -50,15 +51,25 @@ __device__ __forceinline__ void stream_scales(const float (&v)[HC][NM], int hc, 
     __syncthreads();
 }
 
+// A token's streams (or the norm's rows) in a thread's slots; those past hc or n hold the last ones' values.
+template <int HC, int NM>
+__device__ __forceinline__ void stream_slots(const float* __restrict__ rows, int n, int hc, float (&v)[HC][NM]) {
+#pragma unroll
+    for (int c = 0; c < HC; ++c)
+#pragma unroll
+        for (int m = 0; m < NM; ++m) v[c][m] = rows[min(c, hc - 1) * n + min((int)threadIdx.x + 256 * m, n - 1)];
+}
+
 }  // namespace
 
 // k_hc_proj: grid (ceil((hc_lr + hc) / 4), T), 256 threads; block (b, t) takes rows 4b .. 4b + 3 of [down; inj] for
 // token t, one row per wave (lane l adds the 8-element chunks l, l + 64, ... in element order, then the xor butterfly
 // 32..1, as the router).  Every block forms the token's scales and stages act = bf16((R * rs) * w_norm) in LDS; block
 // (0, t) also writes rs[t][c] for k_hc_mix.  Bound by latency at one token (81 work-groups): every load it needs (its
-// streams, norm and weight row) is issued up front, unconditionally (indices clamped into the row), so that one memory
-// round trip covers them all (with the loads under their bounds' branches 13.1 us, of which the bytes take 1.2).
-template <int HC, int NM, int MAXC>
+// streams, norm and weight row) is issued up front, unconditionally, so that one memory round trip covers them all
+// (with the loads under their bounds' branches 13.1 us, of which the bytes take 1.2).  AHEAD: the norm among them
+// (hc_norm_ahead).
+template <int HC, int NM, int MAXC, bool AHEAD>
 __global__ __launch_bounds__(256) void k_hc_proj(const float* __restrict__ R, const float* __restrict__ norm,
                                                   const uint16_t* __restrict__ down, const uint16_t* __restrict__ inj,
                                                   int n, int hc, int hc_lr, float eps, float* __restrict__ proj,
@@ -75,14 +86,8 @@ __global__ __launch_bounds__(256) void k_hc_proj(const float* __restrict__ R, co
     const float* Rt = R + (size_t)t * hd;
     float v[HC][NM], nv[HC][NM];
     uint4 wv[MAXC];
-#pragma unroll
-    for (int c = 0; c < HC; ++c)
-#pragma unroll
-        for (int m = 0; m < NM; ++m) v[c][m] = Rt[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
-#pragma unroll
-    for (int c = 0; c < HC; ++c)
-#pragma unroll
-        for (int m = 0; m < NM; ++m) nv[c][m] = norm[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
+    stream_slots<HC, NM>(Rt, n, hc, v);
+    if constexpr (AHEAD) stream_slots<HC, NM>(norm, n, hc, nv);
 #pragma unroll
     for (int j = 0; j < MAXC; ++j) wv[j] = *reinterpret_cast<const uint4*>(wr + 8 * min(lane + 64 * j, chunks - 1));
     __builtin_amdgcn_sched_barrier(0);
@@ -93,7 +98,9 @@ __global__ __launch_bounds__(256) void k_hc_proj(const float* __restrict__ R, co
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             const int d = tid + 256 * m;
-            if (c < hc && d < n) act_s[c * n + d] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * nv[c][m]);
+            if (c >= hc || d >= n) continue;
+            const float w = AHEAD ? nv[c][m] : norm[c * n + d];
+            act_s[c * n + d] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * w);
         }
     }
     __syncthreads();
@@ -243,14 +250,8 @@ __global__ __launch_bounds__(256) void k_hc_act(const float* __restrict__ R, con
     const int hd = hc * n;
     const float* Rt = R + (size_t)t * hd;
     float v[HC][NM], nv[HC][NM];
-#pragma unroll
-    for (int c = 0; c < HC; ++c)
-#pragma unroll
-        for (int m = 0; m < NM; ++m) v[c][m] = Rt[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
-#pragma unroll
-    for (int c = 0; c < HC; ++c)
-#pragma unroll
-        for (int m = 0; m < NM; ++m) nv[c][m] = norm[min(c, hc - 1) * n + min(tid + 256 * m, n - 1)];
+    stream_slots<HC, NM>(Rt, n, hc, v);
+    if constexpr (hc_norm_fits(HC * NM, 0)) stream_slots<HC, NM>(norm, n, hc, nv);
     __builtin_amdgcn_sched_barrier(0);
     stream_scales<HC, NM>(v, hc, n, eps, wsum, rs_s);
     if (tid < hc) rs_out[(size_t)t * hc + tid] = rs_s[tid];
@@ -259,7 +260,9 @@ __global__ __launch_bounds__(256) void k_hc_act(const float* __restrict__ R, con
 #pragma unroll
         for (int m = 0; m < NM; ++m) {
             const int d = tid + 256 * m;
-            if (c < hc && d < n) act_s[c * n + d] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * nv[c][m]);
+            if (c >= hc || d >= n) continue;
+            const float w = hc_norm_fits(HC * NM, 0) ? nv[c][m] : norm[c * n + d];
+            act_s[c * n + d] = (uint16_t)f32_to_bf16((v[c][m] * rs_s[c]) * w);
         }
     __syncthreads();
     u32x4* dst = reinterpret_cast<u32x4*>(act + (size_t)t * hd);
@@ -483,6 +486,29 @@ __global__ __launch_bounds__(256) void k_hc_mix_mm(const float* __restrict__ R, 
     }
 }
 
+// go(HC, NM) with the slots of hc streams of n values
+template <int V>
+using Int = std::integral_constant<int, V>;
+template <class Go>
+static void hc_slots(int n, int hc, Go go) {
+    auto values = [&](auto HC) {
+        switch (hc_values(n)) {
+            case 2: go(HC, Int<2>{}); break;
+            case 4: go(HC, Int<4>{}); break;
+            case 6: go(HC, Int<6>{}); break;
+            case 8: go(HC, Int<8>{}); break;
+            case 10: go(HC, Int<10>{}); break;
+            case 12: go(HC, Int<12>{}); break;
+            default: go(HC, Int<16>{}); break;
+        }
+    };
+    switch (hc_streams(hc)) {
+        case 2: values(Int<2>{}); break;
+        case 4: values(Int<4>{}); break;
+        default: values(Int<8>{}); break;
+    }
+}
+
 // From how many tokens the read runs on the matrix cores: from 17 tokens (a second 16-token tile) and 2^23 products of
 // the projection, where its four launches cost what the two of the row-per-wave kernels do (hc 2, hc_lr 64, n 2048: 16.3
 // us row-per-wave and 17.3 on the matrix cores at 32 tokens, 23.1 and 20.1 at 64; hc 4, hc_lr 320: 44.6 and 32.7 at 17
@@ -518,20 +544,11 @@ hipError_t launch_hc_read_mm(const float* R, const float* norm, const uint16_t* 
                              const uint16_t* inj, int T, int n, int hc, int hc_lr, float eps, float* rs, uint16_t* act,
                              float* part, uint16_t* lq, float* mixed, float* inject, hipStream_t s) {
     if (!hc_mm_shape(T, n, hc, hc_lr)) return hipErrorInvalidValue;
-    const int hd = hc * n, nm = (n + 255) / 256, rows = hc_lr + hc, ld = hc_ld(hc_lr, hc), kp = hc_kp(hc_lr);
+    const int hd = hc * n, rows = hc_lr + hc, ld = hc_ld(hc_lr, hc), kp = hc_kp(hc_lr);
     const size_t lds = (size_t)hd * 2;
-#define SMOE_HCA(HCv, NMv) \
-    hipLaunchKernelGGL((k_hc_act<HCv, NMv>), dim3((unsigned)T), dim3(256), lds, s, R, norm, n, hc, eps, act, rs)
-    if (hc <= 4) {
-        if (nm <= 2) SMOE_HCA(4, 2);
-        else if (nm <= 8) SMOE_HCA(4, 8);
-        else SMOE_HCA(4, 16);
-    } else {
-        if (nm <= 2) SMOE_HCA(8, 2);
-        else if (nm <= 8) SMOE_HCA(8, 8);
-        else SMOE_HCA(8, 16);
-    }
-#undef SMOE_HCA
+    hc_slots(n, hc, [&](auto HC, auto NM) {
+        hipLaunchKernelGGL((k_hc_act<HC(), NM()>), dim3((unsigned)T), dim3(256), lds, s, R, norm, n, hc, eps, act, rs);
+    });
     const int n_tb = (T + kHpTok - 1) / kHpTok, n_rb = (rows + kHpRows - 1) / kHpRows, chunks = hd / kHpK;
     int splits = hc_splits(n_tb * n_rb, chunks);
     const int per = (chunks + splits - 1) / splits;
@@ -570,27 +587,27 @@ hipError_t launch_hc_read(const float* R, const float* norm, const uint16_t* dow
                           float* inject, hipStream_t s) {
     if (!hc_shape_ok(n, hc, hc_lr) || n_tok <= 0) return hipErrorInvalidValue;
     const int hd = hc * n;
-    const int maxc = (hd / 8 + 63) / 64;
-    const int nm = (n + 255) / 256;
     dim3 g1((unsigned)((hc_lr + hc + 3) / 4), (unsigned)n_tok);
     const size_t lds = (size_t)hd * 2;
-#define SMOE_HCP(HCv, NMv, C)                                                                                       \
-    hipLaunchKernelGGL((k_hc_proj<HCv, NMv, C>), g1, dim3(256), lds, s, R, norm, down, inj, n, hc, hc_lr, eps, proj, \
-                       inject, rs)
-#define SMOE_HCP_C(HCv, NMv)             \
-    if (maxc <= 8) SMOE_HCP(HCv, NMv, 8);  \
-    else if (maxc <= 16) SMOE_HCP(HCv, NMv, 16); \
-    else if (maxc <= 24) SMOE_HCP(HCv, NMv, 24); \
-    else SMOE_HCP(HCv, NMv, 32);
-#define SMOE_HCP_NM(HCv)                 \
-    if (nm <= 2) { SMOE_HCP_C(HCv, 2) }  \
-    else if (nm <= 8) { SMOE_HCP_C(HCv, 8) } \
-    else { SMOE_HCP_C(HCv, 16) }
-    if (hc <= 4) { SMOE_HCP_NM(4) }
-    else { SMOE_HCP_NM(8) }
-#undef SMOE_HCP_NM
-#undef SMOE_HCP_C
-#undef SMOE_HCP
+    hc_slots(n, hc, [&](auto HC, auto NM) {
+        constexpr int slots = HC() * NM();  // a row is at most slots / 2 pieces per lane
+        auto go = [&](auto C) {
+            constexpr int more = 4 * C();
+            const auto k = hc_norm_ahead(slots, more, (int64_t)g1.x * g1.y, (int64_t)hc_lr * hd * 2)
+                               ? k_hc_proj<HC(), NM(), C(), true>
+                               : k_hc_proj<HC(), NM(), C(), hc_norm_fits(slots, more) || (slots + more > 192)>;
+            hipLaunchKernelGGL(k, g1, dim3(256), lds, s, R, norm, down, inj, n, hc, hc_lr, eps, proj, inject, rs);
+        };
+        const int chunks = hc_chunks(n, hc);
+        if (chunks == 8) go(Int<8>{});
+        else if constexpr (slots > 16) {
+            if (chunks == 16) go(Int<16>{});
+            else if constexpr (slots > 32) {
+                if (chunks == 24) go(Int<24>{});
+                else go(Int<32>{});
+            }
+        }
+    });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const int lqc = (hc_lr / 8 + 7) / 8;  // chunks per lane of an up row

@@ -1,0 +1,39 @@
+// stratametal_amd/csrc/smoe_rules.hpp - which kernel a call runs on, where the choice was measured: plain host functions
+// of a call's sizes, so that a CPU test can hold them to the times they come from (tests/test_dispatch_rules.py).
+#pragma once
+
+#include <cstdint>
+
+namespace smoe {
+
+// The register slots of a token's streams in k_hc_proj and k_hc_act: HC streams of NM values per thread.  Every slot is
+// loaded (the indices clamped into the row), so a spare one is a load too: the least that hold hc streams of n values
+// (with 4 and 8 streams of 2, 8 and 16 alone the read of 16 tokens, hc 1, n 1024, hc_lr 320, took 14.0 us, with branches
+// around the loads 13.4, so 10.1).
+constexpr int kHcStreams[] = {2, 4, 8}, kHcValues[] = {2, 4, 6, 8, 10, 12, 16};
+constexpr int hc_streams(int hc) {
+    for (const int s : kHcStreams)
+        if (hc <= s) return s;
+    return 8;
+}
+constexpr int hc_values(int n) {
+    for (const int v : kHcValues)
+        if (n <= 256 * v) return v;
+    return 16;
+}
+// 16-byte pieces of a weight row per lane: hc n / 512 rounded up to eighths.
+constexpr int hc_chunks(int n, int hc) { return (hc * n / 8 + 511) / 512 * 8; }
+
+// The norm's slots are loaded with the streams' (one memory round trip less: 2 us of 13 at one token, n 2560, hc 4)
+// where both fit 256 registers beside the weight row's `more`, two waves per SIMD.
+constexpr bool hc_norm_fits(int slots, int more) { return 2 * slots + more <= 192; }
+// Where they don't, the norm is loaded with the streams by one wave per SIMD or, where the streams and the weight row
+// alone fit, after the scales are formed by two: by two where that halves the rounds of work-groups over the 256 CUs
+// and an XCD's L2 holds the weights (n 2048, hc 6, hc_lr 64: 16 tokens, 288 work-groups, 26.7 us in two rounds of one
+// wave, 21.7 in one of two waves; 14 tokens, 252, 17.6 against 20.2; hc 8, hc_lr 320: 4 tokens, 328, 32.3 against 34.3).
+constexpr bool hc_norm_ahead(int slots, int more, int64_t groups, int64_t weight_bytes) {
+    return hc_norm_fits(slots, more) || slots + more > 192 || (groups + 255) / 256 % 2 == 1 ||
+           weight_bytes > (int64_t)5 << 20;
+}
+
+}  // namespace smoe

@@ -1,0 +1,51 @@
+"""The dispatch rules of stratametal_amd/csrc/smoe_rules.hpp at the sizes whose both sides were measured (the figures
+stand beside the rules): host functions, compiled here and asked for their choice."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CXX = shutil.which("g++") or shutil.which("c++")
+pytestmark = pytest.mark.skipif(CXX is None, reason="no host compiler")
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    """ask(expressions): their values, as whole numbers."""
+    d = tmp_path_factory.mktemp("rules")
+
+    def run(exprs):
+        src, exe = str(d / "rules.cpp"), str(d / "rules")
+        body = "".join(f'    std::printf("%lld\\n", (long long)({e}));\n' for e in exprs)
+        with open(src, "w") as f:
+            f.write('#include <cstdio>\n#include "smoe_rules.hpp"\nusing namespace smoe;\nint main() {\n' + body + "}\n")
+        subprocess.run([CXX, "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "stratametal_amd", "csrc"), src, "-o",
+                        exe], check=True, capture_output=True, text=True)
+        out = subprocess.run([exe], check=True, capture_output=True, text=True).stdout.split()
+        return [int(v) for v in out]
+    return run
+
+
+def test_hc_slots(ask):
+    """The read's slots hold the streams with few to spare: each is loaded."""
+    shapes = [(n, hc) for n in range(8, 4097, 8) for hc in range(1, 9) if hc * n <= 16384]
+    got = ask([e for n, hc in shapes for e in (f"hc_streams({hc})", f"hc_values({n})", f"hc_chunks({n}, {hc})")])
+    for i, (n, hc) in enumerate(shapes):
+        s, v, c = got[3 * i:3 * i + 3]
+        need = (n + 255) // 256
+        assert s >= hc and v >= need, (n, hc)
+        assert s < 2 * hc or s == 2, (n, hc)  # fewer spare streams than streams (a second one beside a single one)
+        assert v - need <= max(1, need // 4) or need == 1, (n, hc)
+        assert 512 * c >= hc * n >= 0 and c - hc * n / 512 <= 8 and c in (8, 16, 24, 32), (n, hc)
+        assert c <= (8 if s * v <= 16 else 16 if s * v <= 32 else 32), (n, hc)  # the kernels that exist
+
+
+def test_hc_norm(ask):
+    """Two waves per SIMD where they halve the rounds: hc, n, hc_lr, tokens -> the norm with the streams."""
+    cases = [(4, 2048, 320, 1, 1), (4, 2048, 320, 16, 1), (4, 2560, 64, 16, 1), (6, 1536, 64, 16, 1), (6, 2048, 64, 14, 1),
+             (6, 2048, 64, 16, 0), (5, 2048, 200, 6, 0), (3, 4096, 64, 16, 0), (8, 2048, 320, 4, 1), (6, 2560, 64, 16, 1)]
+    got = ask([f"hc_norm_ahead(hc_streams({hc}) * hc_values({n}), 4 * hc_chunks({n}, {hc}), {(lr + hc + 3) // 4 * T}, "
+               f"{lr * hc * n * 2})" for hc, n, lr, T, _ in cases])
+    assert got == [c[-1] for c in cases]

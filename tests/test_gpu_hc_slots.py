@@ -1,0 +1,33 @@
+"""GPU parity of the hyper-connection read of few tokens (k_hc_proj) at every count of streams and values per thread that
+has registers of its own, and with the norm loaded after the scales, with the oracle's device order bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as O
+from test_gpu_hc import GUARD, bits, dev, hc_dev, host, say, streams, torch  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # n_embd, hc, hc_lr, T
+    (512, 1, 64, 2), (1016, 2, 8, 3), (1032, 1, 16, 2), (1536, 2, 24, 2), (2560, 2, 40, 1), (3072, 1, 8, 2), (4096, 2, 16, 1),
+    (264, 3, 8, 3), (768, 4, 64, 2), (1288, 4, 16, 2), (2304, 3, 24, 1), (2560, 4, 64, 16), (3000, 4, 8, 2), (4096, 3, 16, 2),
+    (256, 7, 8, 2), (1024, 5, 32, 2), (1536, 6, 64, 16), (2048, 5, 8, 2), (2560, 6, 16, 2), (3072, 5, 16, 1),
+    (2048, 6, 64, 16), (4096, 3, 64, 16), (2048, 8, 64, 15),  # the norm after the scales
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_hc_read_slots(torch, case):  # noqa: F811
+    n, hc, hc_lr, T = CASES[case]
+    say(f"case: hc_read slots n={n} hc={hc} hc_lr={hc_lr} T={T}")
+    w = O.make_hc(n, hc, hc_lr, 500 + case)
+    R = streams(500 + case, T, hc, n)
+    mg = torch.full((T * n + GUARD,), 7.0, dtype=torch.float32, device="cuda")
+    ig = torch.full((T * hc + GUARD,), 7.0, dtype=torch.float32, device="cuda")
+    hc_dev(torch, w, n).read(dev(torch, R), mixed=mg[:T * n], inject=ig[:T * hc])
+    m, i = host(torch, mg), host(torch, ig)
+    assert (m[T * n:] == 7.0).all() and (i[T * hc:] == 7.0).all(), "guard words written"
+    want_m, want_i = O.hc_read_dev(R, n, w)
+    assert np.array_equal(bits(m[:T * n].reshape(T, n)), bits(want_m))
+    assert np.array_equal(bits(i[:T * hc].reshape(T, hc)), bits(want_i))
