@@ -10,7 +10,7 @@
 // For few tokens the read is two bandwidth-bound bf16 GEMVs in a chain (about 10.5 MB of weights per call at n 2048,
 // hc 4, hc_lr 320, as much as the MoE block itself), so it is two launches: k_hc_proj (the norm, the activations staged
 // in LDS, the down and inject rows) and k_hc_mix (lq, the up rows, the gated mean).  Their reduction orders are fixed
-// and restated by the test oracle (or_hc_read_dev, or_hc_write_dev).  For a batch of tokens (kHcMmTokens) both products
+// and restated by the test oracle (or_hc_read_dev, or_hc_write_dev).  For a batch of tokens (hc_mm_gains) both products
 // run on the matrix cores: k_hc_act, k_hc_proj_mm, k_hc_lq, k_hc_mix_mm.
 #include "smoe_device.hpp"
 #include "smoe_gemv.hpp"
@@ -509,13 +509,8 @@ static void hc_slots(int n, int hc, Go go) {
     }
 }
 
-// From how many tokens the read runs on the matrix cores: from 17 tokens (a second 16-token tile) and 2^23 products of
-// the projection, where its four launches cost what the two of the row-per-wave kernels do (hc 2, hc_lr 64, n 2048: 16.3
-// us row-per-wave and 17.3 on the matrix cores at 32 tokens, 23.1 and 20.1 at 64; hc 4, hc_lr 320: 44.6 and 32.7 at 17
-// tokens, 140 and 37 at 64, 1965 and 66 at 1000).  The shapes that do: whole 64-value chunks of a stream and an lq tile
+// The shapes that run on the matrix cores where hc_mm_gains says so: whole 64-value chunks of a stream and an lq tile
 // within 64 KiB of LDS; others keep the row-per-wave kernels.
-constexpr int kHcMmTokens = 17;
-constexpr int64_t kHcMmProducts = (int64_t)1 << 23;
 constexpr int kHcMmMaxLr = 960;
 static int hc_kp(int hc_lr) { return (hc_lr + 63) / 64 * 64; }
 static int hc_ld(int hc_lr, int hc) { return (hc_lr + hc + 3) / 4 * 4; }
@@ -528,8 +523,7 @@ static int hc_splits(int tiles, int chunks) {
 }
 
 bool hc_mm_shape(int64_t T, int n, int hc, int hc_lr) {
-    return T >= kHcMmTokens && hc_shape_ok(n, hc, hc_lr) && T * hc * n * hc_lr >= kHcMmProducts && n % 64 == 0 &&
-           hc_lr <= kHcMmMaxLr;
+    return hc_shape_ok(n, hc, hc_lr) && hc_mm_gains(T, n, hc, hc_lr) && n % 64 == 0 && hc_lr <= kHcMmMaxLr;
 }
 // The scratch of the matrix-core read (act, the K slices' sums, lq), growing with T: part is bounded by the slices'
 // largest count for few tokens, by the launch's work-groups' tiles, or by one slice.

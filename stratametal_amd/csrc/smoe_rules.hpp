@@ -36,4 +36,15 @@ constexpr bool hc_norm_ahead(int slots, int more, int64_t groups, int64_t weight
            weight_bytes > (int64_t)5 << 20;
 }
 
+// Whether the read of a batch runs on the matrix cores: from 17 tokens (a second 16-token tile) and 2^23 products of the
+// projection, where the row-per-wave kernels' time, which grows with the tokens, has passed the four launches', which
+// hardly does but grows with the streams and hc_lr.  Fitted to 60 shapes of 8 to 400 tokens; rows and matrix cores, us:
+// hc 4, hc_lr 320, n 2048 30 and 28 at 17 tokens, 82 and 31 at 64, 1965 and 66 at 1000; n 512 11 and 24 at 17, 24 and 26
+// at 64, 38 and 28 at 128; hc 8, n 256 45 and 36 at 128; hc 4, hc_lr 64, n 2048 17 and 20 at 24, 32 and 21 at 64; hc 1,
+// hc_lr 960, n 4096 114 and 35 at 17.
+constexpr bool hc_mm_gains(int64_t T, int n, int hc, int hc_lr) {
+    return T >= 17 && T * hc * n * hc_lr >= (int64_t)1 << 23 &&
+           120 * T * n * (hc * (hc_lr + 80) + hc_lr + 160) >= (int64_t)92 * 32768 * (960 + 360 * hc + hc_lr);
+}
+
 }  // namespace smoe

@@ -49,3 +49,19 @@ def test_hc_norm(ask):
     got = ask([f"hc_norm_ahead(hc_streams({hc}) * hc_values({n}), 4 * hc_chunks({n}, {hc}), {(lr + hc + 3) // 4 * T}, "
                f"{lr * hc * n * 2})" for hc, n, lr, T, _ in cases])
     assert got == [c[-1] for c in cases]
+
+
+def test_hc_matrix_cores(ask):
+    """n, hc, hc_lr, tokens: the faster of the row-per-wave kernels (0) and the matrix cores (1); more tokens never go
+    back (a workspace for more tokens holds every smaller call)."""
+    cases = [(2048, 4, 320, 16, 0), (2048, 4, 320, 17, 1), (2048, 4, 320, 1000, 1), (512, 4, 320, 17, 0), (512, 4, 320, 64, 0),
+             (512, 4, 320, 128, 1), (512, 2, 320, 32, 0), (512, 8, 320, 24, 0), (256, 8, 320, 64, 0), (256, 8, 320, 128, 1),
+             (512, 8, 960, 24, 0), (2048, 4, 64, 24, 0), (2048, 4, 64, 64, 1), (2048, 2, 200, 24, 0), (1536, 4, 64, 24, 0),
+             (2560, 2, 640, 17, 1), (4096, 1, 960, 17, 1), (4096, 4, 640, 17, 1), (1024, 8, 640, 24, 1)]
+    assert ask([f"hc_mm_gains({T}, {n}, {hc}, {lr})" for n, hc, lr, T, _ in cases]) == [c[-1] for c in cases]
+    shapes = [(n, hc, lr) for n in (64, 512, 2048, 4096) for hc in (1, 4, 8) for lr in (8, 320, 960)]
+    tokens = (1, 16, 17, 40, 64, 100, 1000, 4096, 65535)
+    got = ask([f"hc_mm_gains({T}, {n}, {hc}, {lr})" for n, hc, lr in shapes for T in tokens])
+    for i, s in enumerate(shapes):
+        g = got[i * len(tokens):(i + 1) * len(tokens)]
+        assert g == sorted(g), s
