@@ -604,11 +604,20 @@ hipError_t launch_hc_read(const float* R, const float* norm, const uint16_t* dow
     });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const int lqc = (hc_lr / 8 + 7) / 8;  // chunks per lane of an up row
     dim3 g2((unsigned)(n / 8), (unsigned)n_tok);
-    if (lqc <= 5) hipLaunchKernelGGL((k_hc_mix<5>), g2, dim3(256), 0, s, R, norm, up, proj, rs, n, hc, hc_lr, mixed);
-    else if (lqc <= 8) hipLaunchKernelGGL((k_hc_mix<8>), g2, dim3(256), 0, s, R, norm, up, proj, rs, n, hc, hc_lr, mixed);
-    else hipLaunchKernelGGL((k_hc_mix<32>), g2, dim3(256), 0, s, R, norm, up, proj, rs, n, hc, hc_lr, mixed);
+    auto mix = [&](auto P) {
+        hipLaunchKernelGGL((k_hc_mix<P()>), g2, dim3(256), 0, s, R, norm, up, proj, rs, n, hc, hc_lr, mixed);
+    };
+    switch (hc_pieces(hc_lr)) {
+        case 1: mix(Int<1>{}); break;
+        case 2: mix(Int<2>{}); break;
+        case 3: mix(Int<3>{}); break;
+        case 4: mix(Int<4>{}); break;
+        case 5: mix(Int<5>{}); break;
+        case 8: mix(Int<8>{}); break;
+        case 16: mix(Int<16>{}); break;
+        default: mix(Int<32>{}); break;
+    }
     return hipGetLastError();
 }
 

@@ -24,6 +24,15 @@ constexpr int hc_values(int n) {
 // 16-byte pieces of a weight row per lane: hc n / 512 rounded up to eighths.
 constexpr int hc_chunks(int n, int hc) { return (hc * n / 8 + 511) / 512 * 8; }
 
+// The same for the pieces of an `up` row per lane of k_hc_mix (hc_lr / 64 rounded up; five for one piece: the read of 64
+// tokens, hc 5, n 512, hc_lr 64, 14.5 us, with branches around the loads 13.7, with one 13.0).
+constexpr int kHcPieces[] = {1, 2, 3, 4, 5, 8, 16, 32};
+constexpr int hc_pieces(int hc_lr) {
+    for (const int p : kHcPieces)
+        if (hc_lr <= 64 * p) return p;
+    return 32;
+}
+
 // The norm's slots are loaded with the streams' (one memory round trip less: 2 us of 13 at one token, n 2560, hc 4)
 // where both fit 256 registers beside the weight row's `more`, two waves per SIMD.
 constexpr bool hc_norm_fits(int slots, int more) { return 2 * slots + more <= 192; }

@@ -42,6 +42,14 @@ def test_hc_slots(ask):
         assert c <= (8 if s * v <= 16 else 16 if s * v <= 32 else 32), (n, hc)  # the kernels that exist
 
 
+def test_hc_pieces(ask):
+    """The same for a row of the gate products: no piece to spare up to five, fewer than needed beyond."""
+    widths = list(range(8, 2049, 8))
+    for lr, p in zip(widths, ask([f"hc_pieces({lr})" for lr in widths])):
+        need = (lr + 63) // 64
+        assert p >= need and (p == need if need <= 5 else p < 2 * need), lr
+
+
 def test_hc_norm(ask):
     """Two waves per SIMD where they halve the rounds: hc, n, hc_lr, tokens -> the norm with the streams."""
     cases = [(4, 2048, 320, 1, 1), (4, 2048, 320, 16, 1), (4, 2560, 64, 16, 1), (6, 1536, 64, 16, 1), (6, 2048, 64, 14, 1),

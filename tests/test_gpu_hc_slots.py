@@ -1,5 +1,5 @@
-"""GPU parity of the hyper-connection read of few tokens (k_hc_proj) at every count of streams and values per thread that
-has registers of its own, and with the norm loaded after the scales, with the oracle's device order bit for bit."""
+"""GPU parity of the hyper-connection read of few tokens (k_hc_proj) at every count of streams, values per thread and
+pieces of a gate row that has registers of its own, and with the norm loaded after the scales, with the oracle's device order bit for bit."""
 import numpy as np
 import pytest
 
@@ -14,6 +14,7 @@ CASES = [
     (264, 3, 8, 3), (768, 4, 64, 2), (1288, 4, 16, 2), (2304, 3, 24, 1), (2560, 4, 64, 16), (3000, 4, 8, 2), (4096, 3, 16, 2),
     (256, 7, 8, 2), (1024, 5, 32, 2), (1536, 6, 64, 16), (2048, 5, 8, 2), (2560, 6, 16, 2), (3072, 5, 16, 1),
     (2048, 6, 64, 16), (4096, 3, 64, 16), (2048, 8, 64, 15),  # the norm after the scales
+    (64, 2, 72, 3), (64, 3, 128, 2), (64, 1, 184, 2), (64, 4, 256, 1), (64, 2, 520, 2), (64, 5, 1016, 2), (64, 2, 1032, 1),
 ]
 
 
