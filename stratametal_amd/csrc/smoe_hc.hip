@@ -211,9 +211,8 @@ __global__ __launch_bounds__(256) void k_hc_write(const float* R, const float* _
     out[i] = R[i] + y[t * n + d] * (2.0f * s);
 }
 
-// The same with R, y and out as 16-byte vectors (n % 4 == 0): block (p, t) takes 256 four-value pieces of y of token t
-// through every stream, so y is read once (few tokens: a block per stream).  hc 4, n 2048, a value per thread and this: 1000
-// tokens (73 MB) 20.9 and 11.5 us, 4096 tokens 99 and 48.
+// The same with R, y and out as 16-byte vectors (n % 4 == 0): block (p, c) takes 256 four-value pieces of y of a token
+// through stream c, or with one block in y through every stream, so y is read once (hc_write_kind).
 __global__ __launch_bounds__(256) void k_hc_write4(const float* R, const float* __restrict__ y,
                                                     const float* __restrict__ inject, int n4, int hc, int parts,
                                                     float* out) {
@@ -627,9 +626,10 @@ hipError_t launch_hc_write(const float* R, const float* y, const float* inject, 
     if (total <= 0) return hipErrorInvalidValue;
     const int parts = (n / 4 + 255) / 256;
     const uintptr_t al = reinterpret_cast<uintptr_t>(R) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(out);
-    if (n % 4 == 0 && (al & 15) == 0 && (int64_t)n_tok * parts <= INT32_MAX) {
-        hipLaunchKernelGGL(k_hc_write4, dim3((unsigned)((int64_t)n_tok * parts), n_tok < 64 ? (unsigned)hc : 1u), dim3(256), 0, s, R, y, inject, n / 4, hc,
-                           parts, out);
+    const HcWrite kind = hc_write_kind(n_tok, n, hc);
+    if (kind != kHcWriteValues && n % 4 == 0 && (al & 15) == 0 && (int64_t)n_tok * parts <= INT32_MAX) {
+        const dim3 grid((unsigned)((int64_t)n_tok * parts), kind == kHcWriteStream ? (unsigned)hc : 1u);
+        hipLaunchKernelGGL(k_hc_write4, grid, dim3(256), 0, s, R, y, inject, n / 4, hc, parts, out);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_hc_write, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, R, y, inject, n, hc, total,

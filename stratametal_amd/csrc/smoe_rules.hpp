@@ -56,4 +56,16 @@ constexpr bool hc_mm_gains(int64_t T, int n, int hc, int hc_lr) {
            120 * T * n * (hc * (hc_lr + 80) + hc_lr + 160) >= (int64_t)92 * 32768 * (960 + 360 * hc + hc_lr);
 }
 
+// The write of T tokens: kHcWriteValues a value per thread; else 16-byte vectors (n % 4 == 0 and aligned buffers), a
+// work-group's piece of y through one stream (kHcWriteStream) or through all (kHcWriteStreams: y read once, from where
+// the launch is long; rows of few values leave lanes idle in every piece, and one or two streams re-read little, so
+// earlier).  us by value, by stream and through all: hc 8, n 64, 200 tokens 2.5, 2.6, 3.5, 4000 tokens 7.3, 13.0, 6.5; hc 8,
+// n 512, 64 tokens 2.7, 2.5, 3.4; hc 4, n 2048, 64 tokens 3.3, 2.6, 2.9, 1000 tokens 21.5, 10.6, 11.6, 4000 tokens 98, 56, 44.
+enum HcWrite { kHcWriteValues, kHcWriteStream, kHcWriteStreams };
+constexpr HcWrite hc_write_kind(int64_t T, int n, int hc) {
+    const int64_t limit = n < 512 ? 15 << 16 : n < 768 ? 15 << 17 : hc <= 2 ? 6 << 20 : 11 << 20;
+    const bool all = T * hc * n >= limit;
+    return n < 64 || (n < 256 && !all) ? kHcWriteValues : all ? kHcWriteStreams : kHcWriteStream;
+}
+
 }  // namespace smoe

@@ -73,3 +73,10 @@ def test_hc_matrix_cores(ask):
     for i, s in enumerate(shapes):
         g = got[i * len(tokens):(i + 1) * len(tokens)]
         assert g == sorted(g), s
+
+
+def test_hc_write(ask):
+    """n, hc, tokens: a value per thread (0), vectors stream by stream (1), vectors through all streams (2)."""
+    cases = [(64, 8, 200, 0), (64, 8, 4000, 2), (72, 4, 64, 0), (32, 8, 4000, 0), (512, 8, 64, 1), (256, 8, 16, 1), (256, 8, 1000, 2),
+             (2048, 4, 1, 1), (2048, 4, 64, 1), (2048, 4, 1000, 1), (2048, 4, 4000, 2), (4096, 4, 1000, 2)]
+    assert ask([f"hc_write_kind({T}, {n}, {hc})" for n, hc, T, _ in cases]) == [c[-1] for c in cases]

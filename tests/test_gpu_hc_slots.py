@@ -32,3 +32,23 @@ def test_hc_read_slots(torch, case):  # noqa: F811
     want_m, want_i = O.hc_read_dev(R, n, w)
     assert np.array_equal(bits(m[:T * n].reshape(T, n)), bits(want_m))
     assert np.array_equal(bits(i[:T * hc].reshape(T, hc)), bits(want_i))
+
+
+@pytest.mark.parametrize("n,hc,T", [(60, 8, 30), (64, 8, 1919), (64, 8, 1920), (252, 3, 5), (256, 8, 3), (260, 5, 757), (512, 8, 64),
+                                    (1028, 2, 66), (1028, 2, 3061), (3000, 5, 769), (2048, 4, 3)])
+def test_hc_write_kinds(torch, n, hc, T):  # noqa: F811
+    """The write by values, by stream and through all streams, at the first batches of each and at rows whose last piece
+    is not full; and at streams that are not 16-byte aligned, by values."""
+    say(f"case: hc_write kinds n={n} hc={hc} T={T}")
+    R = streams(n, T, hc, n)
+    y = O.gen_normal(n, 51, T * n).reshape(T, n)
+    inj = (O.gen_normal(n, 52, T * hc) * 4.0).reshape(T, hc).astype(np.float32)
+    want = bits(O.hc_write_dev(R, y, inj, n, hc))
+    H = hc_dev(torch, O.make_hc(n, hc, 8, n), n)
+    og = torch.full((T * hc * n + GUARD,), 7.0, dtype=torch.float32, device="cuda")
+    for at in (0, 1):
+        og.fill_(7.0)
+        H.write(dev(torch, R), dev(torch, y), dev(torch, inj), out=og[at:at + T * hc * n])
+        got = host(torch, og)
+        assert (got[at + T * hc * n:] == 7.0).all() and (got[:at] == 7.0).all()
+        assert np.array_equal(bits(got[at:at + T * hc * n].reshape(T, hc, n)), want)
