@@ -13,6 +13,7 @@
 #include <string>
 
 #include "smoe_launch.hpp"
+#include "smoe_rules.hpp"
 
 namespace {
 
@@ -140,7 +141,9 @@ int max_items_mfma(const smoe_geom& g, int64_t T) {
     return (int)((P < g.n_expert ? P : g.n_expert) + P / C + (sh_fused(g) ? (T + C - 1) / C : 0));
 }
 // The IQ2_S products on the matrix cores take chunks of columns of their own.
-bool iq2_mm(const smoe_geom& g, int64_t T) { return g.w_type == SMOE_IQ2_S && smoe::iq2_mm_batch(T * g.top_k, g.n_expert); }
+bool iq2_mm(const smoe_geom& g, int64_t T) {
+    return g.w_type == SMOE_IQ2_S && smoe::iq2_mm_gains(T * g.top_k, g.n_expert, g.n_embd, g.n_ff);
+}
 int max_items_iq2_mm(const smoe_geom& g, int64_t T) {
     const int64_t P = T * g.top_k, S = smoe::iq2_mm_shared_chunk();
     return (int)((P < g.n_expert ? P : g.n_expert) + P / smoe::iq2_mm_chunk() + (sh_fused(g) ? (T + S - 1) / S : 0));

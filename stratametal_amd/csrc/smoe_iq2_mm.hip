@@ -13,7 +13,7 @@
 //
 // smoe_iq2.hip spends eight dots and about twelve more instructions per row, column and sub-block on the VALU; here it is
 // six, plus two matrix products that serve 16 x 16 of them and a costlier decode (fp16 pairs and their scaled copies), so a
-// tile of 16 columns costs what about six columns cost there (kIq2MmPairs).  Still bound by VALU issue: 600 tokens of 512
+// tile of 16 columns costs what about six columns cost there (iq2_mm_gains).  Still bound by VALU issue: 600 tokens of 512
 // experts (2048, 512 wide) 648 us on the row kernels, 472 here.  A wave's block is loaded at its step (four waves per SIMD
 // cover the load): prefetched a step ahead, its 21 registers spilled others, 482 us.
 #include "smoe_gemv.hpp"
@@ -282,8 +282,9 @@ constexpr int kDownTwoPasses = 2048;
 hipError_t launch_iq2_mm_down(const uint8_t* down_exps, const uint8_t* down_sh, const uint32_t* himg, int h_blocks,
                               const float* sg, const int4* items, int H, int F, int max_items, float* Y, hipStream_t s) {
     if (!iq2_shape_ok(H) || !iq2_shape_ok(F) || h_blocks != F / 32) return hipErrorInvalidValue;
-    // two passes where the halved grid still fills the chip (two work-groups per CU) four times
-    // (600 tokens of 512 experts, 2048 rows of 512: 165 us one by one, 155 in twos)
+    // two passes where the halved grid still fills the chip (two work-groups per CU) four times (600 tokens of 512
+    // experts, 2048 rows of 512: 165 us one by one, 155 in twos; the whole call of 512 experts of 2048 x 1024 1.01 times
+    // as fast; of 256 experts, 1300 work-groups, 1.01 at F 512 and 0.98 at F 1024, at 600 work-groups 0.96)
     const int rp = F <= 1024 && H % 512 == 0 && (int64_t)max_items * (H / 512) >= kDownTwoPasses ? 2 : 1;
     const int n_rb = H / (256 * rp);
     const dim3 grid(xcd_grid(n_rb, max_items));
@@ -299,12 +300,7 @@ hipError_t launch_iq2_mm_down(const uint8_t* down_exps, const uint8_t* down_sh, 
     return hipGetLastError();
 }
 
-// From how many routed pairs per expert on average the IQ2_S layer's products run here (the whole call, row kernels and
-// here: 512 experts 5.9 pairs 389 and 408 us, 11.7 pairs 648 and 472; 256 experts 6.2 pairs 210 and 194; 128 experts 4.7
-// pairs 76 and 84, 14 pairs 139 and 128), and the columns of its items: chunks of four tiles, so that a hot expert's
-// columns spread over work-groups.
-constexpr int kIq2MmPairs = 6;
-bool iq2_mm_batch(int64_t P, int E) { return P >= (int64_t)kIq2MmPairs * E; }
+// The columns of the items: chunks of four tiles, so that a hot expert's columns spread over work-groups.
 int iq2_mm_chunk() { return 4 * kCols; }
 int iq2_mm_shared_chunk() { return kCols; }
 

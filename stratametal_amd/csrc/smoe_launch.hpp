@@ -128,9 +128,8 @@ hipError_t launch_iq2_gu(const uint8_t* gate_exps, const uint8_t* up_exps, const
 hipError_t launch_iq2_down(const uint8_t* down_exps, const uint8_t* down_sh, const uint32_t* himg, int h_blocks,
                            const float* sg, const int4* items, int H, int F, int Fs, int max_items, float* Y,
                            hipStream_t s, const uint64_t* eptr = nullptr, const int32_t* dmap = nullptr);
-// the same products on the matrix cores (smoe_iq2_mm.hip), for batches of many pairs per expert: the items' chunks of
-// routed and shared columns, and whether a batch takes them
-bool iq2_mm_batch(int64_t P, int E);
+// the same products on the matrix cores (smoe_iq2_mm.hip), for the batches that iq2_mm_gains names: the items' chunks of
+// routed and shared columns
 int iq2_mm_chunk();
 int iq2_mm_shared_chunk();
 hipError_t launch_iq2_mm_gu(const uint8_t* gate_exps, const uint8_t* up_exps, const uint8_t* gate_sh, const uint8_t* up_sh,

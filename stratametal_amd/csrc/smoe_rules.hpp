@@ -68,4 +68,17 @@ constexpr HcWrite hc_write_kind(int64_t T, int n, int hc) {
     return n < 64 || (n < 256 && !all) ? kHcWriteValues : all ? kHcWriteStreams : kHcWriteStream;
 }
 
+// Whether an IQ2_S layer's products of P routed pairs run on the matrix cores (tiles of 16 columns; the row kernels'
+// cost grows with the columns).  An item's tiles go one after the other, so few experts leave the chip idle: from seven
+// or eight pairs per expert on where the products' work-groups, each as long as its rows, fill it; else from 64, or 128
+// with fewer than 32 experts, where an expert's pairs are several items.  Rows against matrix cores, the whole call: 512
+// experts of 2048 x 512 389 and 408 us at 5.9 pairs, 648 and 472 at 11.7; 128 experts of 2048 x 512, most pairs in 16 of
+// them, 150 and 189 at 6.3, 1.05 times as fast at 8; 16 experts 70 and 102 at 12.5, 137 and 188 at 38, 1.3 times as fast
+// at 100; 32 experts of 1024 x 2048 0.84 times at 11, 1.34 at 64; of 2048 x 2048 187 and 161 at 12.5.
+constexpr bool iq2_mm_gains(int64_t P, int E, int H, int F) {
+    const bool fills = (E >= 64 || (E >= 32 && H * F >= 2048 * 2048)) && (int64_t)E * F * 8 / H >= 128 &&
+                       (int64_t)E * H * 4 / F >= 128;
+    return P >= (int64_t)E * (fills ? E >= 128 ? 7 : 8 : E >= 32 ? 64 : 128);
+}
+
 }  // namespace smoe

@@ -80,3 +80,17 @@ def test_hc_write(ask):
     cases = [(64, 8, 200, 0), (64, 8, 4000, 2), (72, 4, 64, 0), (32, 8, 4000, 0), (512, 8, 64, 1), (256, 8, 16, 1), (256, 8, 1000, 2),
              (2048, 4, 1, 1), (2048, 4, 64, 1), (2048, 4, 1000, 1), (2048, 4, 4000, 2), (4096, 4, 1000, 2)]
     assert ask([f"hc_write_kind({T}, {n}, {hc})" for n, hc, T, _ in cases]) == [c[-1] for c in cases]
+
+
+def test_iq2_matrix_cores(ask):
+    """n_expert, n_embd, n_ff, pairs per expert: the faster of the row kernels (0) and the matrix cores (1); more pairs
+    never go back."""
+    cases = [(512, 2048, 512, 6, 0), (512, 2048, 512, 8, 1), (512, 2048, 512, 11.7, 1), (128, 2048, 512, 6.25, 0),
+             (128, 2048, 512, 8, 1), (64, 1024, 1024, 6.25, 0), (64, 512, 512, 8, 1), (16, 2048, 512, 8, 0),
+             (16, 2048, 512, 12.5, 0), (16, 2048, 512, 38, 0), (16, 2048, 512, 200, 1), (8, 2048, 1024, 40, 0),
+             (32, 2048, 512, 11, 0), (32, 1024, 2048, 11, 0), (32, 1024, 2048, 64, 1), (64, 512, 2048, 11, 0),
+             (32, 2048, 2048, 12.5, 1)]
+    assert ask([f"iq2_mm_gains({int(p * E)}, {E}, {H}, {F})" for E, H, F, p, _ in cases]) == [c[-1] for c in cases]
+    for E, H, F in [(512, 2048, 512), (64, 512, 2048), (16, 1024, 1024), (1, 512, 512)]:
+        got = ask([f"iq2_mm_gains({int(p * E)}, {E}, {H}, {F})" for p in (0.1, 1, 5, 7, 8, 16, 64, 100, 128, 1000)])
+        assert got == sorted(got) and got[-1] == 1
