@@ -463,7 +463,8 @@ __device__ __forceinline__ bool stage_direct(const Item& it, int c0, int nc, boo
     return !by_token || it.shared || c0 + nc <= 4;
 }
 
-// The rounds from `from` on, each issued and stored in turn.
+// The rounds from piece `from` up to piece `to` (whole rounds of 4 NT pieces, so `to` a multiple of that), each issued and
+// stored in turn.
 template <int NT>
 __device__ __forceinline__ void stage_images(uint32_t* act, const uint32_t* __restrict__ img, int qb, int c0, int nc,
                                              int cap_cols, const Item& it, const int32_t* perm, int k, bool by_token,

@@ -232,13 +232,13 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
         __builtin_amdgcn_sched_barrier(0);
         grid_table_store<64 * NW>(codes, tab);
         stage_commit_direct(sp, smem);
+        if (nc0 > 4)  // columns beyond those rounds
+            stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, kDirect * 64 * NW);
     } else {
         off = load_block_raw(rowp, b, raw);
         grid_table_store<64 * NW>(codes, tab);
-        stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, 0, kDirect * 64 * NW);
+        stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true);
     }
-    if (nc0 > 4)  // columns beyond those rounds
-        stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, kDirect * 64 * NW);
     __syncthreads();
     Iq2Block B[1];
     decode_block(raw, off, tab, B[0]);
