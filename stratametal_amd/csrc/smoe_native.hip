@@ -52,9 +52,17 @@ __device__ __forceinline__ int32_t nl4_bytes(uint32_t idx) {
     const uint32_t sel = idx & 0x07070707u;
     const uint32_t lo = __builtin_amdgcn_perm(0xF6EADDCFu, 0xBFAD9881u, sel);  // -49 -35 -22 -10, -127 -104 -83 -65
     const uint32_t hi = __builtin_amdgcn_perm(0x71594535u, 0x26190D01u, sel);  // 53 69 89 113, 1 13 25 38
-    const uint32_t m = ((idx >> 3) & 0x01010101u) * 0xFFu;
-    return (int32_t)((hi & m) | (lo & ~m));
+    const uint32_t m = (idx >> 3) & 0x01010101u, all = (m << 8) - m;  // 0xFF where the top bit is set
+    return (int32_t)((hi & all) | (lo & ~all));
 }
+
+// Four bytes of v, each at most 127, less `off` (at most 128) in each: signed bytes, no borrow between them (shifts,
+// subtractions and masks throughout: a 32-bit multiply takes four times as long).
+__device__ __forceinline__ int32_t bytes_less(uint32_t v, uint32_t off) {
+    return (int32_t)(((v | 0x80808080u) - off * 0x01010101u) ^ 0x80808080u);
+}
+// The four low bits of b as the lowest bits of four bytes.
+__device__ __forceinline__ uint32_t spread4(uint32_t b) { return __umul24(b & 15u, 0x204081u) & 0x01010101u; }
 
 // Q4_K / Q5_K: the 6-bit scale and min pair of two 32-value groups (iq_k_scale_min, metal/shaders/iq.metal:254-262)
 __device__ __forceinline__ void k_scale_min(const uint8_t* s, int bq8_offset, int (&sc)[2], int (&mn)[2]) {
@@ -88,11 +96,13 @@ struct XLds {
 // offset it subtracts after the dot is subtracted from each byte: the same integer).  dot(x): the partial against a
 // column's activations of the block (x its first 32-value block); the float steps are the reference's, one rounding
 // each (no contraction).  A dot times its scale is a 24-bit multiply: every dot is below 2^20, every scale below 2^8.
-template <int TYPE>
+// RAW: for one column, the codes stay unsigned and the offset is subtracted after the dot, as the reference has it: two to
+// four dots of ones more for the column, eight to sixteen instructions fewer to decode.
+template <int TYPE, bool RAW>
 struct NativePart;
 
-template <>
-struct NativePart<8> {  // Q8_0
+template <bool RAW>
+struct NativePart<8, RAW> {  // Q8_0
     int32_t w[8];
     float d;
     __device__ __forceinline__ void decode(const uint8_t* blk, int) {
@@ -109,8 +119,9 @@ struct NativePart<8> {  // Q8_0
     }
 };
 
-template <int TYPE>
+template <int TYPE, bool RAW>
 struct NativePart16 {  // Q4_0, Q5_0, IQ4_NL: 16 values of a 32-value block, words iqs, iqs + 1 and 4 words on
+    static constexpr int kOff = TYPE == 2 ? 8 : TYPE == 6 ? 16 : 0;
     int32_t lo[2], hi[2];
     float d;
     __device__ __forceinline__ void decode(const uint8_t* blk, int iqs) {
@@ -126,44 +137,36 @@ struct NativePart16 {  // Q4_0, Q5_0, IQ4_NL: 16 values of a 32-value block, wor
                 hi[i] = nl4_bytes(b);
                 continue;
             }
-            if constexpr (TYPE == 6) {  // value - 16: with the high bit the nibble, else the nibble | 0xF0
+            if constexpr (TYPE == 6) {
                 const uint32_t hs = h >> (4 * (iqs + i));
-                uint32_t ha = 0, hb = 0;  // 1 where the high bit is clear
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    ha |= ((~hs >> k) & 1u) << (8 * k);
-                    hb |= ((~hs >> (16 + k)) & 1u) << (8 * k);
-                }
-                a |= ha * 0xF0u;
-                b |= hb * 0xF0u;
-            } else {  // nibble - 8: bytes of n ^ 8, sign-extended from bit 3
-                a ^= 0x08080808u;
-                b ^= 0x08080808u;
-                a |= ((a >> 3) & 0x01010101u) * 0xF0u;
-                b |= ((b >> 3) & 0x01010101u) * 0xF0u;
+                a |= spread4(hs) << 4;
+                b |= spread4(hs >> 16) << 4;
             }
-            lo[i] = (int32_t)a;
-            hi[i] = (int32_t)b;
+            lo[i] = RAW ? (int32_t)a : bytes_less(a, kOff);
+            hi[i] = RAW ? (int32_t)b : bytes_less(b, kOff);
         }
         d = rdh(blk);
     }
     template <class X>
     __device__ __forceinline__ float dot(const X& x, int iqs) const {
-        int32_t s = 0;
+        int32_t s = 0, a = 0;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            s = dot4(lo[i], x.word(iqs + i), s);
-            s = dot4(hi[i], x.word(iqs + i + 4), s);
+            const int32_t u0 = x.word(iqs + i), u1 = x.word(iqs + i + 4);
+            s = dot4(lo[i], u0, s);
+            s = dot4(hi[i], u1, s);
+            if constexpr (RAW && kOff) a = dot4(0x01010101, u1, dot4(0x01010101, u0, a));
         }
+        if constexpr (RAW && kOff) s -= kOff * a;
         return (d * x.scale()) * (float)s;
     }
 };
-template <> struct NativePart<2> : NativePart16<2> {};
-template <> struct NativePart<6> : NativePart16<6> {};
-template <> struct NativePart<20> : NativePart16<20> {};
+template <bool RAW> struct NativePart<2, RAW> : NativePart16<2, RAW> {};
+template <bool RAW> struct NativePart<6, RAW> : NativePart16<6, RAW> {};
+template <bool RAW> struct NativePart<20, RAW> : NativePart16<20, RAW> {};
 
-template <>
-struct NativePart<23> {  // IQ4_XS: 32-value group iqs / 4, its 6-bit scale - 32
+template <bool RAW>
+struct NativePart<23, RAW> {  // IQ4_XS: 32-value group iqs / 4, its 6-bit scale - 32
     int32_t lo[4], hi[4], ls;
     float d;
     __device__ __forceinline__ void decode(const uint8_t* blk, int iqs) {
@@ -235,11 +238,11 @@ struct NativePartK {  // Q4_K, Q5_K: 8 values of two 32-value groups
         return d * sum_d - dmin * sum_m;
     }
 };
-template <> struct NativePart<12> : NativePartK<12> {};
-template <> struct NativePart<13> : NativePartK<13> {};
+template <bool RAW> struct NativePart<12, RAW> : NativePartK<12> {};
+template <bool RAW> struct NativePart<13, RAW> : NativePartK<13> {};
 
-template <>
-struct NativePart<11> {  // Q3_K: 2 low bits, - 4 where the high bit is clear; scale - 32
+template <bool RAW>
+struct NativePart<11, RAW> {  // Q3_K: 2 low bits, - 4 where the high bit is clear; scale - 32
     int32_t v[4];
     int sc[4];
     float d;
@@ -274,8 +277,8 @@ struct NativePart<11> {  // Q3_K: 2 low bits, - 4 where the high bit is clear; s
     }
 };
 
-template <>
-struct NativePart<14> {  // Q6_K: (low nibble | 2 high bits << 4) - 32 times an int8 scale
+template <bool RAW>
+struct NativePart<14, RAW> {  // Q6_K: (low nibble | 2 high bits << 4) - 32 times an int8 scale
     int32_t v[2];
     int sc[2];
     float d;
@@ -286,9 +289,8 @@ struct NativePart<14> {  // Q6_K: (low nibble | 2 high bits << 4) - 32 times an 
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             sc[i] = (int)(int8_t)blk[192 + scale_offset + 4 * i];
-            // six bits - 32: bytes of v ^ 32, sign-extended from bit 5
-            const uint32_t q = (((vl >> (4 * i)) & 0x0F0F0F0Fu) | (((vh >> (4 * i)) << 4) & 0x30303030u)) ^ 0x20202020u;
-            v[i] = (int32_t)(q | ((q >> 5) & 0x01010101u) * 0xC0u);
+            const uint32_t q = ((vl >> (4 * i)) & 0x0F0F0F0Fu) | (((vh >> (4 * i)) << 4) & 0x30303030u);
+            v[i] = RAW ? (int32_t)q : bytes_less(q, 32);
         }
         d = rdh(blk + 208);
     }
@@ -299,7 +301,10 @@ struct NativePart<14> {  // Q6_K: (low nibble | 2 high bits << 4) - 32 times an 
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             const X xi = x.at(2 * i);
-            sumf = sumf + xi.scale() * (float)__mul24(dot4(v[i], xi.word(iqs % 8), 0), sc[i]);
+            const int32_t u = xi.word(iqs % 8);
+            int32_t dq = dot4(v[i], u, 0);
+            if constexpr (RAW) dq -= dot4(0x20202020, u, 0);
+            sumf = sumf + xi.scale() * (float)__mul24(dq, sc[i]);
         }
         return d * sumf;
     }
@@ -310,10 +315,12 @@ struct NativePart<14> {  // Q6_K: (low nibble | 2 high bits << 4) - 32 times an 
 template <int TYPE, class X>
 __device__ __forceinline__ float native_row(const uint8_t* row, int npart, const X& col, float acc, int k) {
     using NT = NativeType<TYPE>;
-    // four partials at a time: their loads are in flight together, their sums added in order (not the wider partials
-    // of Q4_K and Q5_K, 3.3 us against 3.9 for 512 rows of 2048)
-    for (; TYPE != 12 && TYPE != 13 && k + 96 < npart; k += 128) {
-        NativePart<TYPE> p[4];
+    // four partials at a time: their loads are in flight together, their sums added in order (not the wider partials of
+    // Q4_K and Q5_K, 3.3 us against 3.9 for 512 rows of 2048, nor Q4_0 and Q6_K, whose few instructions want the waves
+    // instead: 4096 rows of 4096 4.7 against 5.0 and 5.7 against 6.7 us)
+    constexpr bool four = TYPE == 8 || TYPE == 6 || TYPE == 20 || TYPE == 23 || TYPE == 11;
+    for (; four && k + 96 < npart; k += 128) {
+        NativePart<TYPE, false> p[4];
         float v[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) p[j].decode(row + (size_t)((k + 32 * j) / NT::ipb) * NT::bytes, NT::step * ((k + 32 * j) % NT::ipb));
@@ -324,7 +331,7 @@ __device__ __forceinline__ float native_row(const uint8_t* row, int npart, const
         for (int j = 0; j < 4; ++j) acc = acc + v[j];
     }
     for (; k < npart; k += 32) {
-        NativePart<TYPE> p;
+        NativePart<TYPE, true> p;
         p.decode(row + (size_t)(k / NT::ipb) * NT::bytes, NT::step * (k % NT::ipb));
         acc = acc + p.dot(col.at(k / NT::ipb * (NT::qk / 32)), NT::step * (k % NT::ipb));
     }
@@ -475,7 +482,7 @@ __global__ __launch_bounds__(256) void k_mmvq_native_cols(const uint8_t* __restr
         __syncthreads();
         for (int k = l; k < npart; k += 32) {
             const int kb = k / NT::ipb, iqs = NT::step * (k % NT::ipb);
-            NativePart<TYPE> part[kRw];
+            NativePart<TYPE, false> part[kRw];
 #pragma unroll
             for (int j = 0; j < kRw; ++j) part[j].decode(row[j] + (size_t)(kb0 + kb) * NT::bytes, iqs);
 #pragma unroll
@@ -536,7 +543,7 @@ __device__ __forceinline__ uint2 word_bits(int32_t w) {
 
 // Partial k of a row's 256-value chunk into its fp16 row and its blocks' scales (dw: [8][ROWS]).
 template <int TYPE, int ROWS>
-__device__ __forceinline__ void nm_put(const NativePart<TYPE>& p, int k, uint8_t* wrow, float* dw) {
+__device__ __forceinline__ void nm_put(const NativePart<TYPE, false>& p, int k, uint8_t* wrow, float* dw) {
     if constexpr (TYPE == 8) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -599,7 +606,7 @@ __global__ __launch_bounds__(256) void k_native_mm(const uint8_t* __restrict__ w
         const uint32_t* src = xd + (size_t)(v0 / 32 + min(tid & 7, nb - 1)) * 9;
 #pragma unroll
         for (int m = 0; m < 9; ++m) xw[m] = src[m];
-        NativePart<TYPE> part[U];
+        NativePart<TYPE, false> part[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int p = tid + 256 * u, k = min(p % NP, np - 1);
