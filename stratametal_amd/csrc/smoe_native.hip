@@ -12,6 +12,7 @@
 #include "smoe_device.hpp"
 #include "smoe_gemv.hpp"
 #include "smoe_launch.hpp"
+#include "smoe_rules.hpp"
 
 namespace smoe {
 
@@ -440,6 +441,7 @@ __global__ __launch_bounds__(256) void k_mmvq_native(const uint8_t* __restrict__
 // 512 x 2048 232 and 58 us, IQ4_NL 2048 x 512 609 and 36 us.  Bound by the VALU: about nine instructions per 16 products
 // for IQ4_NL, 22 for Q3_K.
 constexpr int kRw = 2, kXlChunk = 2048;
+static_assert(8 * kRw == kNativeTileRows, "the rows of a work-group");
 template <int TYPE, int C>
 __global__ __launch_bounds__(256) void k_mmvq_native_cols(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                                                           int n_in, int n_out, int n_col,
@@ -731,29 +733,14 @@ int64_t native_row_bytes(int type, int64_t n) {
     return (n <= 0 || n % qk) ? -1 : n / qk * bytes;
 }
 
-// Columns per work-group: the most of 16, 8 and 4 that leaves the chip two work-groups per CU, else 4.  Below
-// kColsGroupsMin work-groups of 4 columns, a work-group per column and eight rows: a tile's chain of columns is then the
-// longer one (by type, 512 x 2048 at 16 columns: 3.9 to 6.6 us against 5.0 to 8.5 in tiles, at 32 columns 5.8 to 10.9
-// against 4.1 to 8.4; 2048 x 512 at 4 columns 2.9 against 3.5, at 8 columns 3.8 to 4.3 against 3.1).
-constexpr int kColsGroups = 512, kColsGroupsMin = 224;
-
 hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y,
                               int ldy, const float* sg, hipStream_t s, const uint8_t* w2, float* y2) {
     if (!native_type(type) || n_in % native_block_values(type)) return hipErrorInvalidValue;
-    const unsigned nz = w2 ? 2 : 1;
-    const int rg = (n_out + 8 * kRw - 1) / (8 * kRw);
-    int cols = 1;
-    if ((int64_t)rg * ((n_col + 3) / 4) * nz >= kColsGroupsMin && n_col >= 4 && n_col / 4 < 65535) {
-        cols = 4;
-        for (int c = 16; c > 4; c /= 2)
-            if ((int64_t)rg * ((n_col + c - 1) / c) * nz >= kColsGroups) {
-                cols = c;
-                break;
-            }
-    }
+    const int nz = w2 ? 2 : 1;
+    const int rg = (n_out + kNativeTileRows - 1) / kNativeTileRows, cols = native_cols(type, n_in, n_out, n_col, nz);
     const int cg = n_col < 64 ? n_col : 64;
-    const dim3 grid1((unsigned)((n_out + 7) / 8), (unsigned)cg, nz);
-    const dim3 gridc((unsigned)rg, (unsigned)((n_col + cols - 1) / cols), nz);
+    const dim3 grid1((unsigned)((n_out + 7) / 8), (unsigned)cg, (unsigned)nz);
+    const dim3 gridc((unsigned)rg, (unsigned)((n_col + cols - 1) / cols), (unsigned)nz);
     const size_t lds = (size_t)cols * (n_in < kXlChunk ? n_in : kXlChunk) / 32 * kXlDw * 4;
 #define SMOE_NATC(T, C) \
     hipLaunchKernelGGL((k_mmvq_native_cols<T, C>), gridc, dim3(256), lds, s, w, w2, n_in, n_out, n_col, xq, y, y2, ldy, sg)

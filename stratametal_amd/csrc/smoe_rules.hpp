@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cstdint>
+#include <initializer_list>
 
 namespace smoe {
 
@@ -79,6 +80,24 @@ constexpr bool iq2_mm_gains(int64_t P, int E, int H, int F) {
     const bool fills = (E >= 64 || (E >= 32 && H * F >= 2048 * 2048)) && (int64_t)E * F * 8 / H >= 128 &&
                        (int64_t)E * H * 4 / F >= 128;
     return P >= (int64_t)E * (fills ? E >= 128 ? 7 : 8 : E >= 32 ? 64 : 128);
+}
+
+// The native types' GEMV of n_col columns (nz matrices by one launch): columns per work-group of the column tiles, or 1
+// for a work-group per column and eight rows.  The most of 16, 8 and 4 that is not half empty and leaves the chip two
+// work-groups per CU, else 4; a tile's chain of columns is the longer one, so few work-groups of 4 columns go by columns (512 x 2048 at 16 columns
+// 3.9 to 6.6 us by type against 5.0 to 8.5 in tiles, at 32 5.8 to 10.9 against 4.1 to 8.4).  Q4_K, Q5_K and Q6_K, whose
+// decode the tiles save little of, from six or eight columns and more work-groups, long rows more yet (by columns and in tiles:
+// Q4_K 256 x 20000 at 4 columns 8.3 and 12.4, Q5_K 512 x 2048 at 5 3.2 and 3.7, Q6_K 8192 x 1000 at 24 40 and 49, at 48 1.4
+// times as fast in tiles).
+constexpr int kNativeTileRows = 16;
+constexpr int native_cols(int type, int n_in, int n_out, int n_col, int nz) {
+    const int64_t rg = ((int64_t)n_out + kNativeTileRows - 1) / kNativeTileRows * nz;
+    const bool k = type == 12 || type == 13 || type == 14;
+    const int64_t least = !k || n_col >= 128 ? 224 : n_in <= 4096 ? 336 : 480;
+    if (n_col < (!k ? 4 : rg >= 256 ? 6 : 8) || n_col / 4 >= 65535 || rg * ((n_col + 3) / 4) < least) return 1;
+    for (const int c : {16, 8})
+        if (2 * n_col > c && rg * ((n_col + c - 1) / c) >= 512) return c;
+    return 4;
 }
 
 }  // namespace smoe
