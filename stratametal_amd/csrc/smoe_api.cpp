@@ -394,7 +394,7 @@ smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float
     auto gemv = [&](int type, const void* wt, const uint8_t* xq, int n_in, int n_out, float* y,
                     const float* gate) -> hipError_t {
         const uint8_t* wb = static_cast<const uint8_t*>(wt);
-        if (mm && smoe::native_mm_ok(type, n_out)) return smoe::launch_native_mm(type, wb, xq, n_in, n_out, T, y, n_out, gate, st);
+        if (mm && smoe::native_mm_ok(type, n_out, T, 1)) return smoe::launch_native_mm(type, wb, xq, n_in, n_out, T, y, n_out, gate, st);
         if (smoe::native_type(type)) return smoe::launch_mmvq_native(type, wb, xq, n_in, n_out, T, y, n_out, gate, st);
         hipError_t e = type == SMOE_IQ2_S ? smoe::launch_iq2_mmvq(wb, xq, n_in, n_out, T, y, st)
                                           : smoe::launch_q2_mmvq(wb, xq, n_in, n_out, T, y, st);
@@ -413,7 +413,7 @@ smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float
     }
     SMOE_TRY(smoe::launch_prep(x, (int64_t)T * H, nxq, nullptr, st), "shared q8_1");
     if (pair) {
-        const auto gu = mm && smoe::native_mm_ok(tg, Fn) ? smoe::launch_native_mm : smoe::launch_mmvq_native;
+        const auto gu = mm && smoe::native_mm_ok(tg, Fn, T, 2) ? smoe::launch_native_mm : smoe::launch_mmvq_native;
         SMOE_TRY(gu(tg, gw, nxq, H, Fn, T, ngu, Fn, nullptr, st, uw, ngu + (size_t)T * Fn), "shared gate/up");
     } else {
         SMOE_TRY(gemv(tg, gw, nxq, H, Fn, ngu, nullptr), "shared gate");

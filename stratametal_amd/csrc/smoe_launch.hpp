@@ -107,7 +107,7 @@ hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int
                               int ldy, const float* sg, hipStream_t s, const uint8_t* w2 = nullptr, float* y2 = nullptr);
 // the product of a prompt's columns on the matrix cores (exact 32-value dots, sums in an order of its own; y 16-byte
 // aligned, ldy % 4 == 0)
-bool native_mm_ok(int type, int n_out);
+bool native_mm_ok(int type, int n_out, int n_col, int nz);
 hipError_t launch_native_mm(int type, const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y,
                             int ldy, const float* sg, hipStream_t s, const uint8_t* w2 = nullptr, float* y2 = nullptr);
 // a native shared expert of a few tokens in two launches (h: T * F floats of scratch; y rows written, or with add added to)

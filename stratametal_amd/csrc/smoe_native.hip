@@ -766,20 +766,21 @@ hipError_t launch_mmvq_native(int type, const uint8_t* w, const uint8_t* xq, int
     return hipGetLastError();
 }
 
-// The prompt's product on the matrix cores: the types k_native_mm takes, rows stored four at a time.
-bool native_mm_ok(int type, int n_out) {
-    return (type == 8 || type == 2 || type == 6 || type == 20 || type == 11) && n_out % 4 == 0;
+// The prompt's product on the matrix cores, where it is the faster: the types k_native_mm takes, rows stored four at a time.
+bool native_mm_ok(int type, int n_out, int n_col, int nz) {
+    return (type == 8 || type == 2 || type == 6 || type == 20 || type == 11) && n_out % 4 == 0 &&
+           native_mm_gains(n_out, n_col, nz);
 }
 
 hipError_t launch_native_mm(int type, const uint8_t* w, const uint8_t* xq, int n_in, int n_out, int n_col, float* y,
                             int ldy, const float* sg, hipStream_t s, const uint8_t* w2, float* y2) {
     const uintptr_t al = reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(y2);
     const int cg = (n_col + kNmCols - 1) / kNmCols;
-    if (!native_mm_ok(type, n_out) || native_row_bytes(type, n_in) <= 0 || n_col < 1 || cg > 65535 || ldy % 4 || (al & 15))
+    const unsigned nz = w2 ? 2 : 1;
+    if (!native_mm_ok(type, n_out, n_col, (int)nz) || native_row_bytes(type, n_in) <= 0 || cg > 65535 || ldy % 4 || (al & 15))
         return hipErrorInvalidValue;
     // 32 rows while 64 leave no second work-group per CU (the layer call at 128, 400 and 900 tokens: 221, 289 and 439 us
     // in 32 rows, 227, 290 and 427 in 64)
-    const unsigned nz = w2 ? 2 : 1;
     const int rows = (int64_t)((n_out + 63) / 64) * cg * nz <= 256 ? 32 : 64;
     const dim3 grid((unsigned)((n_out + rows - 1) / rows), (unsigned)cg, nz);
 #define SMOE_NMR(T, R) \
@@ -799,11 +800,9 @@ hipError_t launch_native_mm(int type, const uint8_t* w, const uint8_t* xq, int n
     return hipGetLastError();
 }
 
-// A native shared expert of up to kNativeFewTokens tokens whose gate and up have one type and whose down is native.
-// (Every work-group quantises its whole row, so more tokens are better served by the stage kernels' column tiles.)
-constexpr int kNativeFewTokens = 4;
+// A native shared expert whose gate and up have one type and whose down is native, where two launches are the faster.
 bool native_few_ok(int gu_type, int d_type, int T, int H, int F) {
-    return T <= kNativeFewTokens && native_row_bytes(gu_type, H) > 0 && native_row_bytes(d_type, F) > 0 && H <= 4096 &&
+    return T <= 4 && native_row_bytes(gu_type, H) > 0 && native_row_bytes(d_type, F) > 0 && H <= 4096 &&
            F <= 4096;
 }
 

@@ -106,3 +106,11 @@ def test_native_columns(ask):
              (8, 256, 20000, 5, 1, 8)]
     assert ask([f"native_cols({t}, {i}, {o}, {c}, {z})" for t, i, o, c, z, _ in cases]) == [c[-1] for c in cases]
     assert ask(["native_cols(8, 32, 2147483647, 2147483647, 2)"]) == [1]  # the grid's y dimension
+
+
+def test_native_shared(ask):
+    """Rows, columns, matrices: the matrix cores (1) or the row kernels (0), which alone a prompt of few tokens takes
+    (traced or not, the same order)."""
+    mm = [(512, 1, 2, 0), (512, 4, 2, 0), (512, 64, 2, 0), (512, 127, 2, 0), (512, 128, 2, 1), (512, 128, 1, 0), (512, 256, 1, 1),
+          (2048, 128, 1, 1), (4096, 32, 1, 0), (256, 128, 1, 0), (256, 1000, 1, 1)]
+    assert ask([f"native_mm_gains({n}, {c}, {z})" for n, c, z, _ in mm]) == [c[-1] for c in mm]
