@@ -802,7 +802,7 @@ hipError_t launch_native_mm(int type, const uint8_t* w, const uint8_t* xq, int n
 
 // A native shared expert whose gate and up have one type and whose down is native, where two launches are the faster.
 bool native_few_ok(int gu_type, int d_type, int T, int H, int F) {
-    return T <= 4 && native_row_bytes(gu_type, H) > 0 && native_row_bytes(d_type, F) > 0 && H <= 4096 &&
+    return native_few_gains(T, H, F) && native_row_bytes(gu_type, H) > 0 && native_row_bytes(d_type, F) > 0 && H <= 4096 &&
            F <= 4096;
 }
 

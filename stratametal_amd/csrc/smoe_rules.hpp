@@ -100,6 +100,13 @@ constexpr int native_cols(int type, int n_in, int n_out, int n_col, int nz) {
     return 4;
 }
 
+// A native shared expert of T tokens in two launches (k_native_gu, k_native_down): every work-group quantises its token's
+// whole row again and takes eight rows of it, so the stage kernels, whose tokens share a row's decode and one quantised
+// row, win where tokens times weights are many (the layer's call with the two launches against it, Q8_0: 4 tokens 2048 x 512
+// 1.16 times as fast, 1 token 4096 x 4096 1.00, 2 tokens 3072 x 1536 1.05, 2048 x 2048 1.14, 4 tokens 0.97, 4096 x 4096
+// 0.63; Q4_K 3 tokens 3072 x 1536 0.93).
+constexpr bool native_few_gains(int T, int H, int F) { return T <= 4 && (int64_t)T * H * F <= (int64_t)10 << 20; }
+
 // The native shared expert's products of a prompt on the matrix cores (nz matrices of n_out rows by one launch): a chunk
 // of K after the other is a chain of latencies, so from 128 columns, and 128 tiles of 32 rows by 32 columns (the layer's
 // call on the matrix cores against the row kernels: Q8_0 2048 x 512 0.81 at 5 columns, 0.88 at 64, 0.98 at 128, 1.05 at 200;

@@ -109,8 +109,11 @@ def test_native_columns(ask):
 
 
 def test_native_shared(ask):
-    """Rows, columns, matrices: the matrix cores (1) or the row kernels (0), which alone a prompt of few tokens takes
-    (traced or not, the same order)."""
+    """Tokens, n_embd, n_ff_shared: two launches (1) or the stage kernels (0); rows, columns, matrices: the matrix cores
+    (1) or the row kernels (0), which alone a prompt of few tokens takes (traced or not, the same order)."""
+    few = [(1, 2048, 512, 1), (4, 2048, 512, 1), (5, 2048, 512, 0), (2, 2048, 2048, 1), (3, 2048, 2048, 0), (4, 4096, 4096, 0),
+           (2, 4096, 4096, 0), (2, 3072, 1536, 1), (3, 3072, 1536, 0), (4, 4096, 256, 1)]
+    assert ask([f"native_few_gains({T}, {H}, {F})" for T, H, F, _ in few]) == [c[-1] for c in few]
     mm = [(512, 1, 2, 0), (512, 4, 2, 0), (512, 64, 2, 0), (512, 127, 2, 0), (512, 128, 2, 1), (512, 128, 1, 0), (512, 256, 1, 1),
           (2048, 128, 1, 1), (4096, 32, 1, 0), (256, 128, 1, 0), (256, 1000, 1, 1)]
     assert ask([f"native_mm_gains({n}, {c}, {z})" for n, c, z, _ in mm]) == [c[-1] for c in mm]

@@ -1,5 +1,5 @@
-"""GPU parity of the native shared expert at the token counts where it changes kernels: the row kernels or the
-matrix cores for a prompt (native_mm_gains).  Where a call
+"""GPU parity of the native shared expert at the token counts where it changes kernels: two launches or the stage kernels
+for a few tokens (native_few_gains), the row kernels or the matrix cores for a prompt (native_mm_gains).  Where a call
 runs the row kernels' order it is theirs bit for bit (smoe_mmvq's chain, the oracle's), traced or not; on the matrix cores
 within the bounds that test_gpu_native_mm.py derives; and a token of infinities or NaN leaves the others' rows."""
 import numpy as np
@@ -36,6 +36,16 @@ def test_prefill_contract_traced_and_not(torch, types, T):  # noqa: F811
     y = host(torch, ml.forward(x, path=S.PATH_MFMA))
     y2, _ = ml.forward(x, path=S.PATH_MFMA, trace=True, stages=True)
     assert np.array_equal(bits(y), bits(host(torch, y2)))
+
+
+@pytest.mark.parametrize("H, F, T", [(2048, 2048, 2), (2048, 2048, 3), (4096, 1024, 3), (4096, 2048, 1), (4096, 4096, 1)])
+def test_few_tokens(torch, H, F, T):  # noqa: F811
+    """The decode contract at both sides of the two-launch line, the oracle's bits."""
+    say(f"case: native shared, few tokens H={H} F={F} T={T}")
+    g, w_host, _, ml = layer(torch, H, F, O.Q3_K, O.Q3_K, O.IQ4_NL, T, 830 + T)
+    x = O.gen_normal(830 + T, 100, T * H).reshape(T, H)
+    want = O.moe_decode_dev(g, w_host, x, n_threads=16)
+    assert np.array_equal(bits(host(torch, ml.forward(dev(torch, x)))), bits(want))
 
 
 MM = [
