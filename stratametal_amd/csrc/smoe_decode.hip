@@ -18,6 +18,7 @@
 #include "smoe_items.hpp"
 #include "smoe_gemv.hpp"
 #include "smoe_launch.hpp"
+#include "smoe_rules.hpp"
 
 namespace smoe {
 
@@ -2849,11 +2850,9 @@ static unsigned router_grid_x(int blocks, int T, int tile) {
     return (unsigned)(T > tile ? (blocks + 7) / 8 * 8 : blocks);
 }
 
-// From kRouterTileTokens tokens a call without the fused junction runs k_router_tile: 512 rows of 2048, k_router and the
-// tiles, bf16 6.3 and 6.3 us at 5 tokens, 8.4 and 6.4 at 16, 19.8 and 7.7 at 64, 126 and 38 at 600; f32 7.8 and 5.9 at 5,
-// 27 and 7.1 at 64, 204 and 41 at 600.  The tile: few tokens need the work-groups (bf16 4 rows by 4 tokens, f32 2 by 8),
-// from kRouterTileWide on 4 by 8 re-reads less (bf16 9.6 against 10.4 us at 100 tokens, 11.4 against 10.7 at 127).
-constexpr int kRouterTileTokens = 5, kRouterTileWide = 112;
+// The tile: few tokens need the work-groups (bf16 4 rows by 4 tokens, f32 2 by 8), from kRouterTileWide on 4 by 8 re-reads
+// less (512 rows of 2048, bf16 9.6 against 10.4 us at 100 tokens, 11.4 against 10.7 at 127).
+constexpr int kRouterTileWide = 112;
 
 template <bool F32, int RR, int TT>
 static hipError_t launch_router_tile(const float* xf, const uint16_t* xb, const void* W, const uint16_t* w_inp,
@@ -2883,7 +2882,7 @@ hipError_t launch_router(const float* xf, const uint16_t* xb, const void* W, con
     // the f32 router runs on the row-per-wave path from f32 x
     if (w_f32 && (tile_rows || !xf || H % 4 || H > 4096)) return hipErrorInvalidValue;
     const bool x16 = xf ? (reinterpret_cast<uintptr_t>(xf) & 15) == 0 : (reinterpret_cast<uintptr_t>(xb) & 15) == 0;
-    if (!tile_rows && !rprev && !clear_n16 && T >= kRouterTileTokens && x16 && H % 8 == 0 && (xf || !w_inp)) {
+    if (!tile_rows && !rprev && !clear_n16 && router_tiles(T, E, H, w_f32 != 0) && x16 && H % 8 == 0 && (xf || !w_inp)) {
 #define SMOE_ROUTER_TILE(F, RR, TT) \
     launch_router_tile<F, RR, TT>(xf, xb, W, w_inp, bias, H, E, T, logits, ld_logits, sg, ximg, img_natural, s)
         if (T >= kRouterTileWide) return w_f32 ? SMOE_ROUTER_TILE(true, 4, 8) : SMOE_ROUTER_TILE(false, 4, 8);

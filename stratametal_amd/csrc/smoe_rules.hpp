@@ -115,4 +115,13 @@ constexpr bool native_mm_gains(int n_out, int n_col, int nz) {
     return n_col >= 128 && (int64_t)((n_out + 31) / 32) * ((n_col + 31) / 32) * nz >= 128;
 }
 
+// Whether the router of T tokens without the fused junction runs k_router_tile: from five tokens on, but for long bf16 rows
+// of few experts, whose waves walk K in stages while most of the chip is idle.  512 rows of 2048, k_router and the tiles, us:
+// bf16 6.3 and 6.3 at 5 tokens, 8.4 and 6.4 at 16, 19.8 and 7.7 at 64, 126 and 38 at 600; f32 7.8 and 5.9 at 5, 27 and 7.1 at
+// 64.  bf16 rows of 4096, the tiles' gain: 8 experts -1.0 at 8 tokens, +1.6 at 64; 32 experts -1.8 at 5; 128 experts -0.4 at
+// 8, +0.3 at 16; 512 experts 0.0 at 5, +2.4 at 16.
+constexpr bool router_tiles(int64_t T, int E, int H, bool f32) {
+    return T >= 5 && (f32 || H <= 2560 || T * (E > 64 ? E : 64) >= 2048);
+}
+
 }  // namespace smoe

@@ -117,3 +117,11 @@ def test_native_shared(ask):
     mm = [(512, 1, 2, 0), (512, 4, 2, 0), (512, 64, 2, 0), (512, 127, 2, 0), (512, 128, 2, 1), (512, 128, 1, 0), (512, 256, 1, 1),
           (2048, 128, 1, 1), (4096, 32, 1, 0), (256, 128, 1, 0), (256, 1000, 1, 1)]
     assert ask([f"native_mm_gains({n}, {c}, {z})" for n, c, z, _ in mm]) == [c[-1] for c in mm]
+
+
+def test_router_tiles(ask):
+    """Tokens, experts, n_embd, f32 rows: k_router (0) or the tiles (1)."""
+    cases = [(4, 512, 2048, 0, 0), (5, 512, 2048, 0, 1), (5, 512, 2048, 1, 1), (5, 8, 512, 0, 1), (5, 32, 4096, 0, 0),
+             (8, 8, 4096, 0, 0), (16, 64, 4096, 0, 0), (64, 8, 4096, 0, 1), (16, 128, 4096, 0, 1), (5, 512, 4096, 0, 1),
+             (5, 8, 4096, 1, 1), (127, 8, 4096, 0, 1)]
+    assert ask([f"router_tiles({T}, {E}, {H}, {f})" for T, E, H, f, _ in cases]) == [c[-1] for c in cases]

@@ -1,0 +1,60 @@
+"""GPU parity of the router and the junction at the token counts where they change kernels (router_tiles, junction_apart),
+bit for bit: the whole decode-contract block with the oracle's device order, and the junction form with residual_rmsnorm
+and the block one after the other; a subnormal token, and a token of infinities or NaN beside the others."""
+import numpy as np
+import pytest
+
+import oracle as O
+import stratametal_amd as S
+from test_gpu_decode import bits, dev, host, torch  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def layer(H, E, router, T, seed):
+    g = O.Geom(n_embd=H, n_ff=128, n_ff_shared=128, n_expert=E, top_k=3, router_dtype=router)
+    return g, S.MoELayer(S.Geom(**vars(g)), S.synth_layer(S.Geom(**vars(g)), seed), max_tokens=T)
+
+
+@pytest.mark.parametrize("H,E,T,router", [(4096, 40, 31, 0), (4096, 40, 32, 0), (4096, 130, 15, 0), (4096, 130, 16, 0),
+                                          (2560, 40, 5, 0), (4096, 9, 5, 1), (2048, 33, 4, 0), (2048, 33, 5, 0)])
+def test_block(torch, H, E, T, router):  # noqa: F811
+    print(f"case: router rule block H={H} E={E} T={T} router {router}", flush=True)
+    g, ml = layer(H, E, router, T, 78)
+    w_host = O.make_weights(g, 78)
+    x = O.gen_normal(78, 100, T * H).reshape(T, H)
+    x[1] *= np.float32(1e-30)
+    x[3] *= np.float32(1e4)
+    y, tr = ml.forward(dev(torch, x), trace=True, path=S.PATH_GEMV)
+    want, wtr = O.moe_decode_dev(g, w_host, x, trace=True, n_threads=8)
+    for k in ("logits", "sgate", "ids", "weights"):
+        assert np.array_equal(bits(host(torch, tr[k])).ravel(), bits(np.asarray(wtr[k])).ravel()), k
+    assert np.array_equal(bits(host(torch, y)), bits(want))
+
+
+@pytest.mark.parametrize("router", [0, 1])
+def test_subnormal_token(torch, router):  # noqa: F811
+    """A token subnormal in f32 and bf16 has the bits of its own one-token call in the tiles too."""
+    H, E, T = 512, 33, 7
+    print(f"case: router tiles with a subnormal token, router {router}", flush=True)
+    _, ml = layer(H, E, router, T, 79)
+    x = O.gen_normal(79, 100, T * H).reshape(T, H)
+    x[1] *= np.float32(1e-39)
+    _, tr = ml.forward(dev(torch, x), trace=True)
+    for t in (0, 1, 6):
+        _, tr1 = ml.forward(dev(torch, x[t:t + 1]), trace=True)
+        for k in ("logits", "sgate", "weights"):
+            assert np.array_equal(bits(host(torch, tr[k])).reshape(T, -1)[t], bits(host(torch, tr1[k])).ravel()), (k, t)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_other_tokens(torch, value):  # noqa: F811
+    H, E, T = 512, 33, 21
+    print(f"case: router tiles with a token of {value}", flush=True)
+    _, ml = layer(H, E, 0, T, 79)
+    x = O.gen_normal(79, 100, T * H).reshape(T, H)
+    y0 = host(torch, ml.forward(dev(torch, x)))
+    x[6, ::3] = value
+    y = host(torch, ml.forward(dev(torch, x)))
+    keep = np.arange(T) != 6
+    assert np.array_equal(bits(y[keep]), bits(y0[keep])) and np.isfinite(y[keep]).all()
