@@ -59,10 +59,6 @@ constexpr int kFusedRouteTokens = 4;
 constexpr int kDispatchMultiPairs = 2048;
 // SMOE_PATH_AUTO runs the MFMA (prefill) contract from this many tokens on.
 constexpr int kMfmaTokens = 128;
-// The decode path runs the junction as a kernel of its own from this many tokens on: before, its fusion into the router
-// kernel saves the launch; from here on the tiled router gains more (junction and router, 512 experts of 2048: 9.9 us fused
-// and 10.0 apart at 8 tokens, 10.3 and 9.7 at 12, 14.6 and 9.8 at 16, 28.8 and 12.0 at 48).
-constexpr int kJunctionApartTokens = 12;
 // The MFMA kernels' buffer offsets into the activation and h records are 31-bit.
 constexpr size_t kMfmaRecordLimit = (size_t)1 << 31;
 // The prefill path's Y (f32 per-pair rows) from this size on is stored and read with streaming accesses (half the
@@ -486,7 +482,8 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
     } while (0)
     SMOE_MARK();
     // the junction is fused into the router kernel of few tokens; more tokens take it as a kernel of its own
-    const bool fused_norm = x_prev && !mfma && n_tokens < kJunctionApartTokens;
+    const bool fused_norm =
+        x_prev && !mfma && !smoe::junction_apart(T, E, H, g->router_dtype == SMOE_ROUTER_F32);
     // the prefill path's per-work-group flags of its fp16 operand limits (folded by a trace or smoe_forward_status)
     int32_t* xflags = mfma ? reinterpret_cast<int32_t*>(ws + L.oflags) : nullptr;
     int32_t* hflags = xflags ? xflags + L.n_xflags : nullptr;

@@ -124,4 +124,14 @@ constexpr bool router_tiles(int64_t T, int E, int H, bool f32) {
     return T >= 5 && (f32 || H <= 2560 || T * (E > 64 ? E : 64) >= 2048);
 }
 
+// Whether the decode path runs the junction of T tokens as a kernel of its own: fused into the router kernel it saves the
+// launch, and repeats the norm in every work-group of the router.  Apart from 12 tokens on where the tiled router's gain
+// passes the launch, us: bf16, 512 experts of 2048 +0.4 at 10 tokens, +0.8 at 12, +3.6 at 16, 28.8 to 12.0 at 48; 64 experts
+// of 2048 -0.6 at 12, -1.3 at 16, +0.3 at 32; of 4096 -1.4 at 12, +4.4 at 32; 256 experts of 512 +0.4 at 12, +1.1 at 32;
+// 8 experts of 512 -0.6 at 32, +7 at 127; f32 rows longer than 2048 +4 and more at any number of experts.
+constexpr bool junction_apart(int64_t T, int E, int H, bool f32) {
+    return T >= 12 && ((f32 && H > 2048) || T >= (H >= 2048 ? 32 : 80) ||
+                       T * E >= (H >= 2560 ? 2048 : H >= 2048 ? 4096 : 8192));
+}
+
 }  // namespace smoe

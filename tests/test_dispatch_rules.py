@@ -125,3 +125,11 @@ def test_router_tiles(ask):
              (8, 8, 4096, 0, 0), (16, 64, 4096, 0, 0), (64, 8, 4096, 0, 1), (16, 128, 4096, 0, 1), (5, 512, 4096, 0, 1),
              (5, 8, 4096, 1, 1), (127, 8, 4096, 0, 1)]
     assert ask([f"router_tiles({T}, {E}, {H}, {f})" for T, E, H, f, _ in cases]) == [c[-1] for c in cases]
+
+
+def test_junction_apart(ask):
+    """Tokens, experts, n_embd, f32 rows: the junction in the router kernel (0) or a kernel of its own (1)."""
+    cases = [(11, 512, 2048, 0, 0), (12, 512, 2048, 0, 1), (12, 64, 2048, 0, 0), (16, 64, 2048, 0, 0), (32, 64, 2048, 0, 1),
+             (16, 256, 512, 1, 0), (32, 256, 512, 0, 1), (12, 8, 4096, 0, 0), (16, 64, 4096, 0, 0), (32, 64, 4096, 0, 1),
+             (12, 1024, 4096, 0, 1), (12, 8, 4096, 1, 1), (12, 8, 2048, 1, 0), (32, 8, 512, 0, 0), (127, 8, 512, 0, 1)]
+    assert ask([f"junction_apart({T}, {E}, {H}, {f})" for T, E, H, f, _ in cases]) == [c[-1] for c in cases]

@@ -58,3 +58,17 @@ def test_other_tokens(torch, value):  # noqa: F811
     y = host(torch, ml.forward(dev(torch, x)))
     keep = np.arange(T) != 6
     assert np.array_equal(bits(y[keep]), bits(y0[keep])) and np.isfinite(y[keep]).all()
+
+
+@pytest.mark.parametrize("H,E,T,router", [(512, 40, 11, 0), (512, 40, 79, 0), (512, 40, 80, 0), (512, 40, 79, 1), (1024, 700, 12, 1),
+                                          (2048, 40, 31, 0), (2048, 40, 32, 0), (2048, 40, 31, 1), (2560, 40, 12, 1),
+                                          (2560, 40, 31, 0), (4096, 40, 31, 0), (4096, 700, 12, 0)])
+def test_junction(torch, H, E, T, router):  # noqa: F811
+    print(f"case: junction rule H={H} E={E} T={T} router {router}", flush=True)
+    _, ml = layer(H, E, router, T, 80)
+    a, r = (dev(torch, O.gen_normal(80, s, T * H).reshape(T, H)) for s in (100, 101))
+    x = torch.empty_like(a)
+    y = ml.forward_residual(a, r, x, eps=1e-6)
+    xn = S.residual_rmsnorm(a, r, 1e-6)
+    assert np.array_equal(bits(host(torch, x)), bits(host(torch, xn)))
+    assert np.array_equal(bits(host(torch, y)), bits(host(torch, ml.forward(xn))))
