@@ -819,7 +819,7 @@ def expert_table(ptrs, device="cuda"):
 def expert_group(ids, k_per_tok: int, n_expert: int, table, stream=None) -> Dict:
     """The hit/miss split of the routed entries `ids` (int32, T * k_per_tok) by the expert table (int64 device
     addresses, 0 = not held), on the device (smoe_expert_group): grp_ptr, grp_expert, grp_start, ent_dst,
-    ent_tok, miss_dst and counts {groups, hits, misses, 0}."""
+    ent_tok, miss_dst and counts {groups, hits, misses, 0}.  The lists are views of two allocations."""
     import torch
     _need(ids, "ids", torch.int32)
     _need(table, "table", torch.int64, numel=n_expert)
@@ -870,7 +870,7 @@ def expert_grouped(g: Geom, groups: Dict, x_q8, n_tokens: int, out, cap_groups: 
 class VerifyWindow:
     """The verify window with the hit/miss split (smoe_verify_begin / smoe_verify_end): `begin` routes the tokens,
     computes the hits from the expert table and the shared expert into rows, and returns the misses for the caller
-    to fill; `end` combines the rows into y."""
+    to fill (miss_dst and counts, views of one small allocation); `end` combines the rows into y."""
 
     def __init__(self, g: Geom, weights: Dict, max_tokens: int, device="cuda"):
         import torch
@@ -891,13 +891,15 @@ class VerifyWindow:
         if T > self.max_tokens:
             raise SmoeError(-1, f"{T} tokens exceed the window's {self.max_tokens}")
         _need(table, "table", torch.int64, numel=self.g.n_expert)
-        dev, n = x.device, (T * K + T) * H
-        rows, counts = _parts(torch.zeros(n + 4, dtype=torch.float32, device=dev), n, 4)  # one fill of zeros
-        r = dict(rows=rows.view(T * K + T, H),
+        dev, m = x.device, max(T * K, 1)
+        # the split writes every count; -1 is what the entries past the misses hold
+        miss, counts = _parts(torch.full((m + 4,), -1, dtype=torch.int32, device=dev), m, 4)
+        if T == 0:
+            counts.zero_()
+        r = dict(rows=torch.zeros((T * K + T, H), dtype=torch.float32, device=dev),
                  ids=torch.empty((T, K), dtype=torch.int32, device=dev),
                  weights=torch.empty((T, K), dtype=torch.float32, device=dev),
-                 miss_dst=torch.full((max(T * K, 1),), -1, dtype=torch.int32, device=dev),
-                 counts=counts.view(torch.int32))
+                 miss_dst=miss, counts=counts)
         _check(lib().smoe_verify_begin(C.byref(self._gc), C.byref(self._wc), table.data_ptr(), x.data_ptr(), T,
                                        r["rows"].data_ptr(), r["ids"].data_ptr(), r["weights"].data_ptr(),
                                        r["miss_dst"].data_ptr(), r["counts"].data_ptr(), self.ws.data_ptr(),
