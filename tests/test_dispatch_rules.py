@@ -133,3 +133,20 @@ def test_junction_apart(ask):
              (16, 256, 512, 1, 0), (32, 256, 512, 0, 1), (12, 8, 4096, 0, 0), (16, 64, 4096, 0, 0), (32, 64, 4096, 0, 1),
              (12, 1024, 4096, 0, 1), (12, 8, 4096, 1, 1), (12, 8, 2048, 1, 0), (32, 8, 512, 0, 0), (127, 8, 512, 0, 1)]
     assert ask([f"junction_apart({T}, {E}, {H}, {f})" for T, E, H, f, _ in cases]) == [c[-1] for c in cases]
+
+
+def test_workspaces_grow_with_tokens():
+    """A workspace sized for more tokens holds every smaller call's, whatever kernels each takes."""
+    import ctypes as C
+
+    import stratametal_amd as S
+    L, p = S.lib(), 0x10000
+    geoms = [S.Geom(), S.Geom(w_type=22, sh_type=22, n_expert=64), S.Geom(sh_type=S.Q3_K, sh_down_type=S.IQ4_NL)]
+    for hc, lr in ((4, 320), (2, 64), (8, 960), (1, 1000)):
+        h = S._Hc(hc, lr, 1e-6, p, p, p, p)
+        tokens = list(range(0, 140)) + [300, 301, 1000, 4096]
+        sizes = [L.smoe_hc_read_workspace_bytes(C.byref(h), 2048, T) for T in tokens]
+        assert sizes == sorted(sizes), (hc, lr)
+        for g in geoms:
+            sizes = [L.smoe_ffn_workspace_bytes(C.byref(g.c()), C.byref(h), T) for T in tokens]
+            assert sizes == sorted(sizes) and sizes[-1] > 0, (hc, lr, vars(g))
