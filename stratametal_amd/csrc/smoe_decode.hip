@@ -760,22 +760,6 @@ __global__ __launch_bounds__(256) void k_router_tile(int H, int E, int T, int n_
     if (row < E && t < T) logits[(size_t)t * ld_logits + row] = bias ? acc[0] + bias[row] : acc[0];
 }
 
-// One stage of a reduce-scatter over per-lane values v[0 .. N): at distance D a lane keeps the half of its items
-// selected by its bit D and adds the partner's copy of them, so every item's sum is formed by exactly the additions
-// of the xor butterfly (own value plus the partner's at every stage, in that stage order).
-template <int D, int N>
-__device__ __forceinline__ void rs_stage(float* v, int lane) {
-    const bool upper = (lane & D) != 0;
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-        const float send = upper ? v[i] : v[i + N / 2];
-        float recv;
-        if constexpr (D == 32) recv = __shfl_xor(send, 32, kWave);
-        else recv = xor_swap<D>(send);
-        v[i] = (upper ? v[i + N / 2] : v[i]) + recv;
-    }
-}
-
 // group_sum of NIT values at once when lpr = 4 NIT (NIT = 2 or 4): a reduce-scatter over the group's upper
 // lane bits leaves lane l with the sum of value (l >> 2) & (NIT - 1), formed by exactly the butterfly's
 // additions (distance lpr / 2 first), then the last two stages as in group_sum.  NIT = 1: group_sum.
@@ -787,10 +771,10 @@ __device__ __forceinline__ float group_sum_rs(float (&v)[NIT], int lpr, int lane
     } else {
         static_assert(NIT == 2 || NIT == 4, "lpr = 4 NIT");
         if constexpr (NIT == 4) {
-            rs_stage<8, 4>(v, lane);
-            rs_stage<4, 2>(v, lane);
+            scatter_step<8, 4>(v, lane);
+            scatter_step<4, 2>(v, lane);
         } else {
-            rs_stage<4, 2>(v, lane);
+            scatter_step<4, 2>(v, lane);
         }
         float r = v[0];
         r = r + xor_swap<2>(r);
@@ -2910,7 +2894,8 @@ hipError_t launch_router(const float* xf, const uint16_t* xb, const void* W, con
     }
     const int chunks = H / 8;
     const int maxc = (chunks + 63) / 64;
-    // tokens staged per block: 4 for decode batches (more blocks, short staging), 16 (<= 64 KiB of bf16) beyond
+    // tokens staged per block: 4 for decode batches (more blocks, short staging), 16 (<= 64 KiB of bf16) beyond (more than
+    // 64 tokens come here with the fused junction or with x not 16-byte aligned)
     if (tile_rows)  // many tokens: bf16 x and W on the matrix cores
         return launch_router_mfma(xb, static_cast<const uint16_t*>(W), w_inp, bias, H, E, rows_total, T, logits,
                                   ld_logits, sg, s);
@@ -2981,9 +2966,10 @@ int gemv_shared_chunk() { return kShCols; }
 
 
 // Passes per wave and units per lane as constants: the unit loads are unconditional, so a kernel with more slots than the
-// row has units reloads the first in the others.  Odd unit counts have kernels of their own (2560 values are five units of
-// four lanes): with eight slots the gate/up and down of 77 tokens, 512 experts of 2560 by 640, took 115 and 68 us, the
-// whole call 198; with five 93, 60 and 171.
+// row has units reloads the first in the others.  Three and five units of one pass have kernels of their own (2560 values
+// are five units of four lanes): with eight slots the gate/up and down of 77 tokens, 512 experts of 2560 by 640, took 115
+// and 68 us, the whole call 198; with five 93, 60 and 171.  Seven units (896, 1792, 3584 values) run with eight slots, three
+// units of two passes (3072) with four.
 #define SMOE_SHAPE_DISPATCH(KERNEL_MACRO)              \
     if (nit == 4 && upl == 1) KERNEL_MACRO(4, 1);      \
     else if (nit == 4) KERNEL_MACRO(4, 2);             \

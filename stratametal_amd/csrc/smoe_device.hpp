@@ -164,6 +164,20 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// q8_1 of a value v in a block of largest magnitude a: its scale, and its int8 (returned).
+__device__ __forceinline__ int q8_1_quant(float v, float a, float& d) {
+    d = a / 127.0f;
+    if (__builtin_fabsf(d) > 65504.0f) d = __builtin_copysignf(65504.0f, d);
+    int q = 0;
+    if (a != 0.0f) {
+        float r = __builtin_roundf(v / d);
+        r = r > 127.0f ? 127.0f : r;
+        r = r < -127.0f ? -127.0f : r;
+        q = (r == r) ? (int)r : 0;
+    }
+    return q;
+}
+
 // q8_1 of one 32-value block held one value per lane of a 32-lane half wave (lane & 31 = position):
 // amax and sum by the xor butterfly 16..1, d = amax / 127 clamped to 65504, q = clamp(round(x / d)),
 // s clamped to 65504, d and s stored as fp16 (metal/shaders/iq.metal:597-627).  A NaN value stores 0.
@@ -175,15 +189,8 @@ __device__ __forceinline__ int q8_1_value(float v, uint32_t* ds) {
         a = __builtin_fmaxf(a, __shfl_xor(a, o, kWave));
         s = s + __shfl_xor(s, o, kWave);
     }
-    float d = a / 127.0f;
-    if (__builtin_fabsf(d) > 65504.0f) d = __builtin_copysignf(65504.0f, d);
-    int q = 0;
-    if (a != 0.0f) {
-        float r = __builtin_roundf(v / d);
-        r = r > 127.0f ? 127.0f : r;
-        r = r < -127.0f ? -127.0f : r;
-        q = (r == r) ? (int)r : 0;
-    }
+    float d;
+    const int q = q8_1_quant(v, a, d);
     const float sc = __builtin_fabsf(s) > 65504.0f ? __builtin_copysignf(65504.0f, s) : s;
     *ds = f32_to_f16(d) | (f32_to_f16(sc) << 16);
     return q;

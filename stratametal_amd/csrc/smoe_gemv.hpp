@@ -266,15 +266,8 @@ __device__ __forceinline__ void q8_image_store(float v, bool store, uint8_t* sc,
                                                uint64_t* xchg = nullptr) {
     const int l32 = threadIdx.x & 31;
     const float a = half_max(__builtin_fabsf(v));
-    float d = a / 127.0f;
-    if (__builtin_fabsf(d) > 65504.0f) d = __builtin_copysignf(65504.0f, d);
-    int q = 0;
-    if (a != 0.0f) {
-        float r = __builtin_roundf(v / d);
-        r = r > 127.0f ? 127.0f : r;
-        r = r < -127.0f ? -127.0f : r;
-        q = (r == r) ? (int)r : 0;
-    }
+    float d;
+    const int q = q8_1_quant(v, a, d);
     const int sq = half_sum_i(q);
     if (natural) {
         sc[l32] = (uint8_t)(int8_t)q;

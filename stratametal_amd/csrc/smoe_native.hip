@@ -357,12 +357,8 @@ __device__ __forceinline__ void quantise_lds(const float* __restrict__ x, int n,
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
             const float a = half_max(__builtin_fabsf(v[m]));
-            float d = a / 127.0f;
-            if (d > 65504.0f) d = 65504.0f;
-            float r = __builtin_roundf(v[m] / d);
-            r = r > 127.0f ? 127.0f : r;
-            r = r < -127.0f ? -127.0f : r;
-            const int q = (a != 0.0f && r == r) ? (int)r : 0;
+            float d;
+            const int q = q8_1_quant(v[m], a, d);
             const int i = i0 + NTH * m;
             if (i < n) {
                 xb[(i >> 5) * (4 * kXlDw) + l] = (uint8_t)(int8_t)q;
