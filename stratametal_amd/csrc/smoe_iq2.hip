@@ -224,6 +224,7 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
     const int nc0 = min(kCols, item.ncol);
     uint32_t raw[21];
     uint32_t off;
+    int staged = 0;
     if (stage_direct(item, 0, nc0, true)) {  // straight-line inside each branch, so no wait lands between the loads
         StageRounds<kDirect> sp;
         stage_issue_direct<64 * NW>(sp, ximg, qb, 0, nc0, kCols, 0, item, true);
@@ -232,13 +233,13 @@ __global__ __launch_bounds__(64 * NW) void k_iq2_gu(const int4* __restrict__ ite
         __builtin_amdgcn_sched_barrier(0);
         grid_table_store<64 * NW>(codes, tab);
         stage_commit_direct(sp, smem);
-        if (nc0 > 4)  // columns beyond those rounds
-            stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, kDirect * 64 * NW);
+        staged = kDirect * 64 * NW;
     } else {
         off = load_block_raw(rowp, b, raw);
         grid_table_store<64 * NW>(codes, tab);
-        stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true);
     }
+    // the columns beyond those rounds, or all
+    if (staged == 0 || nc0 > 4) stage_images<64 * NW>(smem, ximg, qb, 0, nc0, kCols, item, perm, k, true, staged);
     __syncthreads();
     Iq2Block B[1];
     decode_block(raw, off, tab, B[0]);
