@@ -168,14 +168,10 @@ __device__ __forceinline__ float wave_max(float v) {
 __device__ __forceinline__ int q8_1_quant(float v, float a, float& d) {
     d = a / 127.0f;
     if (__builtin_fabsf(d) > 65504.0f) d = __builtin_copysignf(65504.0f, d);
-    int q = 0;
-    if (a != 0.0f) {
-        float r = __builtin_roundf(v / d);
-        r = r > 127.0f ? 127.0f : r;
-        r = r < -127.0f ? -127.0f : r;
-        q = (r == r) ? (int)r : 0;
-    }
-    return q;
+    float r = __builtin_roundf(v / d);
+    r = r > 127.0f ? 127.0f : r;
+    r = r < -127.0f ? -127.0f : r;
+    return (a != 0.0f && r == r) ? (int)r : 0;  // a select, no branch
 }
 
 // q8_1 of one 32-value block held one value per lane of a 32-lane half wave (lane & 31 = position):
