@@ -164,8 +164,8 @@ smoe_status smoe_forward_path(const smoe_geom* g, const smoe_weights* w, const f
 
 /* The stacked configuration's layer junction fused into the next layer's call: x = RMSNorm(x_prev + r_prev)
  * (unit weight; as smoe_residual_rmsnorm forms it) is written to x, then y = MoE(x) as smoe_forward.  On the
- * decode (GEMV) path the norm is formed inside the router kernel; on the prefill path a junction kernel runs
- * first.  Bitwise equal to smoe_residual_rmsnorm followed by smoe_forward.  x must not overlap x_prev, r_prev
+ * decode (GEMV) path the norm of few tokens is formed inside the router kernel; of more, and on the prefill path, a
+ * junction kernel runs first.  Bitwise equal to smoe_residual_rmsnorm followed by smoe_forward.  x must not overlap x_prev, r_prev
  * or y (y may be r_prev); x_prev, r_prev and x 16-byte aligned.  No counterpart in the reference's MoE block
  * (its layer walk normalises in the hyper-connection read, out of this block's scope). */
 smoe_status smoe_forward_residual(const smoe_geom* g, const smoe_weights* w, const float* x_prev, const float* r_prev,
@@ -195,7 +195,12 @@ typedef struct {
 size_t smoe_hc_read_workspace_bytes(const smoe_hc* hc, int32_t n_embd, int32_t max_tokens);
 
 /* gr_read for n_tokens tokens: R [T][hc][n_embd] -> mixed [T][n_embd], inject [T][hc] (inject may be NULL: the
- * final mixer, nothing written).  Replaces gr_read (metal/include/strata/metal/gr.hpp:44-46) with bf16 activations. */
+ * final mixer, nothing written).  Replaces gr_read (metal/include/strata/metal/gr.hpp:44-46) with bf16 activations.
+ * A call of few tokens sums in one fixed order, a token's results the same bits in any such batch.  A larger batch runs on
+ * the matrix cores, whose f32 sums are of another order, as exact: from 17 tokens at n_embd 2048, hc 4, hc_lr 320, later
+ * for smaller shapes, never for n_embd % 64 != 0, hc_lr > 960, or R, norm or mixed not 16-byte aligned.  So the bits of a
+ * token's results depend on which of the two its batch and its buffers' alignment take: `inject` by the rounding of an
+ * f32 sum, `mixed` also where a low-rank value's bf16 rounding falls to the other side. */
 smoe_status smoe_hc_read(const smoe_hc* hc, int32_t n_embd, const float* R, int32_t n_tokens, float* mixed,
                          float* inject, void* workspace, size_t workspace_bytes, void* hip_stream);
 
@@ -210,7 +215,9 @@ size_t smoe_ffn_workspace_bytes(const smoe_geom* g, const smoe_hc* hc, int32_t m
 /* The whole layer call FfnExec::run(residual, out, add_shared, trace) (metal/include/strata/metal/layer_exec.hpp:
  * 135-137, metal/src/layer_exec.cpp:462-531): gr_read of the residual streams, the MoE block on `mixed`
  * (smoe_forward, SMOE_PATH_AUTO), gr_write of its output back onto the streams.  residual and out are
- * [T][hc][n_embd] f32 (out may be residual); `trace` covers the MoE block as in smoe_forward. */
+ * [T][hc][n_embd] f32 (out may be residual); `trace` covers the MoE block as in smoe_forward.  The read's order of sums
+ * changes with the batch as smoe_hc_read's does, so a window of draft tokens in one call and the same tokens one by one
+ * agree bit for bit only up to the batches that it takes by rows. */
 smoe_status smoe_ffn_run(const smoe_geom* g, const smoe_weights* w, const smoe_hc* hc, const float* residual,
                          int32_t n_tokens, float* out, int32_t add_shared, void* workspace, size_t workspace_bytes,
                          const smoe_trace* trace, void* hip_stream);

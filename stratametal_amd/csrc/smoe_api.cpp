@@ -421,8 +421,8 @@ smoe_status native_shared(const smoe_geom& g, const smoe_weights* w, const float
     return SMOE_OK;
 }
 
-// The forward call; with x_prev, x = RMSNorm(x_prev + r_prev) is formed first (fused into the router kernel on the
-// GEMV path, a junction kernel before the call on the MFMA path) and written to x.
+// The forward call; with x_prev, x = RMSNorm(x_prev + r_prev) is formed first (on the GEMV path in the router kernel or,
+// where junction_apart says so, by a kernel before it; on the MFMA path by a junction kernel) and written to x.
 smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io, int32_t n_tokens, float* y,
                          int32_t add_shared, void* workspace, size_t workspace_bytes, const smoe_trace* trace,
                          int32_t path, void* hip_stream, const float* x_prev, const float* r_prev, float eps) {
@@ -481,7 +481,7 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
         if (_m != SMOE_OK) return _m;        \
     } while (0)
     SMOE_MARK();
-    // the junction is fused into the router kernel of few tokens; more tokens take it as a kernel of its own
+    // (bitwise the same norm fused into the router kernel and as a kernel of its own)
     const bool fused_norm =
         x_prev && !mfma && !smoe::junction_apart(T, E, H, g->router_dtype == SMOE_ROUTER_F32);
     // the prefill path's per-work-group flags of its fp16 operand limits (folded by a trace or smoe_forward_status)
@@ -505,7 +505,7 @@ smoe_status forward_impl(const smoe_geom* g, const smoe_weights* w, float* x_io,
         SMOE_TRY(smoe::launch_residual_rmsnorm(x_prev, r_prev, T, H, eps, x_io, st), "junction");
     if (mfma && !x_prev)
         SMOE_TRY(smoe::launch_act_records(x, (int64_t)T * (H / 64), ximg, xbf, st, xflags), "activation records");
-    // the f32 router (router_dtype 1) reads f32 x on the row-per-wave path, also for many tokens
+    // the f32 router (router_dtype 1) reads f32 x, also for many tokens
     const bool f32r = g->router_dtype == SMOE_ROUTER_F32;
     SMOE_TRY(smoe::launch_router(fused_norm ? x_prev : x, f32r ? nullptr : xbf, w->router,
                                  has_sh ? w->gate_inp_sh : nullptr, w->logit_bias, H, E, E + (has_sh ? 1 : 0), T, logits,

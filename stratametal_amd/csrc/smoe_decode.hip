@@ -604,7 +604,7 @@ __global__ __launch_bounds__(256) void k_router(int H, int E, int T, int tok_til
 // sums (63 exchanges for 64 sums instead of 384).  The shared gate row goes one wave per token (n_gate work-groups behind
 // the tiles), then the q8_1 images, eight blocks per work-group.  k_router re-reads and re-stages x for every four rows
 // and reduces every sum by itself: 512 experts of 2048 bf16 values 20 us at 64 tokens and 126 at 600, of 2560 f32 values
-// 84 us at 77; bound by the VALU here (an fma per product, a quarter more to unpack bf16).
+// 84 us at 77; bound by the VALU here (an fma per product, a quarter more to unpack bf16; 72 to 88% of its issue slots).
 constexpr int kRtStage = 512;
 // Two f32 to bf16 (round to nearest even) by the hardware's packed conversion: f32_to_bf16's bits but for the payload of
 // a NaN, which makes a NaN of every sum either way.

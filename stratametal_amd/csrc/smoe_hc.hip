@@ -391,8 +391,8 @@ __global__ __launch_bounds__(256) void k_hc_lq(const float* __restrict__ part, i
 // stream, so that a lane ends with the gates of all streams of its (token, d) and forms the gated mean in registers.
 // lq of the tokens in LDS (pitch kp * 2 + 16 bytes); the wave's `up` rows stream from memory in chunks of 64 of K, the
 // next chunk's loads in flight.  The d ranges are the fastest index, so that where n / 64 is a multiple of 8 the token
-// blocks of a d range share an XCD, whose L2 serves the rows each of them reads again.  Bound by reading R and writing
-// mixed once the rows are in the caches.
+// blocks of a d range share an XCD, whose L2 serves the rows each of them reads again.  1000 tokens of n 2048, hc 4: 29 us,
+// of which the bytes (R, the gates' rows, mixed: 52 MB) take 11 and VALU issue, a sigmoid per value and stream, half.
 template <int HC, int NT>
 __global__ __launch_bounds__(256) void k_hc_mix_mm(const float* __restrict__ R, const float* __restrict__ norm,
                                                     const uint16_t* __restrict__ up, const uint16_t* __restrict__ lq,

@@ -13,8 +13,8 @@
 //
 // smoe_iq2.hip spends eight dots and about twelve more instructions per row, column and sub-block on the VALU; here it is
 // six, plus two matrix products that serve 16 x 16 of them and a costlier decode (fp16 pairs and their scaled copies), so a
-// tile of 16 columns costs what about six columns cost there (iq2_mm_gains).  Still bound by VALU issue: 600 tokens of 512
-// experts (2048, 512 wide) 648 us on the row kernels, 472 here.  A wave's block is loaded at its step (four waves per SIMD
+// tile of 16 columns costs what about six columns cost there (iq2_mm_gains).  Still bound by VALU issue (83 to 85% of its
+// slots, the matrix cores 12% busy): 600 tokens of 512 experts (2048, 512 wide) 648 us on the row kernels, 472 here.  A wave's block is loaded at its step (four waves per SIMD
 // cover the load): prefetched a step ahead, its 21 registers spilled others, 482 us.
 #include "smoe_gemv.hpp"
 #include "smoe_launch.hpp"

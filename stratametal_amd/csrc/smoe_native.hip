@@ -435,7 +435,7 @@ __global__ __launch_bounds__(256) void k_mmvq_native(const uint8_t* __restrict__
 // (each step halves the values a lane holds, 31 exchanges for 32 sums instead of 160), and the results go out through
 // LDS as whole runs of a column's rows.  On 1000 columns, a work-group per column decoding the rows again and this: Q3_K
 // 512 x 2048 232 and 58 us, IQ4_NL 2048 x 512 609 and 36 us.  Bound by the VALU: about nine instructions per 16 products
-// for IQ4_NL, 22 for Q3_K.
+// for IQ4_NL, 22 for Q3_K (81 to 86% of its issue slots).
 constexpr int kRw = 2, kXlChunk = 2048;
 static_assert(8 * kRw == kNativeTileRows, "the rows of a work-group");
 template <int TYPE, int C>
@@ -518,8 +518,8 @@ __global__ __launch_bounds__(256) void k_mmvq_native_cols(const uint8_t* __restr
 // A work-group takes 64 rows (16 per wave) or 32 (16 rows by 16 columns per wave) by 32 columns, 256 values of K at a time
 // through LDS as fp16; the sums run 4 + 4 blocks, two chunks, then in order: short chains, for an error no larger than the
 // row kernels'.  A word's four values lie in the order 0, 2, 1, 3 on both sides.  1000 columns, gate and up of Q3_K
-// 512 x 2048 and down of IQ4_NL 2048 x 512: 124 and 37 us on the row kernels, 32 and 17 here; bound by the latency of a
-// chunk's loads.
+// 512 x 2048 and down of IQ4_NL 2048 x 512: 124 and 37 us on the row kernels, 32 and 17 here: 60 to 65% of that VALU issue (the
+// decode and expansion of both sides), the rest the latency of a chunk's loads; the matrix cores are 5% busy.
 constexpr int kNmCols = 32, kNmPitch = 256 * 2 + 16;  // (the pad spreads 16 rows over the banks)
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
