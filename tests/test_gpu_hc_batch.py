@@ -1,8 +1,9 @@
-"""GPU parity of the hyper-connection read on the matrix cores (batches of tokens, k_hc_proj_mm and k_hc_mix_mm) against
-the oracle's row order on the same inputs.  Both sum exact bf16 products in f32 in different orders, so inject differs
-by the f32 sums' rounding (hc * n products: below 1e-5 of the products' magnitude), and mixed where a low-rank value's
-bf16 rounding falls to the other side: one of hc_lr values moves by up to 2^-8 of itself, so a gate by about
-2^-8 / sqrt(hc_lr) of its argument, and a row's mean by less (sigmoid's slope is at most 1/4)."""
+"""GPU parity of the hyper-connection read of batches, on the matrix cores (k_hc_proj_mm and k_hc_mix_mm) or the
+row-per-wave kernels by hc_mm_gains, against the oracle's row order on the same inputs.  Both sum exact bf16 products in
+f32 in different orders, so inject differs by the f32 sums' rounding (hc * n products: below 1e-5 of the products'
+magnitude), and mixed where a low-rank value's bf16 rounding falls to the other side: one of hc_lr values moves by up to
+2^-8 of itself, so a gate by about 2^-8 / sqrt(hc_lr) of its argument, and a row's mean by less (sigmoid's slope is at
+most 1/4)."""
 import numpy as np
 import pytest
 
@@ -13,17 +14,18 @@ from test_gpu_hc import GUARD, dev, hc_dev, host, rel_l1, streams, torch  # noqa
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # n_embd, hc, hc_lr, T: token tiles of 32 and 64 with remainders, row tiles of 128, K slices, chunk tails
+    # n_embd, hc, hc_lr, T: token tiles of 32 and 64 with remainders, row tiles of 128, K slices, chunk tails (the first
+    # batches of other shapes: test_gpu_hc_mm.py)
     (2048, 4, 320, 17),
     (2048, 4, 320, 130),
     (64, 1, 8, 16400),   # one chunk of K, one row tile mostly empty, the last token tile ragged
-    (192, 3, 200, 75),   # three streams, hc_lr no multiple of 64, an odd chunk count
-    (256, 8, 64, 64),    # eight streams
-    (512, 2, 960, 31),   # the widest low-rank tile
-    (3264, 5, 72, 20),   # five streams of more than 2048 values
+    (192, 3, 200, 75),   # the row-per-wave kernels, as the next three
+    (256, 8, 64, 64),
+    (512, 2, 960, 31),
+    (3264, 5, 72, 20),
     (4096, 4, 512, 95),  # the largest activation row, an lq tile too wide for 64 tokens
     (320, 4, 128, 700),  # many token tiles
-    (2048, 2, 64, 31),   # just below 2^23 products: the row-per-wave kernels
+    (2048, 2, 64, 31),   # the row-per-wave kernels, as the next
     (2048, 2, 64, 32),
     (1088, 1, 1000, 40),  # hc_lr past the matrix-core tile: the row-per-wave kernels
     (72, 3, 24, 40),      # no whole 64-value chunks: the row-per-wave kernels

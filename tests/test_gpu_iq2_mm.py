@@ -1,6 +1,7 @@
-"""GPU parity of the IQ2_S products on the matrix cores (batches of at least six pairs per expert, smoe_iq2_mm.hip) with
-the oracle's device order, bit for bit: every row length on both sides, column tiles with remainders, experts of several
-chunks, one or no column, the shared expert's tiles, and the same call on the row kernels (a traced call runs those)."""
+"""GPU parity of IQ2_S batches of six and more pairs per expert with the oracle's device order, bit for bit: every row length
+on both sides, columns with remainders, one or no column, the shared expert, and the same call traced (which runs the row
+kernels). With so few experts only the batch of 140 pairs per expert is on the matrix cores (smoe_iq2_mm.hip); the lines
+between the two and the other matrix-core batches are test_gpu_iq2_mm_rule.py's."""
 import numpy as np
 import pytest
 
@@ -12,14 +13,14 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # geometry, T, add_shared
-    (dict(n_embd=512, n_ff=512, n_ff_shared=512, n_expert=16, top_k=4, sh_type=22), 23, True),  # one token short of it: the row kernels
-    (dict(n_embd=512, n_ff=512, n_ff_shared=512, n_expert=16, top_k=4, sh_type=22), 24, True),  # the first batch it takes
+    (dict(n_embd=512, n_ff=512, n_ff_shared=512, n_expert=16, top_k=4, sh_type=22), 23, True),
+    (dict(n_embd=512, n_ff=512, n_ff_shared=512, n_expert=16, top_k=4, sh_type=22), 24, True),
     (dict(n_embd=512, n_ff=512, n_ff_shared=512, n_expert=16, top_k=4, sh_type=22), 33, False),
     (dict(n_embd=1024, n_ff=512, n_expert=8, top_k=2, sh_type=-1), 37, True),
     (dict(n_embd=2048, n_ff=512, n_ff_shared=512, n_expert=24, top_k=4, sh_type=22), 50, True),
     (dict(n_embd=512, n_ff=2048, n_ff_shared=2048, n_expert=6, top_k=2, sh_type=22), 33, True),
     (dict(n_embd=2048, n_ff=1024, n_expert=5, top_k=3, sh_type=-1), 23, True),
-    (dict(n_embd=1024, n_ff=1024, n_ff_shared=1024, n_expert=3, top_k=2, sh_type=22), 210, True),  # chunks of 64 columns
+    (dict(n_embd=1024, n_ff=1024, n_ff_shared=1024, n_expert=3, top_k=2, sh_type=22), 210, True),  # the matrix cores: chunks of 64 columns
     (dict(n_embd=512, n_ff=512, n_ff_shared=512, n_expert=16, top_k=4, sh_type=O.Q8_0), 80, True),  # a native shared expert
 ]
 
@@ -54,7 +55,7 @@ def test_forward_iq2_s_batches(torch, case):  # noqa: F811
 
 @pytest.mark.parametrize("n_embd, n_ff", [(2048, 512), (2048, 1024)])
 def test_iq2_s_down_passes(torch, n_embd, n_ff):  # noqa: F811
-    """Enough items for the down kernel's two passes of 256 rows: the row kernels' bits (those of a traced call)."""
+    """Six pairs per expert of 512: the traced call's bits (the down kernel's two passes are test_gpu_iq2_mm_rule.py's)."""
     g = S.Geom(w_type=22, sh_type=22, n_embd=n_embd, n_ff=n_ff, n_ff_shared=n_ff, n_expert=512, top_k=10)
     T = 311
     print(f"case: IQ2_S down passes H={n_embd} F={n_ff} T={T}", flush=True)

@@ -68,8 +68,8 @@ def test_mmvq_native_bitwise(torch, t):
 
 @pytest.mark.parametrize("t", TYPES)
 def test_mmvq_native_column_tiles_bitwise(torch, t):
-    """Column tiles of 4, 8 and 16 (by rows and columns: smoe_native.hip's rule) with remainders of rows, columns and
-    of the 2048 values of K staged at a time."""
+    """Column tiles of 4, 8 and 16 (native_cols; Q4_K, Q5_K and Q6_K take some of these by columns) with remainders of
+    rows, columns and of the 2048 values of K staged at a time."""
     qk = O.NATIVE[t][0]
     for n_in, n_out, n_col in [(qk, 895, 16), (2048 + qk, 1031, 15), (4096 + qk, 512, 29), (256, 2047, 30), (256, 2048, 50),
                                (2304, 1025, 131), (256, 16, 900)]:

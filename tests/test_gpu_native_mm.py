@@ -1,5 +1,6 @@
-"""GPU parity of a prompt's native shared expert on the matrix cores (k_native_mm) against the row kernels' chain
-(smoe_mmvq, bitwise the oracle's): the shared rows are what add_shared adds to the block's output.
+"""GPU parity of the prefill contract's native shared expert against the row kernels' chain (smoe_mmvq, bitwise the
+oracle's): the shared rows are what add_shared adds to the block's output. From 128 columns on the products run on the
+matrix cores (k_native_mm), fewer on the row kernels; more matrix-core cases are test_gpu_native_rule.py's.
 
 Both form every 32-value dot exactly and differ in the order and number of f32 roundings, a few 2^-24 of a sum, and where
 such a difference moves one of h's q8_1 values a step: 1/127 of its block's largest, in a row of n_ff values about
@@ -14,14 +15,14 @@ from test_gpu_native import dev, native_layer, say, torch  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # H, F, gate, up, down, T: column tiles of 32 and row tiles of 32 with remainders, an odd chunk count, a short chunk
+    # H, F, gate, up, down, T
     (2048, 512, O.Q3_K, O.Q3_K, O.IQ4_NL, 160),
     (2560, 640, O.Q3_K, O.Q3_K, O.IQ4_NL, 129),  # down: two chunks and a half
-    (1024, 384, O.Q8_0, O.Q8_0, O.Q8_0, 33),     # down: a chunk and a half
-    (1280, 512, O.Q4_0, O.Q4_0, O.Q5_0, 31),     # gate/up: five chunks
-    (640, 128, O.Q5_0, O.IQ4_NL, O.Q4_0, 1),     # gate and up apart; down: half a chunk
+    (1024, 384, O.Q8_0, O.Q8_0, O.Q8_0, 33),     # the row kernels
+    (1280, 512, O.Q4_0, O.Q4_0, O.Q5_0, 31),     # the row kernels
+    (640, 128, O.Q5_0, O.IQ4_NL, O.Q4_0, 1),     # the row kernels, gate and up apart
     (2048, 512, O.Q8_0, O.Q8_0, O.Q4_0, 545),    # row tiles of 64: more than 256 work-groups
-    (1536, 768, O.Q4_K, O.Q8_0, O.Q3_K, 64),     # one projection keeps the row kernels
+    (1536, 768, O.Q4_K, O.Q8_0, O.Q3_K, 64),     # the row kernels
 ]
 
 

@@ -1,4 +1,4 @@
-"""GPU parity of the tiled router (k_router_tile: calls of at least 5 tokens) with the oracle's device order, bit for bit,
+"""GPU parity of the tiled router (k_router_tile: router_tiles) with the oracle's device order, bit for bit,
 at the edges of its tiles: rows past the last row group, tokens past the last token tile, rows shorter than a stage of 512
 values and no multiple of it, both tile shapes, bf16 and f32 rows, the shared gate and the x images behind the tiles."""
 import numpy as np
