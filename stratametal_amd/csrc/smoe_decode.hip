@@ -2834,10 +2834,6 @@ static unsigned router_grid_x(int blocks, int T, int tile) {
     return (unsigned)(T > tile ? (blocks + 7) / 8 * 8 : blocks);
 }
 
-// The tile: few tokens need the work-groups (bf16 4 rows by 4 tokens, f32 2 by 8), from kRouterTileWide on 4 by 8 re-reads
-// less (512 rows of 2048, bf16 9.6 against 10.4 us at 100 tokens, 11.4 against 10.7 at 127).
-constexpr int kRouterTileWide = 112;
-
 template <bool F32, int RR, int TT>
 static hipError_t launch_router_tile(const float* xf, const uint16_t* xb, const void* W, const uint16_t* w_inp,
                                      const float* bias, int H, int E, int T, float* logits, int ld_logits, float* sg,
@@ -2869,7 +2865,7 @@ hipError_t launch_router(const float* xf, const uint16_t* xb, const void* W, con
     if (!tile_rows && !rprev && !clear_n16 && router_tiles(T, E, H, w_f32 != 0) && x16 && H % 8 == 0 && (xf || !w_inp)) {
 #define SMOE_ROUTER_TILE(F, RR, TT) \
     launch_router_tile<F, RR, TT>(xf, xb, W, w_inp, bias, H, E, T, logits, ld_logits, sg, ximg, img_natural, s)
-        if (T >= kRouterTileWide) return w_f32 ? SMOE_ROUTER_TILE(true, 4, 8) : SMOE_ROUTER_TILE(false, 4, 8);
+        if (router_tile_wide(T, E)) return w_f32 ? SMOE_ROUTER_TILE(true, 4, 8) : SMOE_ROUTER_TILE(false, 4, 8);
         return w_f32 ? SMOE_ROUTER_TILE(true, 2, 8) : SMOE_ROUTER_TILE(false, 4, 4);
 #undef SMOE_ROUTER_TILE
     }

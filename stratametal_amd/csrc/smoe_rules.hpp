@@ -124,6 +124,12 @@ constexpr bool router_tiles(int64_t T, int E, int H, bool f32) {
     return T >= 5 && (f32 || H <= 2560 || T * (E > 64 ? E : 64) >= 2048);
 }
 
+// The tile: few tokens or experts need the work-groups (bf16 4 rows by 4 tokens, f32 2 by 8), many of both re-read less in
+// tiles of 4 by 8 (512 rows of 2048, bf16 9.6 against 10.4 us at 100 tokens, 11.4 against 10.7 at 127; rows of 4096 at 127
+// tokens in tiles of 4 by 8 the same with 400 and 512 experts, 4.6 us longer with 256 and 4.8 with 64; f32 64 experts 3.1
+// us longer at 300 tokens, 128 experts 0.3 at 448).
+constexpr bool router_tile_wide(int64_t T, int E) { return T >= 112 && T * E >= 112 * 512; }
+
 // Whether the decode path runs the junction of T tokens as a kernel of its own: fused into the router kernel it saves the
 // launch, and repeats the norm in every work-group of the router.  Apart from 12 tokens on where the tiled router's gain
 // passes the launch, us: bf16, 512 experts of 2048 +0.4 at 10 tokens, +0.8 at 12, +3.6 at 16, 28.8 to 12.0 at 48; 64 experts

@@ -127,6 +127,11 @@ def test_router_tiles(ask):
     assert ask([f"router_tiles({T}, {E}, {H}, {f})" for T, E, H, f, _ in cases]) == [c[-1] for c in cases]
 
 
+def test_router_tile_wide(ask):
+    cases = [(111, 1024, 0), (112, 512, 1), (127, 256, 0), (224, 256, 1), (127, 64, 0), (300, 64, 0), (600, 128, 1), (600, 8, 0)]
+    assert ask([f"router_tile_wide({T}, {E})" for T, E, _ in cases]) == [c[-1] for c in cases]
+
+
 def test_junction_apart(ask):
     """Tokens, experts, n_embd, f32 rows: the junction in the router kernel (0) or a kernel of its own (1)."""
     cases = [(11, 512, 2048, 0, 0), (12, 512, 2048, 0, 1), (12, 64, 2048, 0, 0), (16, 64, 2048, 0, 0), (32, 64, 2048, 0, 1),

@@ -17,7 +17,8 @@ def layer(H, E, router, T, seed):
 
 
 @pytest.mark.parametrize("H,E,T,router", [(4096, 40, 31, 0), (4096, 40, 32, 0), (4096, 130, 15, 0), (4096, 130, 16, 0),
-                                          (2560, 40, 5, 0), (4096, 9, 5, 1), (2048, 33, 4, 0), (2048, 33, 5, 0)])
+                                          (2560, 40, 5, 0), (4096, 9, 5, 1), (2048, 33, 4, 0), (2048, 33, 5, 0),
+                                          (384, 520, 115, 1), (512, 520, 115, 0), (384, 33, 115, 1), (512, 33, 115, 0)])
 def test_block(torch, H, E, T, router):  # noqa: F811
     print(f"case: router rule block H={H} E={E} T={T} router {router}", flush=True)
     g, ml = layer(H, E, router, T, 78)
