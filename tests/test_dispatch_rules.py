@@ -101,7 +101,8 @@ def test_native_columns(ask):
     q4k, q5k, q6k, q3k, iq4nl = 12, 13, 14, 11, 20
     cases = [(q4k, 256, 20000, 4, 1, 1), (q4k, 256, 20000, 5, 1, 1), (q4k, 2560, 640, 32, 1, 1), (q4k, 2560, 640, 48, 1, 4),
              (q5k, 512, 2048, 5, 1, 1), (q6k, 512, 2048, 5, 1, 1), (q6k, 512, 2048, 12, 1, 4), (q6k, 8192, 1000, 24, 1, 1),
-             (q6k, 8192, 1000, 48, 1, 4), (q6k, 4096, 4096, 7, 1, 4), (q4k, 2048, 64, 250, 1, 4), (q3k, 2048, 512, 16, 1, 1), (q3k, 2048, 512, 16, 2, 4), (q3k, 2048, 512, 1000, 1, 16),
+             (q6k, 8192, 1000, 48, 1, 4), (q6k, 4096, 4096, 7, 1, 4), (q4k, 2048, 64, 250, 1, 4),
+             (q3k, 2048, 512, 16, 1, 1), (q3k, 2048, 512, 16, 2, 4), (q3k, 2048, 512, 1000, 1, 16),
              (iq4nl, 512, 2048, 3, 1, 1), (iq4nl, 512, 2048, 32, 1, 8), (iq4nl, 512, 2048, 4, 1, 1), (8, 256, 20000, 4, 1, 4),
              (8, 256, 20000, 5, 1, 8)]
     assert ask([f"native_cols({t}, {i}, {o}, {c}, {z})" for t, i, o, c, z, _ in cases]) == [c[-1] for c in cases]

@@ -1,5 +1,6 @@
 """GPU parity of the hyper-connection read of few tokens (k_hc_proj) at every count of streams, values per thread and
-pieces of a gate row that has registers of its own, and with the norm loaded after the scales, with the oracle's device order bit for bit."""
+pieces of a gate row that has registers of its own, and with the norm loaded after the scales, with the oracle's device
+order bit for bit."""
 import numpy as np
 import pytest
 
