@@ -387,6 +387,7 @@ smoe_status smoe_router_margin(const float* logits, int32_t n_tokens, int32_t n_
 smoe_status smoe_f32_to_bf16(const float* x, int64_t n, uint16_t* y, void* hip_stream);
 
 /* y[o] = sum_i f32(x[i]) * f32(w[o][i]) for n_tok rows of bf16 x; y is (n_tok, n_out).
+ * A product that a launch's grid does not hold (some 2^31 outputs and more, or 2^26 rows) is SMOE_EINVAL: split it.
  * Replaces bf16_gemv (metal/include/strata/metal/bf16_gemv.hpp:25). */
 smoe_status smoe_bf16_gemv(const uint16_t* x, const uint16_t* w, float* y, int32_t n_in, int32_t n_out,
                            int32_t n_tok, void* hip_stream);

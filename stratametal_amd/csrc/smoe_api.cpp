@@ -945,6 +945,10 @@ smoe_status smoe_bf16_gemv(const uint16_t* x, const uint16_t* w, float* y, int32
     if (n_in % 8 || n_in > 8192) return fail(SMOE_EINVAL, "bf16_gemv: n_in must be a multiple of 8, at most 8192");
     if ((int64_t)n_tok * n_in % 2) return fail(SMOE_EINVAL, "bf16_gemv: odd element count");
     if (!aligned(x, 16) || !aligned(w, 16)) return fail(SMOE_EALIGN, "bf16_gemv: x and w must be 16-byte aligned");
+    if (smoe::router_tiles(n_tok, n_out, n_in, false) ? !smoe::router_tile_fits(n_tok, n_out, n_in, false)
+                                                      : (int64_t)n_out / 4 >= smoe::kGridGroups)
+        return fail(SMOE_EINVAL, "bf16_gemv: " + std::to_string(n_tok) + " tokens by " + std::to_string(n_out) +
+                                     " rows exceed a launch's grid: split them");
     SMOE_TRY(smoe::launch_router(nullptr, x, w, nullptr, nullptr, n_in, n_out, n_out, n_tok, y, n_out, nullptr, nullptr,
                                  0, 0, stream_of(hip_stream)),
              "bf16_gemv");

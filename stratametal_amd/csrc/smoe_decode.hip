@@ -2839,11 +2839,9 @@ static hipError_t launch_router_tile(const float* xf, const uint16_t* xb, const 
                                      const float* bias, int H, int E, int T, float* logits, int ld_logits, float* sg,
                                      uint32_t* ximg, int img_natural, hipStream_t s) {
     const int n_rb = (E + 4 * RR - 1) / (4 * RR), n_tb = (T + TT - 1) / TT;
-    // the smaller of x and W is what every XCD reads
-    const int by_tok = (int64_t)T * 4 > (int64_t)E * (F32 ? 4 : 2) ? 1 : 0;
-    const int64_t tiles = by_tok ? (int64_t)(n_tb + 7) / 8 * 8 * n_rb : (int64_t)(n_rb + 7) / 8 * 8 * n_tb;
+    const int by_tok = router_by_tok(T, E, F32) ? 1 : 0;
+    const int64_t tiles = router_tile_grid(T, E, F32, RR, TT);
     const int64_t gate = w_inp ? (T + 3) / 4 : 0, img = ximg ? ((int64_t)T * (H / 32) + 7) / 8 : 0;
-    if (tiles + gate + img > INT32_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_router_tile<F32, RR, TT>), dim3((unsigned)(tiles + gate + img)), dim3(256), 0, s, H, E, T,
                        (int)tiles, W, xf, xb, n_rb, n_tb, by_tok, (int)gate, w_inp, bias, logits, ld_logits, sg, ximg,
                        img_natural);
@@ -2863,6 +2861,7 @@ hipError_t launch_router(const float* xf, const uint16_t* xb, const void* W, con
     if (w_f32 && (tile_rows || !xf || H % 4 || H > 4096)) return hipErrorInvalidValue;
     const bool x16 = xf ? (reinterpret_cast<uintptr_t>(xf) & 15) == 0 : (reinterpret_cast<uintptr_t>(xb) & 15) == 0;
     if (!tile_rows && !rprev && !clear_n16 && router_tiles(T, E, H, w_f32 != 0) && x16 && H % 8 == 0 && (xf || !w_inp)) {
+        if (!router_tile_fits(T, E, H, w_f32 != 0)) return hipErrorInvalidValue;
 #define SMOE_ROUTER_TILE(F, RR, TT) \
     launch_router_tile<F, RR, TT>(xf, xb, W, w_inp, bias, H, E, T, logits, ld_logits, sg, ximg, img_natural, s)
         if (router_tile_wide(T, E)) return w_f32 ? SMOE_ROUTER_TILE(true, 4, 8) : SMOE_ROUTER_TILE(false, 4, 8);

@@ -134,6 +134,20 @@ constexpr bool router_tiles(int64_t T, int E, int H, bool f32) {
 // f32 64 experts 3.1 us longer at 300 tokens, 128 experts 0.3 at 448).
 constexpr bool router_tile_wide(int64_t T, int E) { return T >= 112 && T * E >= 112 * 512; }
 
+// The tiled router's one-dimensional grid: the tiles of tt tokens by 4 rr rows, those of a row group, or by_tok of a
+// token tile, on one XCD (whole groups of 8).  A launch holds kGridGroups work-groups of 256 threads in a dimension and
+// takes a larger grid modulo that, with no error: a larger product, of some 2^31 outputs and more, is refused.
+constexpr int64_t kGridGroups = 0xFFFFFFFFll / 256;
+constexpr bool router_by_tok(int64_t T, int64_t E, bool f32) { return T * 4 > E * (f32 ? 4 : 2); }  // x, not W, on every XCD
+constexpr int64_t router_tile_grid(int64_t T, int64_t E, bool f32, int rr, int tt) {
+    const int64_t rb = (E + 4 * rr - 1) / (4 * rr), tb = (T + tt - 1) / tt;
+    return router_by_tok(T, E, f32) ? (tb + 7) / 8 * 8 * rb : (rb + 7) / 8 * 8 * tb;
+}
+constexpr bool router_tile_fits(int64_t T, int E, int H, bool f32) {
+    const bool wide = router_tile_wide(T, E);
+    return router_tile_grid(T, E, f32, f32 && !wide ? 2 : 4, !f32 && !wide ? 4 : 8) + T + T * (H / 32) / 8 < kGridGroups;
+}
+
 // Whether the decode path runs the junction of T tokens as a kernel of its own: fused into the router kernel it saves
 // the launch, and repeats the norm in every work-group of the router.  Apart from 12 tokens on where the tiled
 // router's gain passes the launch, us: bf16, 512 experts of 2048 +0.4 at 10 tokens, +0.8 at 12, +3.6 at 16, 28.8 to

@@ -133,6 +133,19 @@ def test_router_tile_wide(ask):
     assert ask([f"router_tile_wide({T}, {E})" for T, E, _ in cases]) == [c[-1] for c in cases]
 
 
+def test_router_tile_grid(ask):
+    """A product whose tiles a launch's grid does not hold (152064 rows by 16384 tokens, 10 GB of logits) is refused
+    before any launch; every smaller one is taken."""
+    cases = [(16384, 152064, 2048, 0, 0), (4096, 152064, 2048, 0, 1), (2056, 1 << 20, 8, 0, 0), (2000, 1 << 20, 8, 0, 1),
+             (65535, 1024, 4096, 1, 1), (100, 1 << 24, 8, 0, 0), (5, 1 << 24, 8, 0, 1)]
+    assert ask([f"router_tile_fits({T}, {E}, {H}, {f})" for T, E, H, f, _ in cases]) == [c[-1] for c in cases]
+    assert ask(["router_tile_grid(203, 700, 0, 4, 8)", "router_tile_grid(16, 513, 0, 4, 4)"]) == [26 * 48, 4 * 40]
+    import stratametal_amd as S
+    for T, E, H in ((16384, 152064, 2048), (2056, 1 << 20, 8), (1, 1 << 26, 8)):
+        assert S.lib().smoe_bf16_gemv(1 << 20, 1 << 20, 1 << 20, H, E, T, None) == -1
+        assert b"exceed a launch's grid" in S.lib().smoe_last_error()
+
+
 def test_junction_apart(ask):
     """Tokens, experts, n_embd, f32 rows: the junction in the router kernel (0) or a kernel of its own (1)."""
     cases = [(11, 512, 2048, 0, 0), (12, 512, 2048, 0, 1), (12, 64, 2048, 0, 0), (16, 64, 2048, 0, 0), (32, 64, 2048, 0, 1),

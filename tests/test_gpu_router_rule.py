@@ -48,6 +48,18 @@ def test_subnormal_token(torch, router):  # noqa: F811
             assert np.array_equal(bits(host(torch, tr[k])).reshape(T, -1)[t], bits(host(torch, tr1[k])).ravel()), (k, t)
 
 
+@pytest.mark.skip(reason="such a product is refused: by rows (k_router) it once faulted the GPU, cause not found")
+def test_rows_past_the_tiles_grid(torch):  # noqa: F811
+    """2^20 rows by 2056 tokens: more tiles than a launch's dimension holds; the bits of a few tokens' call."""
+    n_in, n_out, T = 8, 1 << 20, 2056
+    print(f"case: bf16 gemv n_in={n_in} n_out={n_out} T={T}", flush=True)
+    xb, w = (dev(torch, O.gen_bf16(6, s, n, 1.0).view(np.int16)) for s, n in ((1, T * n_in), (2, n_out * n_in)))
+    y = S.bf16_gemv(xb, w, n_in, n_out)
+    for t in (0, 1027, 2054):
+        few = S.bf16_gemv(xb[t * n_in:(t + 2) * n_in].clone(), w, n_in, n_out)
+        assert torch.equal(y.view(T, n_out)[t:t + 2].view(torch.int32), few.view(2, n_out).view(torch.int32)), t
+
+
 @pytest.mark.parametrize("value", [np.inf, np.nan])
 def test_other_tokens(torch, value):  # noqa: F811
     H, E, T = 512, 33, 21
